@@ -53,11 +53,8 @@ def measured_traffic(workload: str, kernel: str, rows: str, summary: str = "hbm_
 
 
 def resolved_stage_kernel(option: str, nx: int, ny: int) -> str:
-    """The stage kernel the library runs for --stage-kernel auto: strips when 4-row strips of 60
-    output columns give at least 1024 wavefronts, else 8x8 tiles."""
-    if option != "auto":
-        return option
-    return "strip" if ((ny + 59) // 60) * ((nx + 3) // 4) >= 1024 else "tile"
+    """The stage kernel the library runs for --stage-kernel auto: strips at every size."""
+    return option if option != "auto" else "strip"
 
 
 def stage_bytes_per_cell(integrator: str) -> float:

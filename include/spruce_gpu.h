@@ -151,10 +151,10 @@ int spruce_gpu_stream(spruce_gpu_domain* d, void** hip_stream);
 int spruce_gpu_device_grid(spruce_gpu_domain* d, const char* name, double** dev_ptr);
 
 /* Execution options (no reference counterpart; step results are identical for every setting):
- *   "stage_kernel" = "auto" (default: strips when the grid gives at least 1024 4-row strip
- *                    wavefronts, else one thread per cell) | "strip" (wavefront strips marching
- *                    along x) | "cell" (one thread per cell, faces recomputed per cell);
- *   "strip_rows"   = rows per wavefront strip, a multiple of 4 (default: chosen from the grid size);
+ *   "stage_kernel" = "auto" (default: strips) | "strip" (strips of a block of two wavefronts
+ *                    marching along x) | "tile" (8x8 tiles) | "cell" (one thread per cell, faces
+ *                    recomputed per cell);
+ *   "strip_rows"   = rows per strip, a multiple of 4 (default: chosen from the grid size);
  *   "tc_kernel"    = thermal-conduction update: "auto" (default: strips when 8-row strips give at
  *                    least 4096 wavefronts, else one thread per cell) | "strip" (wavefront strips,
  *                    every face computed once, b_hat derivatives formed in the kernel) | "cell";

@@ -193,6 +193,8 @@ class Domain : public DomainBase {
   int kinds_all[4] = {0, 0, 0, 0}, kinds_ucnp[4] = {0, 0, 0, 0}, kinds_live[4] = {0, 0, 0, 0};
   double s1[4] = {1, 1, 1, 1}, s2[4] = {1, 1, 1, 1};
   bool any_open = false;
+  uint64_t row_mask[N_STATIC];   // per static field, 0 where every row equals row 0
+  bool in_range = false;  // the mesh and the external field allow untested divisions (range.hpp)
   int stage_kernel = -1;  // 0: wavefront strips (mhd2.hip), 1: one thread per cell, 2: tiles (mhd.hip), -1: by size
   // the final stage of a step also forms the next step size's per-block minima (tile form, no ghost
   // fill, limiter or module after the integrator)
@@ -432,6 +434,17 @@ class Domain : public DomainBase {
       s1[k] = std::pow(desc.open_boundary_decay_base, dist12 / delta_last);
     }
 
+    const char* statics[N_STATIC] = {"be_x", "be_y", "be_z", "grav_x", "grav_y"};
+    for (int k = 0; k < N_STATIC; ++k) {
+      const std::vector<double>& g = host_grids[statics[k]];
+      bool same = true;
+      for (int i = 1; same && i < nx; ++i) same = std::memcmp(&g[(size_t)i * ny], &g[0], ny * sizeof(double)) == 0;
+      row_mask[k] = same ? 0 : ~(uint64_t)0;
+    }
+    in_range = ax.in_range && ay.in_range && kc.gm1 >= 0x1p-60 && kc.gm1 <= 0x1p+10;
+    for (const char* s : {"be_x", "be_y", "be_z"})
+      for (double v : host_grids[s]) in_range = in_range && field_in_range(v);
+
     L.alloc(N);
     W.alloc(N);
     if (desc.time_integrator == SPRUCE_RK4) {
@@ -455,7 +468,7 @@ class Domain : public DomainBase {
     if (strip_rows == 0) strip_rows = mhd_strip_rows_default(nx, ny);
     if (tc_rows == 0) tc_rows = tc_strip_rows_default(nx, ny);
     if (tc_kernel < 0) tc_kernel = tc_kernel_default(nx, ny);
-    if (stage_kernel < 0) stage_kernel = mhd_stage_kernel_default(nx, ny);
+    if (stage_kernel < 0) stage_kernel = 0;   // the strips are the fastest form at every size
     fuse_dt = stage_kernel == 2 && !(kinds_all[0] || kinds_all[1] || kinds_all[2] || kinds_all[3]) && !any_moc &&
               mods.empty();
     dt_blocks = mhd_dt_blocks(mesh);
@@ -612,6 +625,8 @@ class Domain : public DomainBase {
     a.step = step_ptr ? step_ptr : step.p; a.step_mult = mult; a.mode = mode;
     a.write_pre = any_open ? 1 : 0;
     a.write_n = 1;
+    a.in_range = in_range ? 1 : 0;
+    std::copy(row_mask, row_mask + N_STATIC, a.row_mask);
     a.moc = moc_terms(S);
     if (mode == STAGE_STORE_K) a.kbuf = kout ? kout : kbuf[kslot].p;
     if (mode == STAGE_RK4_FINAL) { a.kbuf = kbuf[0].p; a.k2buf = kbuf[1].p; a.k3buf = kbuf[2].p; }

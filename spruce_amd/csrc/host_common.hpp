@@ -10,6 +10,7 @@
 
 #include "../../include/spruce_gpu.h"
 #include "mhd.hpp"
+#include "range.hpp"
 
 namespace spruce {
 
@@ -52,14 +53,22 @@ struct DBuf {
 struct AxisBufs {
   DBuf d, rd, h, hsq, rhsq, fden, rfden, gup, gdn;
   std::vector<double> hd;  // host copy of the cell sizes
+  FaceGeom* face = nullptr;   // device
+  AxisBufs() = default;
+  AxisBufs(const AxisBufs&) = delete;
+  AxisBufs& operator=(const AxisBufs&) = delete;
+  ~AxisBufs() { if (face) (void)hipFree(face); }
+  bool in_range = false;   // every length on the axis is in the range of the untested divisions
   Axis view(int n, int lo, int hi, int per) const {
-    return Axis{d.p, rd.p, h.p, hsq.p, rhsq.p, fden.p, rfden.p, gup.p, gdn.p, n, lo, hi, per, lo, hi};
+    return Axis{d.p, rd.p, h.p, hsq.p, rhsq.p, fden.p, rfden.p, gup.p, gdn.p, n, lo, hi, per, lo, hi, face};
   }
   // Precomputes the geometry the stencils divide by; every reciprocal is a correctly rounded
   // IEEE division on the host.
   void build(const std::vector<double>& dcell, bool per) {
     const int n = (int)dcell.size();
     hd = dcell;
+    in_range = true;
+    for (double v : dcell) in_range = in_range && geometry_in_range(v);
     std::vector<double> vd(n), vrd(n), vh(n), vhsq(n), vrhsq(n), vf(n, 0.0), vrf(n, 0.0), vgu(n, 0.0), vgd(n, 0.0);
     for (int i = 0; i < n; ++i) {
       vd[i] = dcell[i];
@@ -81,6 +90,15 @@ struct AxisBufs {
     };
     up(d, vd); up(rd, vrd); up(h, vh); up(hsq, vhsq); up(rhsq, vrhsq); up(fden, vf); up(rfden, vrf);
     up(gup, vgu); up(gdn, vgd);
+    std::vector<FaceGeom> vface(n);
+    for (int c = 0; c < n; ++c) {
+      const int cm1 = per ? w(c - 1) : std::max(c - 1, 0), cp1 = per ? w(c + 1) : std::min(c + 1, n - 1);
+      vface[c] = FaceGeom{vh[cm1], vh[c], vf[c], vrf[c], vgu[c], vf[cm1], vrf[cm1], vgd[c], vf[cp1], vrf[cp1], vd[c], vrd[c]};
+    }
+    if (face) (void)hipFree(face);
+    face = nullptr;
+    hip_check(hipMalloc(&face, n * sizeof(FaceGeom)), "hipMalloc");
+    hip_check(hipMemcpy(face, vface.data(), n * sizeof(FaceGeom), hipMemcpyHostToDevice), "upload geometry");
   }
 };
 

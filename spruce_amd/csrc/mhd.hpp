@@ -1,8 +1,19 @@
 // Device-side data layout and kernel launchers of the IdealMHD time step.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 namespace spruce {
+
+// What a face takes from the mesh, gathered so that a kernel reads it in one access, and the cell
+// above the face: interpolation weights and denominator, the extrapolation geometry on both sides
+// (derivs.cpp:477-499), and the cell's size.
+struct FaceGeom {
+  double hlo, hup, den, rden;
+  double gup, denm, rdenm;   // extrapolation through (c-2, c-1)
+  double gdn, denp, rdenp;   // extrapolation through (c+1, c)
+  double d, rd;              // cell c
+};
 
 // One axis of the (separable) mesh: d_x depends on x only and d_y on y only, so each is a 1-D array
 // (the .state file stores them as full grids; setup checks they are separable).
@@ -19,6 +30,7 @@ struct Axis {
   const double* gdn;    // face c: h[c+1] + 2 h[c]     (extrapolation from above)
   int n, lo, hi, per;   // cells, interior bounds, periodic on both sides
   int dlo, dhi;         // bounds of the step-size minimum (plasmadomain.cpp:155-159)
+  const FaceGeom* face; // face c gathered from the arrays above (neighbours wrapped or clamped)
 };
 
 // Per-cell state of one IdealMHD grid set.  rho and n are both kept because after
@@ -31,6 +43,7 @@ struct MhdSet {
 struct MhdStatic {
   const double *bex, *bey, *bez, *gx, *gy;
 };
+enum { ST_BEX = 0, ST_BEY, ST_BEZ, ST_GX, ST_GY, N_STATIC };
 
 struct MhdConst {
   double m, rm;          // ion mass and RN(1/m)
@@ -74,6 +87,11 @@ struct StageArgs {
   int mode;
   int write_pre;         // write rho_pre (open boundaries present)
   int write_n;
+  // per static field: all bits set, or 0 where every row equals row 0 (a field of height only, or
+  // none at all, as gravity, be_z and an absent external field are), which a strip then reads again
+  // from the caches instead of streaming the grid
+  uint64_t row_mask[N_STATIC];
+  int in_range;          // the geometry and static fields allow the untested divisions (range.hpp)
   // Module RHS terms (computeTimeDerivativesModule, equationset.cpp:204-210): k[extra_var[e]] +=
   // extra[e][c] in order, already multiplied by the ghost mask.
   const double* extra[4];
@@ -89,11 +107,9 @@ struct StageArgs {
 constexpr int MAX_RHS_TERMS = 4;
 
 void launch_mhd_stage(const StageArgs& a, hipStream_t s);
-// Wavefront-strip form of the same stage (mhd2.hip); R rows per wavefront, a multiple of 4.
+// Wavefront-strip form of the same stage (mhd2.hip); R >= 1 rows per strip.
 void launch_mhd_stage_strip(const StageArgs& a, int R, hipStream_t s);
 int mhd_strip_rows_default(int nx, int ny);
-// 0 (strips) when the grid gives the strip kernel enough wavefronts, else 2 (tiles)
-int mhd_stage_kernel_default(int nx, int ny);
 // Tile form (mhd.hip): a block of 192 threads owns an 8x8 tile; each face of the tile is computed
 // once, by one thread, into LDS, then one thread per cell combines its four faces.  For grids too
 // small to fill the GPU with strips.  mhd_tile_blocks() blocks (and dt_partial entries).

@@ -1,12 +1,25 @@
 // IdealMHD stage kernel, wavefront-strip form (the production path of launch_mhd_stage).
 //
-// Each 64-lane wavefront owns a strip of 64 columns (y, contiguous in memory) and marches down R
-// rows (x).  Lanes 2..61 produce outputs; lanes 0, 1, 62, 63 only supply the y-halo.  Along x the
-// four rows a face needs (c-2 .. c+1) stay in a rotating register window, so every x-face is
+// A block of two 64-lane wavefronts owns a strip of 64 columns (y, contiguous in memory) and marches
+// down R rows (x).  Lanes 2..61 produce outputs; lanes 0, 1, 62, 63 only supply the y-halo.  Along x
+// the four rows a face needs (c-2 .. c+1) stay in a rotating register window, so every x-face is
 // computed once and reused by the two cells that share it; along y the neighbouring columns are
 // read from the neighbouring lanes with DPP wave shifts, so every y-face is computed once too.
-// Every cell-centred derived value (v = mom/rho, press) is computed once per row.  The arithmetic
-// of each value is the reference's (derivs.cpp, idealmhd.cpp), operation for operation.
+// One wavefront transports the fluid (rho, mom, thermal energy), the other the field (bi, be); each
+// forms the velocities it needs once per row, and the field hands its terms of the momentum
+// equations over in LDS.  The arithmetic of each value is the reference's (derivs.cpp,
+// idealmhd.cpp), operation for operation.
+//
+// What bounds it: FP64 instruction issue and the latency of a row's chain.  Each row is one
+// straight run of about 550 VALU instructions per wavefront, because the divisions' range tests are
+// made once per loaded value (range.hpp) instead of at each of the ~90 divisions per cell, where
+// they cost twice the instructions and ended a basic block each.  One wavefront for all eleven
+// quantities needs more than 256 registers once the code is straight, and a spilled value's reload
+// also waits for the rows being fetched; the split leaves room (249 registers, no spill, two
+// wavefronts per SIMD) to fetch a row two rows ahead.  Measured on 2048x2048 (RK2, periodic): 536 us
+// a stage with tested divisions and one wavefront per strip, 404 us with untested ones, 350 us with
+// the split, 290 us with the longer fetch distance, the gathered geometry and the static rows;
+// 1.09 GB of HBM traffic a launch, VALU 46% busy.  512x1024: 110 -> 40 us; 64x48: 17 (8x8 tiles) -> 9 us.
 #include <cfloat>
 #include <type_traits>
 
@@ -17,9 +30,14 @@
 namespace spruce {
 namespace {
 
-constexpr int NQ = 11;  // transported quantities, in idealmhd.cpp:52-86 order
-enum { Q_RHO = 0, Q_MX, Q_MY, Q_MZ, Q_TE, Q_BIX, Q_BEX, Q_BIY, Q_BEY, Q_BIZ, Q_BEZ };
+
 using namespace strip;
+
+// The eleven transported quantities (idealmhd.cpp:52-86) are split between the two wavefronts of a
+// block: the fluid's and the field's (bi and be, component by component).
+enum Role { FLUID = 0, FIELD = 1 };
+enum { Q_RHO = 0, Q_MX, Q_MY, Q_MZ, Q_TE };                  // FLUID
+enum { Q_BIX = 0, Q_BEX, Q_BIY, Q_BEY, Q_BIZ, Q_BEZ };       // FIELD
 
 // qdiv for a data-dependent divisor: the reciprocal is exact-rounded only if it is a normal number.
 __device__ __forceinline__ double qdiv_d(double a, double b, double rb) {
@@ -28,46 +46,43 @@ __device__ __forceinline__ double qdiv_d(double a, double b, double rb) {
   return a / b;
 }
 
-// Face velocity of one face: interpolated v and press, and the upwind side (derivs.cpp:10-73, 155).
-template <int AX>
-__device__ __forceinline__ FaceDir face_velocity(const double* vlo, const double* vup, double plo, double pup,
-                                                 const FaceGeom& g, double* iv, double& ip) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) iv[k] = interp(g, vlo[k], vup[k]);
-  ip = interp(g, plo, pup);
-  return face_dir(iv[AX], g);
+// What a block shares.  The geometry of every column's lower y-face and its cell size are read from
+// here once per row (24 registers otherwise, or a chain of an address and a load at the head of
+// every row); force holds the field's terms of the momentum equations for the row being finished,
+// in two slots so that one barrier per row orders the wavefronts; out_of_range says whether a
+// wavefront found a value outside the range of the untested divisions in a row it loaded.
+enum { F_EXT0 = 0, F_EXT1, F_IN0, F_IN1, F_INZ0, F_INZ1, F_EXTZ0, F_EXTZ1, F_ZEXT, F_ZIN, NF };
+struct Shared {
+  double2 geom[6][64];
+  double force[2][NF][64];
+  int out_of_range[2][2];
+};
+__device__ __forceinline__ void put_ygeom(Shared& s, const Axis& ax, int j, int l) {
+  const FaceGeom g = face_geom(ax, j);
+  s.geom[0][l] = double2{g.hlo, g.hup};
+  s.geom[1][l] = double2{g.den, g.rden};
+  s.geom[2][l] = double2{g.gup, g.denm};
+  s.geom[3][l] = double2{g.rdenm, g.gdn};
+  s.geom[4][l] = double2{g.denp, g.rdenp};
+  s.geom[5][l] = double2{g.d, g.rd};
+}
+__device__ __forceinline__ FaceGeom get_ygeom(const Shared& s, int l) {
+  const double2 a = s.geom[0][l], b = s.geom[1][l], c = s.geom[2][l], d = s.geom[3][l], e = s.geom[4][l],
+                f = s.geom[5][l];
+  return FaceGeom{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, e.x, e.y, f.x, f.y};
+}
+// LDS written before is seen by both wavefronts after; loads from memory stay in flight
+__device__ __forceinline__ void block_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-__device__ __forceinline__ void load_row(const StageArgs& a, int i, bool ivalid, int j, bool jvalid, double* q) {
-  if (ivalid && jvalid) {
-    const size_t c = (size_t)i * a.mesh.ny + j;
-    q[Q_RHO] = a.S.rho[c];
-    q[Q_MX] = a.S.mx[c];
-    q[Q_MY] = a.S.my[c];
-    q[Q_MZ] = a.S.mz[c];
-    q[Q_TE] = a.S.te[c];
-    q[Q_BIX] = a.S.bx[c];
-    q[Q_BEX] = a.st.bex[c];
-    q[Q_BIY] = a.S.by[c];
-    q[Q_BEY] = a.st.bey[c];
-    q[Q_BIZ] = a.S.bz[c];
-    q[Q_BEZ] = a.st.bez[c];
-  } else {
-#pragma unroll
-    for (int k = 0; k < NQ; ++k) q[k] = 0.0;
-    q[Q_RHO] = 1.0;
-  }
-}
-
-// v = mom/rho (idealmhd.cpp:248-250) and press = (gamma-1) te (idealmhd.cpp:253)
-__device__ __forceinline__ void derive(const double* q, const MhdConst& K, double* v, double& p) {
-  const double rho = q[Q_RHO];
-  const double rr = 1.0 / rho;
-  v[0] = qdiv_d(q[Q_MX], rho, rr);
-  v[1] = qdiv_d(q[Q_MY], rho, rr);
-  v[2] = qdiv_d(q[Q_MZ], rho, rr);
-  p = q[Q_TE] * K.gm1;
-}
+// This lane's column in a strip.
+struct Column {
+  int j;                     // wrapped (periodic) or clamped
+  bool interior, out;        // inside the interior bounds; this lane writes it
+};
 
 // Strip of a workgroup: launch index L mapped XCD-aware (xcd_tile) onto the strips in column-major
 // order, so strips that run together on one XCD are x-neighbours and share their halo rows in L2.
@@ -77,236 +92,388 @@ __device__ __forceinline__ void strip_of(int L, int nstrips, int total, int& col
   strip = t - col * nstrips;
 }
 
-template <int MODE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
-k_mhd_stage_strip(StageArgs a, int R, int nstrips) {
+// One wavefront's row: its transported quantities, and for the field the fluid values v needs.
+template <int ROLE> struct Row;
+template <> struct Row<FLUID> {
+  double q[5];
+  __device__ __forceinline__ bool out_of_range() const {
+    RangeTest t;
+    t.density(q[Q_RHO]);
+#pragma unroll
+    for (int k = Q_MX; k <= Q_TE; ++k) t.add(q[k]);
+    return t.out();
+  }
+};
+template <> struct Row<FIELD> {
+  double q[6];
+  double rho, m[3];
+  __device__ __forceinline__ bool out_of_range() const {   // be is checked at set-up, the fluid by the other wavefront
+    RangeTest t;
+    t.add(q[Q_BIX]);
+    t.add(q[Q_BIY]);
+    t.add(q[Q_BIZ]);
+    return t.out();
+  }
+};
+
+// Rows and columns beyond a closed side are clamped to the grid: their values reach only the faces
+// of ghost cells, whose derivatives are masked.
+template <int ROLE>
+__device__ __forceinline__ void load_row(const StageArgs& a, int i, uint32_t jb, Row<ROLE>& r) {
+  const size_t row = (size_t)i * a.mesh.ny;
+  lane_offset(jb);
+  if constexpr (ROLE == FLUID) {
+    r.q[Q_RHO] = ld_row(a.S.rho, row, jb);
+    r.q[Q_MX] = ld_row(a.S.mx, row, jb);
+    r.q[Q_MY] = ld_row(a.S.my, row, jb);
+    r.q[Q_MZ] = ld_row(a.S.mz, row, jb);
+    r.q[Q_TE] = ld_row(a.S.te, row, jb);
+  } else {
+    r.rho = ld_row(a.S.rho, row, jb);
+    r.m[0] = ld_row(a.S.mx, row, jb);
+    r.m[1] = ld_row(a.S.my, row, jb);
+    r.m[2] = ld_row(a.S.mz, row, jb);
+    r.q[Q_BIX] = ld_row(a.S.bx, row, jb);
+    r.q[Q_BEX] = ld_row(a.st.bex, row & a.row_mask[ST_BEX], jb);
+    r.q[Q_BIY] = ld_row(a.S.by, row, jb);
+    r.q[Q_BEY] = ld_row(a.st.bey, row & a.row_mask[ST_BEY], jb);
+    r.q[Q_BIZ] = ld_row(a.S.bz, row, jb);
+    r.q[Q_BEZ] = ld_row(a.st.bez, row & a.row_mask[ST_BEZ], jb);
+  }
+}
+
+// v = mom/rho (idealmhd.cpp:248-250), N components (the fluid's wavefront never needs v_z)
+template <bool IN, int N>
+__device__ __forceinline__ void velocities(double rho, const double* m, double* v) {
+  const double rr = 1.0 / rho;
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = IN ? qdiv_in(m[k], rho, rr) : qdiv_d(m[k], rho, rr);
+}
+
+// Rows rs .. rend-1 of a strip for one of the block's two wavefronts.  IN: the untested divisions;
+// every row is tested as it is loaded, and both wavefronts stop before the first row whose stencil
+// holds a value out of range.  Returns the row they stopped at (rend when done).  SAME: the update's
+// base is the set the derivatives are evaluated on.
+template <int ROLE, int MODE, bool IN, bool SAME>
+__device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shared& sh, double stepv, int rs, int rend) {
+  constexpr int NQ = ROLE == FLUID ? 5 : 6;     // transported quantities
+  constexpr int NV = ROLE == FLUID ? 2 : 3;     // velocity components held per row
+  constexpr int NO = ROLE == FLUID ? 5 : 3;     // evolved variables
+  constexpr int O0 = ROLE == FLUID ? 0 : 5;     // the first of them in evolved order
   const Mesh& M = a.mesh;
   const MhdConst& K = a.k;
-  const int nx = M.nx, ny = M.ny;
-  const int lane = threadIdx.x;
-  int col, strip;
-  strip_of(blockIdx.x, nstrips, gridDim.x, col, strip);
-  const int jraw = col * OUT_COLS + lane - 2;
-  int j;
-  bool jvalid;
-  if (M.y.per) { j = wrapn(jraw, ny); jvalid = true; }
-  else { jvalid = jraw >= 0 && jraw < ny; j = clampn(jraw, ny); }
-  const bool out_lane = lane >= 2 && lane < 62 && jraw >= 0 && jraw < ny;
-  const bool yint = jvalid && j >= M.y.lo && j <= M.y.hi;
-  const double stepv = a.step_mult * (*a.step);
+  const int nx = M.nx, ny = M.ny, lane = threadIdx.x;
   const size_t N = (size_t)nx * ny;
-  const int r0 = strip * R;
-
-  auto row_of = [&](int r, bool& ok) -> int {
-    if (M.x.per) { ok = true; return wrapn(r, nx); }
-    ok = r >= 0 && r < nx;
-    return clampn(r, nx);
+  const uint32_t jcol = 8u * (uint32_t)col.j;
+  auto row_of = [&](int r) -> int { return M.x.per ? wrap_near(r, nx) : clampn(r, nx); };
+  // whether either wavefront saw a value out of range, after the next barrier
+  auto post_test = [&](bool bad, int slot) {
+    const bool any = __any(bad);
+    if (lane == 0) sh.out_of_range[slot][ROLE] = any ? 1 : 0;
+  };
+  auto tested_out = [&](int slot) -> bool {
+    return __builtin_amdgcn_readfirstlane(sh.out_of_range[slot][0] | sh.out_of_range[slot][1]) != 0;
   };
 
-  double q[4][NQ];      // rotating window of rows r-1 .. r+2
-  double v[2][3], p[2];  // v and press of rows r and r+1
-  double Px[NQ];         // flux of row r's lower x-face (the upper face of row r-1)
-  double xiv[2][3], xip[2], xib0[2], xib1[2];   // interpolated values of the lower/upper x-face
+  Row<ROLE> w[4], next;       // rotating window of rows r-1 .. r+2, and row r+3 arriving
+  double v[2][NV], p[2];      // velocities and (fluid) pressure of rows r and r+1
+  double Px[NQ];              // flux through row r's lower x-face
+  double gdx, grdx;           // size of row r's cells
+  double xiv[NV], xip = 0.0, xib0 = 0.0, xib1 = 0.0;   // interpolated values of that face
+  auto derive = [&](const Row<ROLE>& r, double* vv, double& pp) {
+    if constexpr (ROLE == FLUID) {
+      velocities<IN, NV>(r.q[Q_RHO], r.q + Q_MX, vv);
+      pp = r.q[Q_TE] * K.gm1;                          // press = (gamma-1) te (idealmhd.cpp:253)
+    } else {
+      velocities<IN, NV>(r.rho, r.m, vv);
+      pp = 0.0;
+    }
+  };
 
-  {  // prologue: rows r0-2 .. r0+1 and the lower face of row r0
-    bool ok;
-    int i;
-    i = row_of(r0 - 2, ok); load_row(a, i, ok, j, jvalid, q[3]);
-    i = row_of(r0 - 1, ok); load_row(a, i, ok, j, jvalid, q[0]);
-    i = row_of(r0, ok);     load_row(a, i, ok, j, jvalid, q[1]);
-    i = row_of(r0 + 1, ok); load_row(a, i, ok, j, jvalid, q[2]);
-    double vt[3], pt;
-    derive(q[0], K, vt, pt);
-    derive(q[1], K, v[0], p[0]);
-    const FaceGeom gx = face_geom(M.x, r0);
-    const FaceDir fd = face_velocity<0>(vt, v[0], pt, p[0], gx, xiv[0], xip[0]);
+  {  // prologue: rows rs-2 .. rs+1 and the lower x-face of row rs
+    load_row<ROLE>(a, row_of(rs - 2), jcol, w[3]);
+    load_row<ROLE>(a, row_of(rs - 1), jcol, w[0]);
+    load_row<ROLE>(a, row_of(rs), jcol, w[1]);
+    load_row<ROLE>(a, row_of(rs + 1), jcol, w[2]);
+    load_row<ROLE>(a, row_of(rs + 2), jcol, next);
+    if (IN) {
+      post_test(w[3].out_of_range() || w[0].out_of_range() || w[1].out_of_range() || w[2].out_of_range(), (rs + 1) & 1);
+      block_barrier();
+      if (tested_out((rs + 1) & 1)) return rs;
+    }
+    double vt[NV], pt;
+    derive(w[0], vt, pt);
+    derive(w[1], v[0], p[0]);
+    const FaceGeom gx = face_geom(M.x, rs);
+    gdx = gx.d;
+    grdx = gx.rd;
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (ROLE == FIELD || k == 0) xiv[k] = interp<IN>(gx, vt[k], v[0][k]);
+    if (ROLE == FLUID) xip = interp<IN>(gx, pt, p[0]);
+    const FaceDir fd = face_dir(xiv[0], gx);
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
       double d2;
-      Px[k] = face_flux(q[3][k], q[0][k], q[1][k], q[2][k], gx, fd, d2);
-      if (k == Q_BIY) xib0[0] = d2;
-      if (k == Q_BIZ) xib1[0] = d2;
+      Px[k] = face_flux<IN>(w[3].q[k], w[0].q[k], w[1].q[k], w[2].q[k], gx, fd, d2);
+      if (ROLE == FIELD && k == Q_BIY) xib0 = d2;
+      if (ROLE == FIELD && k == Q_BIZ) xib1 = d2;
     }
   }
 
-  auto step = [&](auto BC, int r) {
+  // one row; false when the march ends before it
+  auto step = [&](auto BC, int r) -> bool {
     constexpr int B = decltype(BC)::value;
     constexpr int SM = B % 4, S0 = (B + 1) % 4, S1 = (B + 2) % 4, S2 = (B + 3) % 4;
     constexpr int D0 = B % 2, D1 = (B + 1) % 2;
-    bool ok;
-    // row r+2 is loaded first and arrives while row r's y-faces are computed
-    const int i2 = row_of(r + 2, ok);
-    load_row(a, i2, ok, j, jvalid, q[S2]);
-    if (r >= nx) return;
-    const int i = row_of(r, ok);
-    // lower y-face of this lane's column in row r (cells j-2, j-1, j, j+1 from neighbouring lanes),
-    // one transported quantity at a time: the upper y-face of the column is the next lane's lower one
-    double fyiv[3], fyip, fyib0 = 0.0, fyib1 = 0.0;
-    double vm1[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) vm1[k] = shr1(v[D0][k]);
-    // geometry of this lane's lower y-face (between j-1 and j), re-read per row (cached) rather
-    // than held in registers for the whole strip
-    const FaceGeom gy = face_geom(M.y, j);
-    const double dy = M.y.d[j], rdy = M.y.rd[j];
-    const FaceDir fdy = face_velocity<1>(vm1, v[D0], shr1(p[D0]), p[D0], gy, fyiv, fyip);
+    if (r >= rend) return false;
+    const int slot = r & 1;
+    // row r+2 was asked for a row ago; row r+3, the update's base and gravity are on their way while
+    // row r is computed
+    w[S2] = next;
+    load_row<ROLE>(a, row_of(r + 3), jcol, next);
+    const size_t row = (size_t)r * ny;
+    uint32_t jb = jcol;
+    lane_offset(jb);
+    double b[NO], grx = 0.0, gry = 0.0;
+    if constexpr (ROLE == FLUID) {
+      if (!SAME) {
+        b[0] = ld_row(a.B.rho, row, jb); b[1] = ld_row(a.B.mx, row, jb); b[2] = ld_row(a.B.my, row, jb);
+        b[3] = ld_row(a.B.mz, row, jb); b[4] = ld_row(a.B.te, row, jb);
+      }
+      grx = ld_row(a.st.gx, row & a.row_mask[ST_GX], jb);
+      gry = ld_row(a.st.gy, row & a.row_mask[ST_GY], jb);
+    } else if (!SAME) {
+      b[0] = ld_row(a.B.bx, row, jb); b[1] = ld_row(a.B.by, row, jb); b[2] = ld_row(a.B.bz, row, jb);
+    }
+    const FaceGeom gx = face_geom(M.x, r + 1);
+    const double dx = gdx, rdx = grdx;   // cell r's size came with its lower face
+    gdx = gx.d;
+    grdx = gx.rd;
+    // lower y-face of this lane's column in row r (cells j-2, j-1, j, j+1 from neighbouring lanes):
+    // the upper y-face of the column is the next lane's lower one
+    const FaceGeom gy = get_ygeom(sh, lane);
+    auto ddx = [&](double up, double lo) { return qdiv_t<IN>(up - lo, dx, rdx); };
+    auto ddy = [&](double lo) { return qdiv_t<IN>(shl1(lo) - lo, gy.d, gy.rd); };
+    const double fvy = interp<IN>(gy, shr1(v[D0][1]), v[D0][1]);
+    const FaceDir fdy = face_dir(fvy, gy);
+    // derivative1D along y (derivs.cpp:259)
+    const double dvy_y = ddy(fvy);
+    double dpy = 0.0, dvx_y = 0.0, dvz_y = 0.0, dbix_y = 0.0, dbiz_y = 0.0;
+    if constexpr (ROLE == FLUID) {
+      dpy = ddy(interp<IN>(gy, shr1(p[D0]), p[D0]));
+    } else {
+      dvx_y = ddy(interp<IN>(gy, shr1(v[D0][0]), v[D0][0]));
+      dvz_y = ddy(interp<IN>(gy, shr1(v[D0][2]), v[D0][2]));
+    }
     double tdiv[NQ];       // y part first; the x part is added when the upper x-face is known
 #pragma unroll
     for (int k = 0; k < NQ; ++k) {
-      const double qc_k = q[S0][k];
-      const double qm1 = shr1(qc_k);
+      const double qc = w[S0].q[k];
+      const double qm1 = shr1(qc);
       const double qm2 = shr1(qm1);
-      const double qp1 = shl1(qc_k);
+      const double qp1 = shl1(qc);
       double d2;
-      const double Pl = face_flux(qm2, qm1, qc_k, qp1, gy, fdy, d2);
-      // y-faces feed derivative1D(bi_x, 1) and derivative1D(bi_z, 1)
-      if (k == Q_BIX) fyib0 = d2;
-      if (k == Q_BIZ) fyib1 = d2;
-      tdiv[k] = qdiv(shl1(Pl) - Pl, dy, rdy);
+      const double Pl = face_flux<IN>(qm2, qm1, qc, qp1, gy, fdy, d2);
+      if (ROLE == FIELD && k == Q_BIX) dbix_y = ddy(d2);
+      if (ROLE == FIELD && k == Q_BIZ) dbiz_y = ddy(d2);
+      tdiv[k] = ddy(Pl);
     }
-    const double ivu0 = shl1(fyiv[0]), ivu1 = shl1(fyiv[1]), ivu2 = shl1(fyiv[2]);
-    const double ipu = shl1(fyip), ibu0 = shl1(fyib0), ibu1 = shl1(fyib1);
+    // row r+2: its values are the only ones of row r's stencil not tested yet
+    if (IN) post_test(w[S2].out_of_range(), slot);
     // upper x-face of row r from rows r-1 .. r+2; divergence term (up - lo)/dx + y term
-    derive(q[S1], K, v[D1], p[D1]);
-    const double dx = M.x.d[i], rdx = M.x.rd[i];
+    derive(w[S1], v[D1], p[D1]);
+    double dpx = 0.0, dvx_x = 0.0, dvy_x = 0.0, dvz_x = 0.0, dbiy_x = 0.0, dbiz_x = 0.0;
     {
-      const FaceGeom gx = face_geom(M.x, r + 1);
-      const FaceDir fd = face_velocity<0>(v[D0], v[D1], p[D0], p[D1], gx, xiv[D1], xip[D1]);
+      double niv[NV];
+#pragma unroll
+      for (int k = 0; k < NV; ++k)
+        if (ROLE == FIELD || k == 0) niv[k] = interp<IN>(gx, v[D0][k], v[D1][k]);
+      const FaceDir fd = face_dir(niv[0], gx);
+      dvx_x = ddx(niv[0], xiv[0]);
+      xiv[0] = niv[0];
+      if constexpr (ROLE == FLUID) {
+        const double nip = interp<IN>(gx, p[D0], p[D1]);
+        dpx = ddx(nip, xip);
+        xip = nip;
+      } else {
+        dvy_x = ddx(niv[1], xiv[1]);
+        dvz_x = ddx(niv[2], xiv[2]);
+        xiv[1] = niv[1];
+        xiv[2] = niv[2];
+      }
 #pragma unroll
       for (int k = 0; k < NQ; ++k) {
         double d2;
-        const double Pn = face_flux(q[SM][k], q[S0][k], q[S1][k], q[S2][k], gx, fd, d2);
-        // x-faces feed derivative1D(bi_y, 0) and derivative1D(bi_z, 0)
-        if (k == Q_BIY) xib0[D1] = d2;
-        if (k == Q_BIZ) xib1[D1] = d2;
-        const double tx = qdiv(Pn - Px[k], dx, rdx);
+        const double Pn = face_flux<IN>(w[SM].q[k], w[S0].q[k], w[S1].q[k], w[S2].q[k], gx, fd, d2);
+        if (ROLE == FIELD && k == Q_BIY) { dbiy_x = ddx(d2, xib0); xib0 = d2; }
+        if (ROLE == FIELD && k == Q_BIZ) { dbiz_x = ddx(d2, xib1); xib1 = d2; }
+        const double tx = ddx(Pn, Px[k]);
         tdiv[k] = tx + tdiv[k];
         Px[k] = Pn;
       }
     }
-    if (!out_lane) return;
-    const size_t c = (size_t)i * ny + j;
-    double k8[8];
-    if (i >= M.x.lo && i <= M.x.hi && yint) {
-      auto ddx = [&](double up, double lo) { return qdiv(up - lo, dx, rdx); };
-      auto ddy = [&](double up, double lo) { return qdiv(up - lo, dy, rdy); };
-      const double dpx = ddx(xip[D1], xip[D0]), dpy = ddy(ipu, fyip);
-      const double dvx_x = ddx(xiv[D1][0], xiv[D0][0]), dvx_y = ddy(ivu0, fyiv[0]);
-      const double dvy_x = ddx(xiv[D1][1], xiv[D0][1]), dvy_y = ddy(ivu1, fyiv[1]);
-      const double dvz_x = ddx(xiv[D1][2], xiv[D0][2]), dvz_y = ddy(ivu2, fyiv[2]);
-      const double dbiy_x = ddx(xib0[D1], xib0[D0]), dbix_y = ddy(ibu0, fyib0);
-      const double dbiz_x = ddx(xib1[D1], xib1[D0]), dbiz_y = ddy(ibu1, fyib1);
-      const double* qc = q[S0];
-      const double rho = qc[Q_RHO];
-      const double press = p[D0];
-      const double vx = v[D0][0], vy = v[D0][1], vz = v[D0][2];
+    const double* qc = w[S0].q;
+    if constexpr (ROLE == FIELD) {
+      // the momentum equations' field terms (idealmhd.cpp:54-60), in the order they are summed
       const double bix = qc[Q_BIX], biy = qc[Q_BIY], biz = qc[Q_BIZ];
       const double bex = qc[Q_BEX], bey = qc[Q_BEY], bez = qc[Q_BEZ];
-      const double curl_db = qdiv(dbiy_x - dbix_y, 4.0 * PI, K.r4pi);
-      const double ext0 = (-curl_db) * bey, ext1 = curl_db * bex;
-      const double in0 = (-curl_db) * biy, in1 = curl_db * bix;
+      const double curl_db = qdiv_t<IN>(dbiy_x - dbix_y, 4.0 * PI, K.r4pi);
       const double cz0 = dbiz_y, cz1 = -dbiz_x;
-      const double bzi = qdiv(biz, 4.0 * PI, K.r4pi), bze = qdiv(bez, 4.0 * PI, K.r4pi);
-      const double inz0 = bzi * cz1, inz1 = (-bzi) * cz0;
-      const double extz0 = bze * cz1, extz1 = (-bze) * cz0;
-      const double fz_ext = qdiv(cz0 * bey - cz1 * bex, 4.0 * PI, K.r4pi);
-      const double fz_in = qdiv(cz0 * biy - cz1 * bix, 4.0 * PI, K.r4pi);
-      k8[0] = -tdiv[Q_RHO] + 0.0;
-      k8[1] = (-tdiv[Q_MX] - dpx + rho * a.st.gx[c] + ext0 + in0 + inz0 + extz0) + (rho * 0.0 + vx * 0.0);
-      k8[2] = (-tdiv[Q_MY] - dpy + rho * a.st.gy[c] + ext1 + in1 + inz1 + extz1) + (rho * 0.0 + vy * 0.0);
-      k8[3] = (-tdiv[Q_MZ] + fz_ext + fz_in) + (rho * 0.0 + vz * 0.0);
-      k8[4] = (-tdiv[Q_TE] - press * (dvx_x + dvy_y)) + 0.0;
-      k8[5] = (-tdiv[Q_BIX] - tdiv[Q_BEX] + (bix + bex) * dvx_x + (biy + bey) * dvx_y) + 0.0;
-      k8[6] = (-tdiv[Q_BIY] - tdiv[Q_BEY] + (bix + bex) * dvy_x + (biy + bey) * dvy_y) + 0.0;
-      k8[7] = (-tdiv[Q_BIZ] - tdiv[Q_BEZ] + (bix + bex) * dvz_x + (biy + bey) * dvz_y) + 0.0;
+      const double bzi = qdiv_t<IN>(biz, 4.0 * PI, K.r4pi), bze = qdiv_t<IN>(bez, 4.0 * PI, K.r4pi);
+      double(*f)[64] = sh.force[slot];
+      f[F_EXT0][lane] = (-curl_db) * bey;
+      f[F_EXT1][lane] = curl_db * bex;
+      f[F_IN0][lane] = (-curl_db) * biy;
+      f[F_IN1][lane] = curl_db * bix;
+      f[F_INZ0][lane] = bzi * cz1;
+      f[F_INZ1][lane] = (-bzi) * cz0;
+      f[F_EXTZ0][lane] = bze * cz1;
+      f[F_EXTZ1][lane] = (-bze) * cz0;
+      f[F_ZEXT][lane] = qdiv_t<IN>(cz0 * bey - cz1 * bex, 4.0 * PI, K.r4pi);
+      f[F_ZIN][lane] = qdiv_t<IN>(cz0 * biy - cz1 * bix, 4.0 * PI, K.r4pi);
+    }
+    block_barrier();
+    if (IN && tested_out(slot)) return false;
+    if (!col.out) return true;
+    double k8[NO];
+    if (r >= M.x.lo && r <= M.x.hi && col.interior) {
+      if constexpr (ROLE == FLUID) {
+        const double rho = qc[Q_RHO], vx = v[D0][0], vy = v[D0][1];
+        const double(*f)[64] = sh.force[slot];
+        k8[0] = -tdiv[Q_RHO] + 0.0;
+        k8[1] = (-tdiv[Q_MX] - dpx + rho * grx + f[F_EXT0][lane] + f[F_IN0][lane] + f[F_INZ0][lane] + f[F_EXTZ0][lane]) +
+                (IN ? 0.0 : rho * 0.0 + vx * 0.0);
+        k8[2] = (-tdiv[Q_MY] - dpy + rho * gry + f[F_EXT1][lane] + f[F_IN1][lane] + f[F_INZ1][lane] + f[F_EXTZ1][lane]) +
+                (IN ? 0.0 : rho * 0.0 + vy * 0.0);
+        // v_z enters only through v_z * 0 (NaN or a zero's sign)
+        k8[3] = (-tdiv[Q_MZ] + f[F_ZEXT][lane] + f[F_ZIN][lane]) +
+                (IN ? 0.0 : rho * 0.0 + (qc[Q_MZ] / rho) * 0.0);
+        k8[4] = (-tdiv[Q_TE] - p[D0] * (dvx_x + dvy_y)) + 0.0;
+      } else {
+        const double btx = qc[Q_BIX] + qc[Q_BEX], bty = qc[Q_BIY] + qc[Q_BEY];
+        k8[0] = (-tdiv[Q_BIX] - tdiv[Q_BEX] + btx * dvx_x + bty * dvx_y) + 0.0;
+        k8[1] = (-tdiv[Q_BIY] - tdiv[Q_BEY] + btx * dvy_x + bty * dvy_y) + 0.0;
+        k8[2] = (-tdiv[Q_BIZ] - tdiv[Q_BEZ] + btx * dvz_x + bty * dvz_y) + 0.0;
+      }
     } else if (a.moc) {  // open_moc ghost cells: masked RHS (0) + characteristic terms (idealmhd.cpp:99-103)
 #pragma unroll
-      for (int w = 0; w < 8; ++w) k8[w] = 0.0 + a.moc[w * N + c];
+      for (int o = 0; o < NO; ++o) k8[o] = 0.0 + ld_row(a.moc, (O0 + o) * N + row, jb);
     } else {
 #pragma unroll
-      for (int w = 0; w < 8; ++w) k8[w] = 0.0;
+      for (int o = 0; o < NO; ++o) k8[o] = 0.0;
     }
     for (int e = 0; e < a.n_extra; ++e) {
 #pragma unroll
-      for (int w = 0; w < 8; ++w)
-        if (w == a.extra_var[e]) k8[w] = k8[w] + a.extra[e][c];
+      for (int o = 0; o < NO; ++o)
+        if (O0 + o == a.extra_var[e]) k8[o] = k8[o] + ld_row(a.extra[e], row, jb);
     }
     if (MODE == STAGE_STORE_K) {
 #pragma unroll
-      for (int w = 0; w < 8; ++w) a.kbuf[w * N + c] = k8[w];
+      for (int o = 0; o < NO; ++o) st_row(a.kbuf, (O0 + o) * N + row, jb, k8[o]);
     } else if (MODE == STAGE_RK4_FINAL) {
 #pragma unroll
-      for (int w = 0; w < 8; ++w) {
-        const double k1 = a.kbuf[w * N + c], k2 = a.k2buf[w * N + c], k3 = a.k3buf[w * N + c];
-        k8[w] = qdiv(k1 + k8[w], 6.0, K.r6) + qdiv(k2 + k3, 3.0, K.r3);
+      for (int o = 0; o < NO; ++o) {
+        const double k1 = ld_row(a.kbuf, (O0 + o) * N + row, jb), k2 = ld_row(a.k2buf, (O0 + o) * N + row, jb),
+                     k3 = ld_row(a.k3buf, (O0 + o) * N + row, jb);
+        k8[o] = qdiv(k1 + k8[o], 6.0, K.r6) + qdiv(k2 + k3, 3.0, K.r3);
       }
       if (a.kf_out) {
 #pragma unroll
-        for (int w = 0; w < 8; ++w) a.kf_out[w * N + c] = k8[w];
+        for (int o = 0; o < NO; ++o) st_row(a.kf_out, (O0 + o) * N + row, jb, k8[o]);
       }
     }
-    double b[8];
-    if (a.B.rho == a.S.rho) {
-      b[0] = q[S0][Q_RHO]; b[1] = q[S0][Q_MX]; b[2] = q[S0][Q_MY]; b[3] = q[S0][Q_MZ];
-      b[4] = q[S0][Q_TE]; b[5] = q[S0][Q_BIX]; b[6] = q[S0][Q_BIY]; b[7] = q[S0][Q_BIZ];
-    } else {
-      b[0] = a.B.rho[c]; b[1] = a.B.mx[c]; b[2] = a.B.my[c]; b[3] = a.B.mz[c];
-      b[4] = a.B.te[c]; b[5] = a.B.bx[c]; b[6] = a.B.by[c]; b[7] = a.B.bz[c];
+    if (SAME) {
+#pragma unroll
+      for (int o = 0; o < NO; ++o) b[o] = ROLE == FLUID ? qc[o] : qc[2 * o];
     }
-    const double rho_new = b[0] + k8[0] * stepv;
-    const double rho1 = smax(qdiv(rho_new, K.m, K.rm), K.nmin) * K.m;
-    const double te1 = smax(b[4] + k8[4] * stepv, K.temin);
-    const double n = smax(qdiv(rho1, K.m, K.rm), K.nmin);
-    a.T.rho[c] = n * K.m;
-    if (a.write_n) a.T.n[c] = n;
-    if (a.write_pre) a.T.rho_pre[c] = rho1;
-    a.T.mx[c] = b[1] + k8[1] * stepv;
-    a.T.my[c] = b[2] + k8[2] * stepv;
-    a.T.mz[c] = b[3] + k8[3] * stepv;
-    a.T.te[c] = smax(te1, K.temin);
-    a.T.bx[c] = b[5] + k8[5] * stepv;
-    a.T.by[c] = b[6] + k8[6] * stepv;
-    a.T.bz[c] = b[7] + k8[7] * stepv;
+    if constexpr (ROLE == FLUID) {
+      const double rho_new = b[0] + k8[0] * stepv;
+      const double rho1 = smax(qdiv(rho_new, K.m, K.rm), K.nmin) * K.m;
+      const double te1 = smax(b[4] + k8[4] * stepv, K.temin);
+      const double n = smax(qdiv(rho1, K.m, K.rm), K.nmin);
+      st_row(a.T.rho, row, jb, n * K.m);
+      if (a.write_n) st_row(a.T.n, row, jb, n);
+      if (a.write_pre) st_row(a.T.rho_pre, row, jb, rho1);
+      st_row(a.T.mx, row, jb, b[1] + k8[1] * stepv);
+      st_row(a.T.my, row, jb, b[2] + k8[2] * stepv);
+      st_row(a.T.mz, row, jb, b[3] + k8[3] * stepv);
+      st_row(a.T.te, row, jb, smax(te1, K.temin));
+    } else {
+      st_row(a.T.bx, row, jb, b[0] + k8[0] * stepv);
+      st_row(a.T.by, row, jb, b[1] + k8[1] * stepv);
+      st_row(a.T.bz, row, jb, b[2] + k8[2] * stepv);
+    }
+    return true;
   };
 
-  for (int r = r0; r < r0 + R; r += 4) {
-    step(std::integral_constant<int, 0>{}, r);
-    step(std::integral_constant<int, 1>{}, r + 1);
-    step(std::integral_constant<int, 2>{}, r + 2);
-    step(std::integral_constant<int, 3>{}, r + 3);
+  for (int r = rs; r < rend; r += 4) {
+    if (!step(std::integral_constant<int, 0>{}, r)) return r;
+    if (!step(std::integral_constant<int, 1>{}, r + 1)) return r + 1;
+    if (!step(std::integral_constant<int, 2>{}, r + 2)) return r + 2;
+    if (!step(std::integral_constant<int, 3>{}, r + 3)) return r + 3;
   }
+  return rend;
+}
+
+template <int ROLE, int MODE, bool SAME>
+__device__ __forceinline__ void strip_rows(const StageArgs& a, const Column& col, Shared& sh, double stepv, int r,
+                                           int rend) {
+  if (a.in_range) r = march<ROLE, MODE, true, SAME>(a, col, sh, stepv, r, rend);
+  if (r < rend) (void)march<ROLE, MODE, false, SAME>(a, col, sh, stepv, r, rend);
+}
+
+template <int MODE, bool SAME>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+k_mhd_stage_strip(StageArgs a, int R, int nstrips) {
+  const Mesh& M = a.mesh;
+  __shared__ Shared sh;
+  const int lane = threadIdx.x;
+  int tile, strip;
+  strip_of(blockIdx.x, nstrips, gridDim.x, tile, strip);
+  const int jraw = tile * OUT_COLS + lane - 2;
+  Column col;
+  bool valid = true;
+  if (M.y.per) col.j = wrapn(jraw, M.ny);
+  else { valid = jraw >= 0 && jraw < M.ny; col.j = clampn(jraw, M.ny); }
+  col.out = lane >= 2 && lane < 62 && jraw >= 0 && jraw < M.ny;
+  col.interior = valid && col.j >= M.y.lo && col.j <= M.y.hi;
+  const double stepv = a.step_mult * (*a.step);
+  const int r0 = strip * R, rend = min(r0 + R, M.nx);
+  put_ygeom(sh, M.y, col.j, lane);   // both wavefronts write, and each reads, the same values
+  if (__builtin_amdgcn_readfirstlane(threadIdx.y) == 0) strip_rows<FLUID, MODE, SAME>(a, col, sh, stepv, r0, rend);
+  else strip_rows<FIELD, MODE, SAME>(a, col, sh, stepv, r0, rend);
 }
 
 }  // namespace
 
 int mhd_strip_rows_default(int nx, int ny) {
-  // the tallest strip that still leaves about 32 wavefronts per CU (256 CUs); shorter strips re-read
-  // more halo rows, but on 2048x2048 and 512x1024 the extra waves hide more latency than that costs
+  // 1024 blocks (2 wavefronts per SIMD) run at once and a strip costs its rows plus about three (four
+  // halo rows read, one face and the start of the pipeline): the height with the least rounds x cost,
+  // the taller one of equals, which reads fewer halo rows
   const long tiles = (ny + OUT_COLS - 1) / OUT_COLS;
-  for (int R : {32, 16, 8}) {
-    const long waves = tiles * ((nx + R - 1) / R);
-    if (waves >= 8192) return R;
+  int best = 1;
+  long least = 0;
+  for (int R = 1; R <= 96; ++R) {
+    const long rounds = (tiles * ((nx + R - 1) / R) + 1023) / 1024;
+    const long cost = rounds * (R + 3);
+    if (R == 1 || cost <= least) { best = R; least = cost; }
   }
-  return 4;
-}
-
-int mhd_stage_kernel_default(int nx, int ny) {
-  // with 4-row strips a 256x256 grid gives 320 wavefronts, too few to fill 256 CUs (strips 49 us,
-  // one thread per cell 30 us, 8x8 tiles 21 us per stage); from about four wavefronts per CU on
-  // (512x512: strips 127 us per step, tiles 139 us), the strips are faster
-  const long waves = (long)((ny + OUT_COLS - 1) / OUT_COLS) * ((nx + 3) / 4);
-  return waves >= 1024 ? 0 : 2;
+  return best;
 }
 
 void launch_mhd_stage_strip(const StageArgs& a, int R, hipStream_t s) {
   const int cols = (a.mesh.ny + OUT_COLS - 1) / OUT_COLS, nstrips = (a.mesh.nx + R - 1) / R;
   const dim3 grid(cols * nstrips);
-  if (a.mode == STAGE_STORE_K)
-    hipLaunchKernelGGL(k_mhd_stage_strip<STAGE_STORE_K>, grid, dim3(64), 0, s, a, R, nstrips);
-  else if (a.mode == STAGE_RK4_FINAL)
-    hipLaunchKernelGGL(k_mhd_stage_strip<STAGE_RK4_FINAL>, grid, dim3(64), 0, s, a, R, nstrips);
-  else
-    hipLaunchKernelGGL(k_mhd_stage_strip<STAGE_PLAIN>, grid, dim3(64), 0, s, a, R, nstrips);
+  const bool same = a.B.rho == a.S.rho;
+  auto go = [&](auto mode) {
+    constexpr int M = decltype(mode)::value;
+    if (same) hipLaunchKernelGGL((k_mhd_stage_strip<M, true>), grid, dim3(64, 2), 0, s, a, R, nstrips);
+    else hipLaunchKernelGGL((k_mhd_stage_strip<M, false>), grid, dim3(64, 2), 0, s, a, R, nstrips);
+  };
+  if (a.mode == STAGE_STORE_K) go(std::integral_constant<int, STAGE_STORE_K>{});
+  else if (a.mode == STAGE_RK4_FINAL) go(std::integral_constant<int, STAGE_RK4_FINAL>{});
+  else go(std::integral_constant<int, STAGE_PLAIN>{});
 }
 
 }  // namespace spruce

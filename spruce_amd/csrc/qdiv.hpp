@@ -30,6 +30,21 @@ SPRUCE_QD double qdiv(double a, double b, double rb) {
   return a / b;
 }
 
+// qdiv without its range test, for operands known to be in range: a is 0, or |a| and |a/b| lie in
+// 2^-960 .. 2^900.  The residual b*q - a is then exact (its last place is at least 2^(-960-105)) and
+// the result is RN(a/b) by the same theorem.  A zero a gives q = a, residual +0 and -0*rb + q = q, so
+// the quotient keeps the sign of a as a/b does.  Straight-line code: a stencil's dozens of divisions
+// interleave instead of each ending a basic block, and cost 3 instructions instead of about 9.
+SPRUCE_QD double qdiv_in(double a, double b, double rb) {
+  const double q = a * rb;
+  const double r = fma(b, q, -a);
+  return fma(-r, rb, q);
+}
+template <bool IN>
+SPRUCE_QD double qdiv_t(double a, double b, double rb) {
+  return IN ? qdiv_in(a, b, rb) : qdiv(a, b, rb);
+}
+
 // whether qdiv takes the corrected-reciprocal path for (a, q = a*rb)
 SPRUCE_QD bool qdiv_safe(double a, double q) {
   return fabs(q) > 0x1p-900 && fabs(q) < 0x1p+900 && fabs(a) > 0x1p-900;

@@ -1,0 +1,84 @@
+"""Values outside the range of the strip kernels' untested divisions take the tested ones, bit for bit.
+
+Each case plants values out of range (range.hpp) in part of the grid, or takes the mesh or the external
+field out of range, and compares every evolved grid and step size with the CPU restatement.
+"""
+import numpy as np
+import pytest
+
+from oracle.oracle import OracleDomain
+from spruce_amd import workloads as W
+from spruce_amd.gpu import GpuDomain
+from spruce_amd.spec import spec_from_files
+
+pytestmark = pytest.mark.gpu
+EVOLVED = ("rho", "mom_x", "mom_y", "mom_z", "thermal_energy", "bi_x", "bi_y", "bi_z")
+
+
+def wave(nx, ny, integrator, bc, d=1e7):
+    st = W.periodic_wave_state(nx, ny, d=d, seed=nx)
+    g = st.grids
+    g["mom_z"] = 1e-3 * g["mom_y"]
+    g["bi_z"] = np.full((nx, ny), 0.5)
+    return st, W.base_config("ideal_mhd", bc, integrator, epsilon=0.2, density_min=1.0, temp_min=1.0,
+                             thermal_energy_min=1e-12, open_boundary_strength=0.1, open_boundary_decay_base=0.9)
+
+
+def plant(st, what):
+    g, i, j = st.grids, st.xdim // 2, st.ydim // 2
+    if what == "tiny":          # below 2^-170, and denormal
+        g["mom_z"][i:, :] = 1e-60
+        g["bi_z"][:, :j] = 1e-200
+        g["mom_y"][i, j] = 5e-310
+    elif what == "one":         # a single cell: its strips stop at it
+        g["bi_x"][i, j] = -3e-58
+    elif what == "large":       # above 2^150
+        g["bi_y"][i, j] = 1e46
+    elif what == "zeros":       # in range: both signs of zero
+        for k in ("mom_z", "bi_z"):
+            g[k][:] = 0.0
+        g["mom_z"][i:, :] = -0.0
+    elif what == "be":
+        g["be_x"] = np.full((st.xdim, st.ydim), 1e-60)
+
+
+def check(st, cfg, options, steps=3):
+    spec = spec_from_files(cfg, st)
+    gpu, ora = GpuDomain(spec, options), OracleDomain(spec)
+    try:
+        a, b = gpu.step(steps), ora.step(steps)
+        assert np.array_equal(a.view(np.int64), b.view(np.int64)), (a, b)
+        for v in EVOLVED:
+            x, y = gpu.grid(v), ora.grid(v)
+            assert np.array_equal(x.view(np.int64), y.view(np.int64)) or np.array_equal(x, y, equal_nan=True), \
+                (v, np.argwhere(x != y)[:4])
+    finally:
+        gpu.close()
+        ora.close()
+
+
+PERIODIC, CLOSED = ("periodic",) * 4, ("fixed", "reflect", "reflect", "fixed")
+
+
+@pytest.mark.parametrize("what", ["tiny", "one", "large", "zeros", "be"])
+@pytest.mark.parametrize("integrator,bc", [("rk2", PERIODIC), ("rk4", CLOSED), ("euler", ("periodic", "periodic", "fixed", "open"))])
+def test_planted_values(what, integrator, bc):
+    st, cfg = wave(23, 124, integrator, bc)
+    plant(st, what)
+    check(st, cfg, {"stage_kernel": "strip", "strip_rows": 8})
+
+
+@pytest.mark.parametrize("nx,ny,rows", [(5, 5, 4), (9, 59, 4), (13, 60, 8), (16, 61, 16), (33, 121, 12)])
+@pytest.mark.parametrize("bc", [PERIODIC, CLOSED])
+def test_tile_edges(nx, ny, rows, bc):
+    if bc is CLOSED:
+        nx, ny = max(nx, 7), max(ny, 7)
+    st, cfg = wave(nx, ny, "rk2", bc)
+    check(st, cfg, {"stage_kernel": "strip", "strip_rows": rows})
+    plant(st, "tiny")
+    check(st, cfg, {"stage_kernel": "strip", "strip_rows": rows})
+
+
+def test_mesh_out_of_range():
+    st, cfg = wave(14, 70, "rk2", PERIODIC, d=1e-15)
+    check(st, cfg, {"stage_kernel": "strip", "strip_rows": 4})
