@@ -155,9 +155,9 @@ int spruce_gpu_device_grid(spruce_gpu_domain* d, const char* name, double** dev_
  *                    marching along x) | "tile" (8x8 tiles) | "cell" (one thread per cell, faces
  *                    recomputed per cell);
  *   "strip_rows"   = rows per strip, a multiple of 4 (default: chosen from the grid size);
- *   "tc_kernel"    = thermal-conduction update: "auto" (default: strips when 8-row strips give at
- *                    least 4096 wavefronts, else one thread per cell) | "strip" (wavefront strips,
- *                    every face computed once, b_hat derivatives formed in the kernel) | "cell";
+ *   "tc_kernel"    = thermal-conduction update: "auto" (default: strips) | "strip" (wavefront strips,
+ *                    every face computed once, b_hat derivatives formed in the kernel) | "cell" (one
+ *                    thread per cell);
  *   "tc_rows"      = rows per conduction strip, 1..256 (default: chosen from the grid size);
  *   "adjoint_tc_rows" = spruce_gpu_adjoint's reverse of Euler conduction subcycles without flux
  *                    saturation: rows per wavefront strip, 1..256, 0 (default: 8 where the grid

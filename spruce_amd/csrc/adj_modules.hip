@@ -482,30 +482,16 @@ __global__ void __launch_bounds__(64) k_adj_tc_strip(TcStepArgs a, const double*
   const int tile = t / nstrips, sidx = t - tile * nstrips;
   const int lane = threadIdx.x;
   const int jc = tile * 60 + lane - 2;
-  tcs::Lane L;
-  L.j = tcs::row_index(jc, M.ny, M.y.per, L.val);
-  L.iny = L.val && L.j >= M.y.lo && L.j <= M.y.hi;
+  tcs::Lane L = tcs::lane_at(M, jc);
   L.out = lane >= 2 && lane <= 61 && jc < M.ny;
-  {
-    bool vp;
-    const int jp = tcs::row_index(L.j + 1, M.ny, M.y.per, vp);
-    L.hc = M.y.h[jp];
-    L.hn = M.y.h[L.j];
-    L.fd = M.y.fden[jp];
-    L.rfd = M.y.rfden[jp];
-    L.dy = M.y.d[L.j];
-    L.rdy = M.y.rd[L.j];
-    L.hsq = M.y.hsq[L.j];
-    L.rhsq = M.y.rhsq[L.j];
-  }
   const bool cmp = lane >= 1 && lane <= 62 && L.val;   // reverses its cells
   const double wc = L.hc * L.rfd, wn = L.hn * L.rfd;   // d(upper y-face)/d(own value, next lane's)
   const int r0 = sidx * R, r1 = min(r0 + R, M.nx);
   tcs::Raw rw = tcs::load_raw<false>(a, L, r0 - 2);
-  const tcs::Row first = tcs::make_row<false, false>(a, L, r0 - 2, rw);
+  const tcs::Row first = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r0 - 2, rw);
   rw = tcs::load_raw<false>(a, L, r0 - 1);
-  tcs::Row cur = tcs::make_row<false, false>(a, L, r0 - 1, rw);
-  tcs::XFaces lo = tcs::xfaces<false, false>(M, first, cur);
+  tcs::Row cur = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r0 - 1, rw);
+  tcs::XFaces lo = tcs::xfaces<false, tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, cur.i), first, cur);
   double cn = rw.n;
   tcs::Raw ahead = tcs::load_raw<false>(a, L, r0);
   // adjoints of the previous row (p*) and of the face between it and the current row (f*): T, gy
@@ -518,14 +504,14 @@ __global__ void __launch_bounds__(64) k_adj_tc_strip(TcStepArgs a, const double*
   for (int r = r0 - 1; r <= r1; ++r) {
     const tcs::Raw raw = ahead;
     if (r < r1) ahead = tcs::load_raw<false>(a, L, r + 2);
-    const tcs::Row nxt = tcs::make_row<false, false>(a, L, r + 1, raw);
-    const tcs::XFaces hi = tcs::xfaces<false, false>(M, cur, nxt);
+    const tcs::Row nxt = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r + 1, raw);
+    const tcs::XFaces hi = tcs::xfaces<false, tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, nxt.i), cur, nxt);
     // the cell of row r, as the forward forms it
     const int i = cur.i;
     const double rdx = M.x.rd[i];
     const bool in = cur.inx && L.iny;
     const double gx = (hi.T - lo.T) * rdx;
-    const double dgx_y = tcs::yderiv<false>(L, tcs::yface<false>(L, in ? gx : 0.0));
+    const double dgx_y = tcs::yderiv<tcs::DIV_PRODUCT>(L, tcs::yface<tcs::DIV_PRODUCT>(L, in ? gx : 0.0));
     const bool live = cmp && cur.val;
     double lv = 0.0;
     tcc::TcCombAdj G{0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};

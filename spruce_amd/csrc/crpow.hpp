@@ -46,6 +46,32 @@ SPRUCE_HD double pow_2p5(double x) {
   return p + (pe + (a * t + ae * s));
 }
 
+#ifdef __HIPCC__
+// x^1.5 and x^2.5 for x in 2^-200 .. 2^200, from one square root: s within an ulp of sqrt(x) and
+// t = (x - s*s) / (2 s) to 2^-52 relative, so that s + t is sqrt(x) to 2^-104 as in sqrt_dd; then the
+// same double-double products, so the same correctly rounded values.  v_rsq_f64's 2^-23 is squared
+// by each of two Newton steps (Goldschmidt's form: g -> sqrt(x), h -> 1/(2 sqrt(x))).
+__device__ __forceinline__ void pow_1p5_2p5_in(double x, double& p15, double& p25) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = fma(-h, g, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  r = fma(-h, g, 0.5);
+  h = fma(h, r, h);
+  const double s = fma(fma(-g, g, x), h, g);
+  const double t = fma(-s, s, x) * h;
+  const double p = x * s;
+  const double e = fma(x, s, -p);
+  p15 = p + (e + x * t);
+  const double a = x * x;
+  const double ae = fma(x, x, -a);
+  const double q = a * s;
+  const double qe = fma(a, s, -q);
+  p25 = q + (qe + (a * t + ae * s));
+}
+#endif
+
 // x^-1.5 = 1 / (x sqrt(x))
 SPRUCE_HD double pow_m1p5(double x) {
   if (!(x > 0.0) || !(x < 0x1p+600) || !(x > 0x1p-600)) return pow(x, -1.5);

@@ -467,7 +467,7 @@ class Domain : public DomainBase {
 
     if (strip_rows == 0) strip_rows = mhd_strip_rows_default(nx, ny);
     if (tc_rows == 0) tc_rows = tc_strip_rows_default(nx, ny);
-    if (tc_kernel < 0) tc_kernel = tc_kernel_default(nx, ny);
+    if (tc_kernel < 0) tc_kernel = 0;   // the strips are the faster form at every size
     if (stage_kernel < 0) stage_kernel = 0;   // the strips are the fastest form at every size
     fuse_dt = stage_kernel == 2 && !(kinds_all[0] || kinds_all[1] || kinds_all[2] || kinds_all[3]) && !any_moc &&
               mods.empty();
@@ -1045,6 +1045,7 @@ struct TcModule : GpuModule {
     a.k1 = k1.p; a.k2 = k2.p; a.k3 = k3.p; a.h = h; a.mult = mult; a.mode = mode; a.p = p; a.k = d.kc;
     a.dbxx = dbxx.p; a.dbxy = dbxy.p; a.dbyx = dbyx.p; a.dbyy = dbyy.p;
     a.mesh = d.mesh;
+    a.in_range = d.in_range ? 1 : 0;
     a.rows = d.tc_kernel == 1 ? 0 : d.tc_rows;
     d.timed("tc_step", [&] { launch_tc_step(a, d.stream); });
   }

@@ -93,7 +93,8 @@ struct AxisBufs {
     std::vector<FaceGeom> vface(n);
     for (int c = 0; c < n; ++c) {
       const int cm1 = per ? w(c - 1) : std::max(c - 1, 0), cp1 = per ? w(c + 1) : std::min(c + 1, n - 1);
-      vface[c] = FaceGeom{vh[cm1], vh[c], vf[c], vrf[c], vgu[c], vf[cm1], vrf[cm1], vgd[c], vf[cp1], vrf[cp1], vd[c], vrd[c]};
+      vface[c] = FaceGeom{vh[cm1], vh[c], vf[c], vrf[c], vgu[c], vf[cm1], vrf[cm1], vgd[c], vf[cp1], vrf[cp1], vd[c], vrd[c],
+                          vhsq[c], vrhsq[c]};
     }
     if (face) (void)hipFree(face);
     face = nullptr;

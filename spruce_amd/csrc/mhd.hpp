@@ -12,7 +12,8 @@ struct FaceGeom {
   double hlo, hup, den, rden;
   double gup, denm, rdenm;   // extrapolation through (c-2, c-1)
   double gdn, denp, rdenp;   // extrapolation through (c+1, c)
-  double d, rd;              // cell c
+  double d, rd;              // cell c: size, (d/2)^2 and their reciprocals
+  double hsq, rhsq;
 };
 
 // One axis of the (separable) mesh: d_x depends on x only and d_y on y only, so each is a 1-D array

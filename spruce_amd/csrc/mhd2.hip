@@ -18,8 +18,9 @@
 // also waits for the rows being fetched; the split leaves room (249 registers, no spill, two
 // wavefronts per SIMD) to fetch a row two rows ahead.  Measured on 2048x2048 (RK2, periodic): 536 us
 // a stage with tested divisions and one wavefront per strip, 404 us with untested ones, 350 us with
-// the split, 290 us with the longer fetch distance, the gathered geometry and the static rows;
-// 1.09 GB of HBM traffic a launch, VALU 46% busy.  512x1024: 110 -> 40 us; 64x48: 17 (8x8 tiles) -> 9 us.
+// the split, 281 us with the longer fetch distance, the geometry gathered and read through the scalar
+// cache, and the static rows; 1.09 GB of HBM traffic a launch, VALU 46% busy.  512x1024: 110 -> 41 us;
+// 64x48: 17 (8x8 tiles) -> 9 us.
 #include <cfloat>
 #include <type_traits>
 
@@ -69,7 +70,7 @@ __device__ __forceinline__ void put_ygeom(Shared& s, const Axis& ax, int j, int 
 __device__ __forceinline__ FaceGeom get_ygeom(const Shared& s, int l) {
   const double2 a = s.geom[0][l], b = s.geom[1][l], c = s.geom[2][l], d = s.geom[3][l], e = s.geom[4][l],
                 f = s.geom[5][l];
-  return FaceGeom{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, e.x, e.y, f.x, f.y};
+  return FaceGeom{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, e.x, e.y, f.x, f.y, 0.0, 0.0};
 }
 // LDS written before is seen by both wavefronts after; loads from memory stay in flight
 __device__ __forceinline__ void block_barrier() {
@@ -145,7 +146,7 @@ __device__ __forceinline__ void load_row(const StageArgs& a, int i, uint32_t jb,
 // v = mom/rho (idealmhd.cpp:248-250), N components (the fluid's wavefront never needs v_z)
 template <bool IN, int N>
 __device__ __forceinline__ void velocities(double rho, const double* m, double* v) {
-  const double rr = 1.0 / rho;
+  const double rr = IN ? recip_in(rho) : 1.0 / rho;
 #pragma unroll
   for (int k = 0; k < N; ++k) v[k] = IN ? qdiv_in(m[k], rho, rr) : qdiv_d(m[k], rho, rr);
 }
@@ -204,7 +205,7 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
     double vt[NV], pt;
     derive(w[0], vt, pt);
     derive(w[1], v[0], p[0]);
-    const FaceGeom gx = face_geom(M.x, rs);
+    const FaceGeom gx = face_geom_row(M.x, rs);
     gdx = gx.d;
     grdx = gx.rd;
 #pragma unroll
@@ -246,7 +247,7 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
     } else if (!SAME) {
       b[0] = ld_row(a.B.bx, row, jb); b[1] = ld_row(a.B.by, row, jb); b[2] = ld_row(a.B.bz, row, jb);
     }
-    const FaceGeom gx = face_geom(M.x, r + 1);
+    const FaceGeom gx = face_geom_row(M.x, r + 1);
     const double dx = gdx, rdx = grdx;   // cell r's size came with its lower face
     gdx = gx.d;
     grdx = gx.rd;

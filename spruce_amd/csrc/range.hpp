@@ -19,6 +19,8 @@
 #include <hip/hip_runtime.h>
 #include <math.h>
 
+#include "qdiv.hpp"
+
 namespace spruce {
 
 constexpr int RANGE_G = 48;     // lengths (cell sizes, halves, face sums): 2^-48 .. 2^48
@@ -45,6 +47,16 @@ struct RangeTest {
   // frexp_exp(2^-L) is 1 - L
   __device__ __forceinline__ bool out() const { return high || emin < 1 - RANGE_L; }
 };
+
+// The reciprocal that the hardware's IEEE division of doubles works with, without the scaling its
+// extreme exponents need: qdiv_in(a, b, recip_in(b)) is then that division's own sequence, a/b
+// correctly rounded, for a and b within 2^-200 .. 2^200 (or a = 0): 8 instructions instead of 11, and
+// 3 for each further dividend.
+__device__ __forceinline__ double recip_in(double b) {
+  double y = __builtin_amdgcn_rcp(b);
+  y = fma(y, fma(-b, y, 1.0), y);
+  return fma(y, fma(-b, y, 1.0), y);
+}
 
 // The hardware's minimum and maximum: std::min and std::max where neither operand is NaN, up to the
 // sign of a zero.  Written as instructions because the compiler's own form first canonicalises both

@@ -259,90 +259,98 @@ __global__ void __launch_bounds__(256) k_tc_step(TcStepArgs a) {
 // frozen b_hat are formed here from b_hat, so a subcycle reads te, n, b_hat_x, b_hat_y and writes
 // te.  Each value is the same sequence of IEEE operations as tc_core's (tc_cell.hpp), so the result
 // is bit-identical to the one-thread-per-cell form.
-
-// Four wavefronts per SIMD (at most 128 VGPRs; the compiler spills about 16 bytes per lane, outside
-// the row loop): 79.9 us per subcycle on the 2048x2048 arcade against 84.3 us at 152 VGPRs and three
-// wavefronts per SIMD.  Reading the four b_hat derivatives from grids written once per step instead
-// of forming them here was slower (102 us): the kernel is bound by latency and issue, not by the
-// VALU work those derivatives take.
-template <int MODE, bool SAT, bool SEP>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
-k_tc_strip(TcStepArgs a, int R, int nstrips, int total) {
+//
+// What bounds it: HBM and the latency of a row's chain.  A 2048x2048 subcycle moves at least 168 MB
+// (40 B per cell), 34 us at the 4.9 TB/s a large copy reaches here; an 18-row strip's halo rows and
+// lanes make it 188 MB.  The divisions' range tests are made once per row (range.hpp) instead of at
+// each of ~20 divisions and both powers share one square root, so a row is about 250 VALU
+// instructions in one run instead of 400 in twenty pieces (1.78e7 against 2.79e7 a launch), and the
+// row's geometry comes through the scalar cache, so that nothing waits for the row being fetched but
+// its use.  Measured per subcycle: 2048x2048 79.5 -> 52.7 us, 512x1024 17.5 (one thread per cell) ->
+// 13.5 us, 133x197 7.7 -> 7.2 us.  109 VGPRs, four wavefronts per SIMD.
+//
+// Rows rs .. rend-1.  D = DIV_IN: the geometric divisions and the powers without their operand tests;
+// every row is tested once it is formed, and the march stops before the first row whose stencil holds
+// a value out of range.  Returns the row it stopped at (rend when done).
+template <int MODE, bool SAT, bool SEP, int D>
+__device__ __forceinline__ int tc_march(const TcStepArgs& a, const tcs::Lane& L, int rs, int rend) {
   using namespace tcs;
   const Mesh& M = a.mesh;
-  const int t = strip::xcd_tile(blockIdx.x, total);
-  const int tile = t / nstrips, sidx = t - tile * nstrips;
-  const int lane = threadIdx.x;
-  Lane L;
-  {
-    const int jc = tile * 62 + lane - 1;
-    L.j = row_index(jc, M.ny, M.y.per, L.val);
-    L.iny = L.val && L.j >= M.y.lo && L.j <= M.y.hi;
-    L.out = lane >= 1 && lane <= 62 && jc < M.ny;
-    bool vp;
-    const int jp = row_index(L.j + 1, M.ny, M.y.per, vp);
-    L.hc = M.y.h[jp];
-    L.hn = M.y.h[L.j];
-    L.fd = M.y.fden[jp];
-    L.rfd = M.y.rfden[jp];
-    L.dy = M.y.d[L.j];
-    L.rdy = M.y.rd[L.j];
-    L.hsq = M.y.hsq[L.j];
-    L.rhsq = M.y.rhsq[L.j];
-  }
-  const int r0 = sidx * R, r1 = min(r0 + R, M.nx);
-  Row cur = make_row<SAT>(a, L, r0, load_raw<SAT>(a, L, r0));
+  constexpr bool IN = D == DIV_IN;
+  Row cur;
+  FaceGeom g = strip::face_geom_row(M.x, rs);
   XFaces lo;
   {
-    const Row prev = make_row<SAT>(a, L, r0 - 1, load_raw<SAT>(a, L, r0 - 1));
-    lo = xfaces<SAT>(M, prev, cur);
+    const Raw rp = load_raw<SAT>(a, L, rs - 1), rc = load_raw<SAT>(a, L, rs);
+    const Row prev = make_row<SAT, D>(a, L, rs - 1, rp);
+    cur = make_row<SAT, D>(a, L, rs, rc);
+    if (IN && __any(row_out<SAT>(prev, rp) || row_out<SAT>(cur, rc))) return rs;
+    lo = xfaces<SAT, D>(g, prev, cur);
   }
-  Raw ahead = load_raw<SAT>(a, L, r0 + 1);
-  for (int r = r0; r < r1; ++r) {
+  Raw ahead = load_raw<SAT>(a, L, rs + 1);
+  for (int r = rs; r < rend; ++r) {
     const Raw raw = ahead;
-    if (r + 1 < r1) ahead = load_raw<SAT>(a, L, r + 2);
-    const Row nxt = make_row<SAT>(a, L, r + 1, raw);
-    const XFaces hi = xfaces<SAT>(M, cur, nxt);
+    ahead = load_raw<SAT>(a, L, r + 2);
+    const size_t row = (size_t)r * M.ny;
+    uint32_t jb = 8u * (uint32_t)L.j;
+    strip::lane_offset(jb);
+    const double base = SEP ? strip::ld_row(a.te_base, row, jb) : cur.te;
+    const FaceGeom gn = strip::face_geom_row(M.x, r + 1);
+    const Row nxt = make_row<SAT, D>(a, L, r + 1, raw);
+    if (IN && __any(row_out<SAT>(nxt, raw))) return r;
+    const XFaces hi = xfaces<SAT, D>(gn, cur, nxt);
     // cell values at row r along x
-    const int i = cur.i;
-    const double dx = M.x.d[i], rdx = M.x.rd[i];
+    const double dx = g.d, rdx = g.rd;
     const bool in = cur.inx && L.iny;
-    const double gx = qdiv(hi.T - lo.T, dx, rdx);
+    const double gx = qd<D>(hi.T - lo.T, dx, rdx);
     // dtemp_dx is zero outside the interior; its y-derivative takes the neighbouring lanes' values
-    const double dgx_y = yderiv(L, yface(L, in ? gx : 0.0));
-    if (L.out && cur.val) {
-      const size_t c = (size_t)i * M.ny + L.j;
-      const double base = SEP ? a.te_base[c] : cur.te;
-      if (!in) {
-        // mask = 0: te + 0*dE; every derivative is zero there, so dE = 0
-        a.te_out[c] = smax(base + 0.0, a.k.temin);
-        if (MODE == TC_STORE_K) a.k_out[c] = 0.0;
-      } else {
-        const double s0 = qdiv(hi.T - 2.0 * cur.T + lo.T, M.x.hsq[i], M.x.rhsq[i]);
-        const double dgy_x = qdiv(hi.gy - lo.gy, dx, rdx);
-        const double dbxx = qdiv(hi.bx - lo.bx, dx, rdx);
-        const double dbyx = qdiv(hi.by - lo.by, dx, rdx);
-        double dE = tcc::tc_combine<double>(cur.T, gx, cur.gy, s0, cur.s1, dgx_y, dgy_x, cur.bx, cur.by, dbxx,
-                                            cur.dbxy, dbyx, cur.dbyy, a.p.k0);
-        if (SAT) {                                              // thermalconduction.cpp:171-174, 255-271
-          const double dcx = qdiv(hi.coef - lo.coef, dx, rdx);
-          const double add = -1.0 * (dcx * a.rx[c] + cur.dcy * a.ry[c]);
-          dE = cur.coef * dE + add;
-        }
-        double v;
-        if (MODE == TC_RK4_FINAL) {
-          const double sum = a.k1[c] + 2.0 * a.k2[c] + 2.0 * a.k3[c] + dE;
-          v = base + qdiv(1.0 * a.h * sum, 6.0, a.k.r6);
-        } else {
-          if (MODE == TC_STORE_K) a.k_out[c] = dE;
-          v = base + 1.0 * (a.mult * a.h) * dE;
-        }
-        a.te_out[c] = smax(v, a.k.temin);
-      }
+    const double dgx_y = yderiv<D>(L, yface<D>(L, in ? gx : 0.0));
+    const double s0 = qd<D>(hi.T - 2.0 * cur.T + lo.T, g.hsq, g.rhsq);
+    const double dgy_x = qd<D>(hi.gy - lo.gy, dx, rdx);
+    const double dbxx = qd<D>(hi.bx - lo.bx, dx, rdx);
+    const double dbyx = qd<D>(hi.by - lo.by, dx, rdx);
+    double dE = tcc::tc_combine<double, IN>(cur.T, gx, cur.gy, s0, cur.s1, dgx_y, dgy_x, cur.bx, cur.by, dbxx, cur.dbxy,
+                                            dbyx, cur.dbyy, a.p.k0);
+    if (SAT) {                                                  // thermalconduction.cpp:171-174, 255-271
+      const double dcx = qd<D>(hi.coef - lo.coef, dx, rdx);
+      const double add = -1.0 * (dcx * strip::ld_row(a.rx, row, jb) + cur.dcy * strip::ld_row(a.ry, row, jb));
+      dE = cur.coef * dE + add;
+    }
+    dE = in ? dE : 0.0;   // every derivative is zero outside the interior
+    double v;
+    if (MODE == TC_RK4_FINAL) {
+      const double sum = strip::ld_row(a.k1, row, jb) + 2.0 * strip::ld_row(a.k2, row, jb) +
+                         2.0 * strip::ld_row(a.k3, row, jb) + dE;
+      v = base + qdiv(1.0 * a.h * sum, 6.0, a.k.r6);
+    } else {
+      v = base + 1.0 * (a.mult * a.h) * dE;
+    }
+    // mask = 0 there: te + 0*dE
+    const double te = smax(in ? v : base + 0.0, a.k.temin);
+    if (L.out) {
+      if (MODE == TC_STORE_K) strip::st_row(a.k_out, row, jb, dE);
+      strip::st_row(a.te_out, row, jb, te);
     }
     cur = nxt;
     lo = hi;
+    g = gn;
   }
+  return rend;
+}
+
+template <int MODE, bool SAT, bool SEP>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+k_tc_strip(TcStepArgs a, int R, int nstrips, int total) {
+  const Mesh& M = a.mesh;
+  const int t = strip::xcd_tile(blockIdx.x, total);
+  const int tile = t / nstrips, sidx = t - tile * nstrips;
+  const int lane = threadIdx.x, jc = tile * 62 + lane - 1;
+  tcs::Lane L = tcs::lane_at(M, jc);
+  L.out = lane >= 1 && lane <= 62 && jc < M.ny;
+  const int r0 = sidx * R, r1 = min(r0 + R, M.nx);
+  int r = r0;
+  if (a.in_range) r = tc_march<MODE, SAT, SEP, tcs::DIV_IN>(a, L, r, r1);
+  if (r < r1) (void)tc_march<MODE, SAT, SEP, tcs::DIV_TESTED>(a, L, r, r1);
 }
 
 // RadiativeLosses::computeLosses at one interior cell (radiativelosses.cpp:149-197).
@@ -469,20 +477,17 @@ void launch_tc_sat(const double* te_src, const double* n, const double* rho, con
                      coef);
 }
 
-// Measured on one MI355X: on the 2048x2048 arcade strips of 8 rows (8704 wavefronts) take 80 us
-// per subcycle, against 85 us with 4 rows, 92 us with 16 and 124 us with one thread per cell; on the
-// 512x1024 arcade the strips give too few wavefronts (2176 with 4 rows) and one thread per cell is
-// faster (20.3 us against 22.0 us).
 int tc_strip_rows_default(int nx, int ny) {
-  const int tiles = (ny + 61) / 62;
-  for (int R : {8, 4})
-    if (tiles * ((nx + R - 1) / R) >= 4096) return R;
-  return 2;
-}
-
-int tc_kernel_default(int nx, int ny) {
-  const int tiles = (ny + 61) / 62;
-  return tiles * ((nx + 7) / 8) >= 4096 ? 0 : 1;
+  // 4096 wavefronts (4 per SIMD) run at once and a strip costs its rows plus about five (three rows to
+  // start with, the launch): the height with the least rounds x cost, the taller one of equals
+  const long tiles = (ny + 61) / 62;
+  int best = 1;
+  long least = 0;
+  for (int R = 1; R <= 96; ++R) {
+    const long cost = (tiles * ((nx + R - 1) / R) + 4095) / 4096 * (R + 5);
+    if (R == 1 || cost <= least) { best = R; least = cost; }
+  }
+  return best;
 }
 
 template <int MODE, bool SAT>

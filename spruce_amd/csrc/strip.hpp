@@ -58,6 +58,15 @@ __device__ __forceinline__ FaceGeom face_geom(const Axis& ax, int c) {
   return ax.face[ax.per ? wrap_near(c, ax.n) : clampn(c, ax.n)];
 }
 
+// The same face for an index that is the same in every lane, through the scalar cache: the table never
+// changes, so its address space is the constant one.  As vector loads these would be waited for in
+// order with the rows being fetched.
+__device__ __forceinline__ FaceGeom face_geom_row(const Axis& ax, int c) {
+  using cdouble = const __attribute__((address_space(4))) double;
+  cdouble* p = reinterpret_cast<cdouble*>(reinterpret_cast<uint64_t>(ax.face + (ax.per ? wrap_near(c, ax.n) : clampn(c, ax.n))));
+  return FaceGeom{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7], p[8], p[9], p[10], p[11], p[12], p[13]};
+}
+
 // boundaryInterpolate(a at the lower cell, b at the upper cell) (derivs.cpp:477-487); IN: the
 // operands are in range (range.hpp)
 template <bool IN = false>

@@ -46,8 +46,8 @@ template <class S> __host__ __device__ __forceinline__ S zero() { return Zero<S>
 // The energy derivative from the cell's temperature Tc, its gradient (gx, gy), second derivatives
 // (s0 = d2T/dx2, s1 = d2T/dy2), the cross derivatives of the gradient (dgx_y = d(dT/dx)/dy,
 // dgy_x = d(dT/dy)/dx), b_hat and the four derivatives of b_hat (thermalconduction.cpp:158-176,
-// operation for operation).
-template <class S>
+// operation for operation).  IN (device, S = double): Tc lies in 2^-200 .. 2^200.
+template <class S, bool IN = false>
 __host__ __device__ __forceinline__ S tc_combine(const S& Tc, const S& gx, const S& gy, const S& s0, const S& s1,
                                                  const S& dgx_y, const S& dgy_x, const S& bx, const S& by,
                                                  const S& dbx_x, const S& dbx_y, const S& dby_x, const S& dby_y,
@@ -57,7 +57,12 @@ __host__ __device__ __forceinline__ S tc_combine(const S& Tc, const S& gx, const
   const S t2x = gx * dbx_x + gy * dbx_y, t2y = gx * dby_x + gy * dby_y;
   const S curl = dby_x - dbx_y;
   const S t3x = (-(-1.0 * curl)) * gy, t3y = (-1.0 * curl) * gx;
-  const S q15 = p15(Tc), q25 = p25(Tc);
+  S q15, q25;
+#ifdef __HIP_DEVICE_COMPILE__
+  if constexpr (IN) pow_1p5_2p5_in(Tc, q15, q25);
+  else
+#endif
+  { q15 = p15(Tc); q25 = p25(Tc); }
   const S ttx = 5.0 / 2.0 * q15 * gx * bdg + q25 * (t1x + t2x + t3x);
   const S tty = 5.0 / 2.0 * q15 * gy * bdg + q25 * (t1y + t2y + t3y);
   const S divb = dbx_x + dby_y;

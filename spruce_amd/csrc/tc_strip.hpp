@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "arith.hpp"
+#include "range.hpp"
 #include "solar.hpp"
 #include "strip.hpp"
 
@@ -17,6 +18,15 @@ namespace tcs {
 // temp = max((gamma-1) te / (2 K_B n), temp_min) (thermalconduction.cpp:109; idealmhd.cpp:254)
 __device__ __forceinline__ double temp_of(double te, double n, const MhdConst& K) {
   return smax(te * K.gm1 / (n * (2.0 * K_B)), K.tmin);
+}
+
+// How the geometric divisions are taken: as products with the prepared reciprocal (within an ulp; the
+// adjoint's recompute of the values its partial derivatives take), IEEE divisions (qdiv), or the same
+// without the operand test, for rows in range (range.hpp).
+enum Div { DIV_PRODUCT, DIV_TESTED, DIV_IN };
+template <int D>
+__device__ __forceinline__ double qd(double a, double b, double rb) {
+  return D == DIV_PRODUCT ? a * rb : (D == DIV_IN ? qdiv_in(a, b, rb) : qdiv(a, b, rb));
 }
 
 // one row of the strip at this lane: cell values and the quantities that need only y-neighbours
@@ -36,83 +46,106 @@ struct Lane {
   double dy, rdy, hsq, rhsq;
 };
 
+// k (at most n away from the grid) wrapped on a periodic axis, else clamped; val: whether it exists
 __device__ __forceinline__ int row_index(int k, int n, int per, bool& val) {
-  if (per) { k %= n; if (k < 0) k += n; val = true; return k; }
+  if (per) { val = true; return strip::wrap_near(k, n); }
   val = k >= 0 && k < n;
-  return k < 0 ? 0 : (k >= n ? n - 1 : k);
+  return strip::clampn(k, n);
 }
 
-// The quotient a/b: the IEEE one (EX, what the forward takes), or the product with the prepared
-// reciprocal rb (within an ulp; the adjoint's recompute of the values its partial derivatives take)
-template <bool EX>
-__device__ __forceinline__ double qd(double a, double b, double rb) {
-  return EX ? qdiv(a, b, rb) : a * rb;
+// column jc of the mesh as this lane's (out is left to the caller)
+__device__ __forceinline__ Lane lane_at(const Mesh& M, int jc) {
+  Lane L;
+  bool vp;
+  L.j = row_index(M.y.per ? strip::wrapn(jc, M.ny) : jc, M.ny, M.y.per, L.val);
+  L.iny = L.val && L.j >= M.y.lo && L.j <= M.y.hi;
+  const int jp = row_index(L.j + 1, M.ny, M.y.per, vp);
+  L.hc = M.y.h[jp];
+  L.hn = M.y.h[L.j];
+  L.fd = M.y.fden[jp];
+  L.rfd = M.y.rfden[jp];
+  L.dy = M.y.d[L.j];
+  L.rdy = M.y.rd[L.j];
+  L.hsq = M.y.hsq[L.j];
+  L.rhsq = M.y.rhsq[L.j];
+  L.out = false;
+  return L;
 }
 
 // boundaryInterpolate across this lane's upper y-face (derivs.cpp:477-487), from its own value and
 // the next lane's
-template <bool EX = true>
+template <int D>
 __device__ __forceinline__ double yface(const Lane& L, double q) {
   const double up = strip::shl1(q);
-  return qd<EX>(q * L.hc + up * L.hn, L.fd, L.rfd);
+  return qd<D>(q * L.hc + up * L.hn, L.fd, L.rfd);
 }
 // derivative1D along y at this lane from the upper faces of this lane and of the previous one
-template <bool EX = true>
+template <int D>
 __device__ __forceinline__ double yderiv(const Lane& L, double fup) {
-  return qd<EX>(fup - strip::shr1(fup), L.dy, L.rdy);
+  return qd<D>(fup - strip::shr1(fup), L.dy, L.rdy);
 }
 
+// Rows and columns outside a closed side are read from the nearest cell: what they hold reaches only
+// values that are masked.
 template <bool SAT>
 __device__ __forceinline__ Raw load_raw(const TcStepArgs& a, const Lane& L, int k) {
-  Raw r{0.0, 0.0, 0.0, 0.0, 0.0};
   bool v;
-  const int i = row_index(k, a.mesh.nx, a.mesh.x.per, v);
-  if (v && L.val) {
-    const size_t c = (size_t)i * a.mesh.ny + L.j;
-    r.te = a.te_src[c];
-    r.n = a.n[c];
-    r.bx = a.bhx[c];
-    r.by = a.bhy[c];
-    if (SAT) r.coef = a.coef[c];
-  }
+  const size_t row = (size_t)row_index(k, a.mesh.nx, a.mesh.x.per, v) * a.mesh.ny;
+  uint32_t jb = 8u * (uint32_t)L.j;
+  strip::lane_offset(jb);
+  Raw r;
+  r.te = strip::ld_row(a.te_src, row, jb);
+  r.n = strip::ld_row(a.n, row, jb);
+  r.bx = strip::ld_row(a.bhx, row, jb);
+  r.by = strip::ld_row(a.bhy, row, jb);
+  r.coef = SAT ? strip::ld_row(a.coef, row, jb) : 0.0;
   return r;
 }
 
-template <bool SAT, bool EX = true>
+template <bool SAT, int D>
 __device__ __forceinline__ Row make_row(const TcStepArgs& a, const Lane& L, int k, const Raw& r) {
   const Mesh& M = a.mesh;
   Row w;
   w.i = row_index(k, M.nx, M.x.per, w.val);
   w.inx = w.val && w.i >= M.x.lo && w.i <= M.x.hi;
-  const bool ok = w.val && L.val;
   w.te = r.te;
-  w.T = ok ? temp_of(r.te, r.n, a.k) : 0.0;
+  const double den = r.n * (2.0 * K_B);
+  w.T = D == DIV_IN ? smax(qdiv_in(r.te * a.k.gm1, den, recip_in(den)), a.k.tmin) : temp_of(r.te, r.n, a.k);
   w.bx = r.bx;
   w.by = r.by;
-  const double fT = yface<EX>(L, w.T);
+  const double fT = yface<D>(L, w.T);
   const double fTlo = strip::shr1(fT);
   // dtemp_dy is zero outside the interior (derivs.cpp:229-233)
-  w.gy = (w.inx && L.iny) ? qd<EX>(fT - fTlo, L.dy, L.rdy) : 0.0;
-  w.s1 = qd<EX>(fT - 2.0 * w.T + fTlo, L.hsq, L.rhsq);      // secondDerivative1D (derivs.cpp:450)
-  w.dbxy = yderiv<EX>(L, yface<EX>(L, w.bx));
-  w.dbyy = yderiv<EX>(L, yface<EX>(L, w.by));
+  w.gy = (w.inx && L.iny) ? qd<D>(fT - fTlo, L.dy, L.rdy) : 0.0;
+  w.s1 = qd<D>(fT - 2.0 * w.T + fTlo, L.hsq, L.rhsq);      // secondDerivative1D (derivs.cpp:450)
+  w.dbxy = yderiv<D>(L, yface<D>(L, w.bx));
+  w.dbyy = yderiv<D>(L, yface<D>(L, w.by));
   if (SAT) {
     w.coef = r.coef;
-    w.dcy = yderiv<EX>(L, yface<EX>(L, w.coef));
+    w.dcy = yderiv<D>(L, yface<D>(L, w.coef));
   }
   return w;
 }
 
-// boundaryInterpolate across the x-face between rows A (lower) and B (upper)
-template <bool SAT, bool EX = true>
-__device__ __forceinline__ XFaces xfaces(const Mesh& M, const Row& A, const Row& B) {
-  const double ha = M.x.h[A.i], hb = M.x.h[B.i], fd = M.x.fden[B.i], rfd = M.x.rfden[B.i];
+// whether a row's values at this lane are outside the range of the untested divisions and powers
+template <bool SAT>
+__device__ __forceinline__ bool row_out(const Row& w, const Raw& r) {
+  RangeTest t;
+  t.add(w.bx);
+  t.add(w.by);
+  if (SAT) t.add(w.coef);
+  return t.out() || !(w.T >= 0x1p-100 && w.T <= 0x1p+100) || !(r.n >= 0x1p-100 && r.n <= 0x1p+150);
+}
+
+// boundaryInterpolate across the x-face between rows A (lower) and B (upper), whose geometry is g
+template <bool SAT, int D>
+__device__ __forceinline__ XFaces xfaces(const FaceGeom& g, const Row& A, const Row& B) {
   XFaces f;
-  f.T = qd<EX>(A.T * hb + B.T * ha, fd, rfd);
-  f.gy = qd<EX>(A.gy * hb + B.gy * ha, fd, rfd);
-  f.bx = qd<EX>(A.bx * hb + B.bx * ha, fd, rfd);
-  f.by = qd<EX>(A.by * hb + B.by * ha, fd, rfd);
-  if (SAT) f.coef = qd<EX>(A.coef * hb + B.coef * ha, fd, rfd);
+  f.T = qd<D>(A.T * g.hup + B.T * g.hlo, g.den, g.rden);
+  f.gy = qd<D>(A.gy * g.hup + B.gy * g.hlo, g.den, g.rden);
+  f.bx = qd<D>(A.bx * g.hup + B.bx * g.hlo, g.den, g.rden);
+  f.by = qd<D>(A.by * g.hup + B.by * g.hlo, g.den, g.rden);
+  if (SAT) f.coef = qd<D>(A.coef * g.hup + B.coef * g.hlo, g.den, g.rden);
   return f;
 }
 

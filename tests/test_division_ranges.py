@@ -9,8 +9,6 @@ nothing may reach 2**900.
 import os
 import re
 
-import pytest
-
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CONST = dict((k, int(v)) for k, v in re.findall(r"constexpr int (RANGE_\w+) = (\d+);",
                                                 open(os.path.join(ROOT, "spruce_amd/csrc/range.hpp")).read()))
@@ -62,8 +60,7 @@ def diff(x):
     return qdiv_in(x + x, H)
 
 
-@pytest.mark.parametrize("species", ["mhd"])
-def test_stage_chains(species):
+def test_stage_chains():
     q = magnitude(-L, U)                                  # transported value
     rho = magnitude(-R, RU)
     v = qdiv_in(q, rho)                                   # v = mom / rho
@@ -78,6 +75,20 @@ def test_stage_chains(species):
     qdiv_in(db + db, FOUR_PI)                             # curl / 4 pi
     qdiv_in(q, FOUR_PI)
     qdiv_in(db * q + db * q, FOUR_PI)                     # (curl_z x b) / 4 pi
+
+
+def test_conduction_chains():
+    """The conduction update: T and n tested to 2**-100 .. 2**100 and 2**-100 .. 2**150, b_hat and the
+    saturation coefficient as transported values."""
+    T, b = magnitude(-100, 100), magnitude(-L, U)
+    den = magnitude(-100, 150) * magnitude(-52, -51)      # n * 2 K_B
+    qdiv_in(T * den, den)                                 # te (gamma - 1) = T den
+    hsq = magnitude(-2 * G, 2 * G)
+    f = interp(T)
+    qdiv_in(f + T + f, hsq)                               # second derivative
+    g = diff(f)
+    diff(interp(g))                                       # derivative of the other axis's gradient
+    diff(interp(b))
 
 
 def test_ranges_cover_ordinary_states():

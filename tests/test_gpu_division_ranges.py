@@ -82,3 +82,27 @@ def test_tile_edges(nx, ny, rows, bc):
 def test_mesh_out_of_range():
     st, cfg = wave(14, 70, "rk2", PERIODIC, d=1e-15)
     check(st, cfg, {"stage_kernel": "strip", "strip_rows": 4})
+
+
+@pytest.mark.parametrize("sat,integ", [(False, "euler"), (True, "rk2"), (False, "rk4")])
+@pytest.mark.parametrize("what", ["bhat", "mesh"])
+def test_conduction_out_of_range(sat, integ, what):
+    """A field direction with a component below 2^-170 in some columns, and a mesh above 2^46."""
+    from oracle.oracle import set_pow_mode
+    st = W.arcade_state(22, 130, stretch=1.01)
+    if what == "bhat":
+        st.grids["be_x"][:, 40:90] = 1e-55
+    else:
+        for k in ("d_x", "d_y", "pos_x", "pos_y"):
+            st.grids[k] = st.grids[k] * 1e10
+        st.grids["grav_y"][:] = 0.0
+    cfg = W.base_config("ideal_mhd", ("periodic", "periodic", "fixed", "open"), "rk2", epsilon=0.2, density_min=1.0, temp_min=1e4,
+                        thermal_energy_min=1e-8,
+                        modules=[("thermal_conduction", [("flux_saturation", str(sat).lower()), ("epsilon", "0.5"),
+                                                         ("dt_subcycle_min", "1e-9"),
+                                                         ("time_integrator", integ)])])
+    set_pow_mode(1)
+    try:
+        check(st, cfg, {"tc_kernel": "strip", "tc_rows": 4}, steps=2)
+    finally:
+        set_pow_mode(0)
