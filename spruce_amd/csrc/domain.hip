@@ -116,6 +116,8 @@ struct GpuModule {
   virtual void add_rhs(Domain&, const MhdSet&, double*) {}
   // postIterateModule: after the integrator's final propagate, before the next step size
   virtual void post(Domain&) {}
+  // whether post() may change the live grids
+  virtual bool acts_after_integrator() const { return true; }
   // the values commandLineMessage prints that live on the device (empty for most modules)
   virtual std::vector<double> report(Domain&) { return {}; }
   // Module::fileOutput (modulehandler.cpp:123-130): the grids this module appends to every stored
@@ -195,10 +197,11 @@ class Domain : public DomainBase {
   bool any_open = false;
   uint64_t row_mask[N_STATIC];   // per static field, 0 where every row equals row 0
   bool in_range = false;  // the mesh and the external field allow untested divisions (range.hpp)
-  int stage_kernel = -1;  // 0: wavefront strips (mhd2.hip), 1: one thread per cell, 2: tiles (mhd.hip), -1: by size
-  // the final stage of a step also forms the next step size's per-block minima (tile form, no ghost
-  // fill, limiter or module after the integrator)
+  int stage_kernel = 0;   // 0: wavefront strips (mhd2.hip), 1: one thread per cell (mhd.hip)
+  // the final stage of a step also forms the next step size's per-block minima (strip form, no
+  // limiter or module after the integrator)
   bool fuse_dt = false;
+  int dt_still = 0;       // sides whose ghost fill zeroes the momenta of the interior row next to them
   int strip_rows = 0;     // rows per wavefront strip; 0 = chosen from the grid size
   int tc_kernel = -1;     // conduction update: 0 wavefront strips, 1 one thread per cell, -1 by size
   int tc_rows = 0;        // rows per conduction strip; 0 = chosen from the grid size
@@ -214,7 +217,7 @@ class Domain : public DomainBase {
     if (k == "stage_kernel") {
       require(v == "strip" || v == "cell" || v == "tile" || v == "auto", SPRUCE_E_ARG,
               "stage_kernel must be strip, cell, tile or auto");
-      stage_kernel = v == "cell" ? 1 : (v == "strip" ? 0 : (v == "tile" ? 2 : -1));
+      stage_kernel = v == "cell" ? 1 : 0;   // "tile" named a form that the strips have replaced
     } else if (k == "strip_rows") {
       const int r = std::stoi(v);
       require(r >= 4 && r <= 256 && r % 4 == 0, SPRUCE_E_ARG, "strip_rows must be a multiple of 4 in [4, 256]");
@@ -468,11 +471,12 @@ class Domain : public DomainBase {
     if (strip_rows == 0) strip_rows = mhd_strip_rows_default(nx, ny);
     if (tc_rows == 0) tc_rows = tc_strip_rows_default(nx, ny);
     if (tc_kernel < 0) tc_kernel = 0;   // the strips are the faster form at every size
-    if (stage_kernel < 0) stage_kernel = 0;   // the strips are the fastest form at every size
-    fuse_dt = stage_kernel == 2 && !(kinds_all[0] || kinds_all[1] || kinds_all[2] || kinds_all[3]) && !any_moc &&
-              mods.empty();
+    fuse_dt = !any_moc;
+    for (auto& m : mods) fuse_dt = fuse_dt && !m->acts_after_integrator();
+    for (int k = 0; k < 4; ++k)
+      if (bc[k] == SPRUCE_BC_FIXED || bc[k] == SPRUCE_BC_REFLECT) dt_still |= 1 << k;
     dt_blocks = mhd_dt_blocks(mesh);
-    partial.alloc(std::max(dt_blocks, mhd_tile_blocks(mesh)));
+    partial.alloc(std::max(dt_blocks, mhd_strip_blocks(mesh, std::min(4, strip_rows))));
     step.alloc(1);
     history.alloc(1);
     hip_check(hipMalloc(&err_flag, sizeof(int)), "hipMalloc");
@@ -604,6 +608,7 @@ class Domain : public DomainBase {
              double* dt_partial = nullptr) {
     StageArgs a = stage_args(S.view(), B.view(), T.view(), mult, mode, kslot, step_ptr, nullptr);
     a.dt_partial = dt_partial;
+    a.dt_still = dt_still;
     launch_stage_mods(a);
   }
   // a stage with the modules' right-hand-side terms at its state a.S
@@ -634,7 +639,6 @@ class Domain : public DomainBase {
   }
   void launch_stage(const StageArgs& a) {
     if (stage_kernel == 1) timed("mhd_stage", [&] { launch_mhd_stage(a, stream); });
-    else if (stage_kernel == 2) timed("mhd_stage", [&] { launch_mhd_stage_tile(a, stream); });
     else timed("mhd_stage", [&] { launch_mhd_stage_strip(a, strip_rows, stream); });
   }
 
@@ -648,7 +652,7 @@ class Domain : public DomainBase {
   // (evolution.cpp:62) written on the device.
   void finish_step(int idx, bool fused = false) {
     if (!fused) timed("mhd_dt", [&] { launch_mhd_dt(L.view(), stat(), kc, mesh, nullptr, partial.p, stream); });
-    const int nb = fused ? mhd_tile_blocks(mesh) : dt_blocks;
+    const int nb = fused ? mhd_strip_blocks(mesh, strip_rows) : dt_blocks;
     timed("reduce_step", [&] {
       launch_reduce_step(partial.p, nb, kc.eps, step.p, idx >= 0 ? history.p : nullptr, idx, err_flag, stream);
     });
@@ -667,7 +671,7 @@ class Domain : public DomainBase {
   void advance(int s) {
     if (!mods.empty()) run_modules(s);
     const int integ = desc.time_integrator;
-    const bool fused = fuse_dt && !rec;
+    const bool fused = fuse_dt && stage_kernel == 0 && !rec;
     double* dtp = fused ? partial.p : nullptr;
     if (integ == SPRUCE_EULER) {                       // evolution.cpp:84-88
       if (rec) launch_stage_mods(stage_args(L.view(), L.view(), W.view(), 1.0, STAGE_STORE_K, 0, nullptr, rec->k1));
@@ -944,6 +948,7 @@ class Domain : public DomainBase {
 // ThermalConduction (source/modules/solar/thermalconduction.cpp)
 // ---------------------------------------------------------------------------------------------
 struct TcModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   TcParams p{};
   double eps = 0.0;
   std::string integ = "euler";
@@ -1131,6 +1136,7 @@ void TcModule::record(Domain& d, int s, int k, const double* src) {
 // RadiativeLosses (source/modules/solar/radiativelosses.cpp)
 // ---------------------------------------------------------------------------------------------
 struct RlModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   RlParams p{};
   std::string integ = "euler";
   bool inactive = false;
@@ -1221,6 +1227,7 @@ static std::vector<std::string> split_list(const std::string& v) {  // splitStri
 }
 
 struct ViscModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   struct Term {
     std::string opt, diff, evol, species;
     double strength = 0.0, length = 0.0;
@@ -1607,6 +1614,7 @@ struct HeatModule : GpuModule {
 // PhysicalViscosity (source/modules/solar/physicalviscosity.cpp)
 // ---------------------------------------------------------------------------------------------
 struct PvModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   double coeff = 0.0, ramp = 0.0, epsilon = 1.0;
   double msf = 0.0;   // ms_electron_heating_fraction (physicalviscosity.hpp:33)
   bool heating_on = true, force_on = true, inactive = false, grad_corr = false, to_file = false;
@@ -2059,6 +2067,7 @@ struct HeatSinkModule : PostSourceModule {
 
 // FieldHeating (fieldheating.cpp)
 struct FieldHeatModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   FheatParams p{};
   bool inactive = false, to_file = false;
   DBuf heat;   // after a step: mask * (dt * heating), the energy the step added
@@ -2212,6 +2221,7 @@ struct ParamHeatModule : PostSourceModule {
 
 // AnomalousResistivity (anomalousresistivity.cpp)
 struct ResistModule : GpuModule {
+  bool acts_after_integrator() const override { return false; }
   std::string integ = "euler", tmode = "flood_fill", model = "time_scale";
   double safety = 1.0, frob_coeff = 1.0e50, ff_threshold = 1.0, ff_ramp = 1.0e-5, ff_argmin_radius = 5.0e9;
   double sigma = 3.0, ts = -1.0, ff_max_radius = -1.0, ff_min_current = -1.0;

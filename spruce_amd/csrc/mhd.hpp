@@ -101,9 +101,12 @@ struct StageArgs {
   // open_moc characteristic terms (8 * nx*ny, evolved order), added to the ghost cells' RHS; null
   // without open_moc sides
   const double* moc;
-  // tile form only, null otherwise: one minimum per block of the target's per-cell dt over the dt
-  // bounds (the final stage of a step that no ghost fill, limiter or module follows)
+  // strip form only, null otherwise: one minimum per block of the target's per-cell dt over the
+  // interior (the final stage of a step that no limiter or module follows); dt_still: a bit per side
+  // (x lower, x upper, y lower, y upper) whose ghost fill zeroes the momenta of the interior row next
+  // to it
   double* dt_partial;
+  int dt_still;
 };
 constexpr int MAX_RHS_TERMS = 4;
 
@@ -111,11 +114,8 @@ void launch_mhd_stage(const StageArgs& a, hipStream_t s);
 // Wavefront-strip form of the same stage (mhd2.hip); R >= 1 rows per strip.
 void launch_mhd_stage_strip(const StageArgs& a, int R, hipStream_t s);
 int mhd_strip_rows_default(int nx, int ny);
-// Tile form (mhd.hip): a block of 192 threads owns an 8x8 tile; each face of the tile is computed
-// once, by one thread, into LDS, then one thread per cell combines its four faces.  For grids too
-// small to fill the GPU with strips.  mhd_tile_blocks() blocks (and dt_partial entries).
-void launch_mhd_stage_tile(const StageArgs& a, hipStream_t s);
-int mhd_tile_blocks(const Mesh& m);
+// blocks (and dt_partial entries) of a launch
+int mhd_strip_blocks(const Mesh& m, int R);
 void launch_mhd_populate(MhdSet L, const double* temp, MhdConst k, int nx, int ny, hipStream_t s);
 // Ghost fill of the sides whose kinds[] entry is non-zero; s1/s2 are the open-boundary decay
 // factors of each side (evolution.cpp:166-167), computed on the host with the C library's pow.

@@ -56,6 +56,7 @@ enum { F_EXT0 = 0, F_EXT1, F_IN0, F_IN1, F_INZ0, F_INZ1, F_EXTZ0, F_EXTZ1, F_ZEX
 struct Shared {
   double2 geom[6][64];
   double force[2][NF][64];
+  double b2[2][64];          // |b|^2 after the update, for the step size
   int out_of_range[2][2];
 };
 __device__ __forceinline__ void put_ygeom(Shared& s, const Axis& ax, int j, int l) {
@@ -151,12 +152,76 @@ __device__ __forceinline__ void velocities(double rho, const double* m, double* 
   for (int k = 0; k < N; ++k) v[k] = IN ? qdiv_in(m[k], rho, rr) : qdiv_d(m[k], rho, rr);
 }
 
+// The inverse of IdealMHD::recomputeDT at one cell (idealmhd.cpp:279-304).  IN: rho, te, mom and b2 are
+// in range and te is positive.  There |v| stands for sqrt(v*v), which equals it, and the slow speed,
+// never above the fast one (or NaN with it), is left out of the maximum.
+template <bool IN>
+__device__ __forceinline__ double dt_inverse(double rho, double te, double mx, double my, double b2, const MhdConst& K,
+                                             double dx, double rdx, double dy, double rdy) {
+  const double press = te * K.gm1;
+  if constexpr (IN) {
+    const double rr = recip_in(rho);
+    const double vx = qdiv_in(mx, rho, rr), vy = qdiv_in(my, rho, rr);
+    const double bmag = b2 == 0.0 ? 0.0 : sqrt_in(b2);
+    const double cs = sqrt_in(qdiv_in(press * K.gamma, rho, rr));
+    const double cs2 = cs * cs;
+    const double den = sqrt_in(rho * (4.0 * PI));
+    const double va = qdiv_in(bmag, den, recip_in(den));
+    const double va2 = va * va;
+    const double sum = cs2 + va2, sum2 = sum * sum;
+    const double delta = sqrt(1.0 - qdiv_in(cs2 * 4.0 * va2, sum2, recip_in(sum2)));
+    const double vfast = sqrt_in(sum * 0.5 * (1.0 + delta));
+    const double cmax = smax(smax(cs, va), vfast);
+    return qdiv_in(__builtin_fabs(vx) + cmax, dx, rdx) + qdiv_in(__builtin_fabs(vy) + cmax, dy, rdy);
+  } else {
+    const double bmag = sqrt(b2);
+    const double vx = mx / rho, vy = my / rho;
+    const double cs = sqrt(press * K.gamma / rho);
+    const double cs2 = cs * cs;
+    const double va = bmag / sqrt(rho * (4.0 * PI));
+    const double va2 = va * va;
+    const double sum = cs2 + va2;
+    const double delta = sqrt(1.0 - cs2 * 4.0 * va2 / (sum * sum));
+    const double vfast = sqrt(sum * 0.5 * (1.0 + delta));
+    const double vslow = sqrt(sum * 0.5 * (1.0 - delta));
+    const double vmx = sqrt(vx * vx), vmy = sqrt(vy * vy);
+    const double cmax = smax(smax(smax(cs, va), vfast), vslow);
+    return qdiv(vmx + cmax, dx, rdx) + qdiv(vmy + cmax, dy, rdy);
+  }
+}
+// What the fluid's wavefront keeps of an updated row until the field's |b|^2 of it is there, and the
+// largest inverse step size so far (1/x falls as x grows, so the smallest step size is 1 over the
+// largest inverse; a NaN never replaces it, as std::min drops it).
+struct DtState {
+  double rho, te, mx, my, dx, rdx;
+  bool cell = false;           // this lane's cell takes part
+  bool pending = false;
+  double worst = 0.0;
+  __device__ __forceinline__ void finish(double b2, const MhdConst& K, double dy, double rdy) {
+    RangeTest t;
+    t.density(rho);
+    t.add(te);
+    t.add(mx);
+    t.add(my);
+    t.add(b2);
+    const bool out = t.out() || !(te > 0.0);
+    double s;
+    if (__any(cell && out)) s = dt_inverse<false>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
+    else s = dt_inverse<true>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
+    worst = (cell && s > worst) ? s : worst;
+    pending = false;
+  }
+};
+
 // Rows rs .. rend-1 of a strip for one of the block's two wavefronts.  IN: the untested divisions;
 // every row is tested as it is loaded, and both wavefronts stop before the first row whose stencil
 // holds a value out of range.  Returns the row they stopped at (rend when done).  SAME: the update's
-// base is the set the derivatives are evaluated on.
-template <int ROLE, int MODE, bool IN, bool SAME>
-__device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shared& sh, double stepv, int rs, int rend) {
+// base is the set the derivatives are evaluated on.  DT: the final stage of a step that nothing but a
+// ghost fill follows: the fluid's wavefront also forms the step size of each updated row, one row
+// later, when the field's wavefront has put its |b|^2 into LDS.
+template <int ROLE, int MODE, bool IN, bool SAME, bool DT>
+__device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shared& sh, double stepv, int rs, int rend,
+                                     DtState& dt) {
   constexpr int NQ = ROLE == FLUID ? 5 : 6;     // transported quantities
   constexpr int NV = ROLE == FLUID ? 2 : 3;     // velocity components held per row
   constexpr int NO = ROLE == FLUID ? 5 : 3;     // evolved variables
@@ -335,8 +400,11 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
       f[F_ZIN][lane] = qdiv_t<IN>(cz0 * biy - cz1 * bix, 4.0 * PI, K.r4pi);
     }
     block_barrier();
+    if (DT && ROLE == FLUID && dt.pending) dt.finish(sh.b2[slot ^ 1][lane], K, gy.d, gy.rd);
     if (IN && tested_out(slot)) return false;
-    if (!col.out) return true;
+    if (!DT && !col.out) return true;
+    double o_rho = 1.0, o_te = 1.0, o_mx = 0.0, o_my = 0.0, o_b2 = 0.0;   // what the step size reads
+    if (!DT || col.out) {
     double k8[NO];
     if (r >= M.x.lo && r <= M.x.hi && col.interior) {
       if constexpr (ROLE == FLUID) {
@@ -393,17 +461,41 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
       const double rho1 = smax(qdiv(rho_new, K.m, K.rm), K.nmin) * K.m;
       const double te1 = smax(b[4] + k8[4] * stepv, K.temin);
       const double n = smax(qdiv(rho1, K.m, K.rm), K.nmin);
-      st_row(a.T.rho, row, jb, n * K.m);
+      o_rho = n * K.m;
+      o_mx = b[1] + k8[1] * stepv;
+      o_my = b[2] + k8[2] * stepv;
+      o_te = smax(te1, K.temin);
+      st_row(a.T.rho, row, jb, o_rho);
       if (a.write_n) st_row(a.T.n, row, jb, n);
       if (a.write_pre) st_row(a.T.rho_pre, row, jb, rho1);
-      st_row(a.T.mx, row, jb, b[1] + k8[1] * stepv);
-      st_row(a.T.my, row, jb, b[2] + k8[2] * stepv);
+      st_row(a.T.mx, row, jb, o_mx);
+      st_row(a.T.my, row, jb, o_my);
       st_row(a.T.mz, row, jb, b[3] + k8[3] * stepv);
-      st_row(a.T.te, row, jb, smax(te1, K.temin));
+      st_row(a.T.te, row, jb, o_te);
     } else {
-      st_row(a.T.bx, row, jb, b[0] + k8[0] * stepv);
-      st_row(a.T.by, row, jb, b[1] + k8[1] * stepv);
-      st_row(a.T.bz, row, jb, b[2] + k8[2] * stepv);
+      const double nbx = b[0] + k8[0] * stepv, nby = b[1] + k8[1] * stepv, nbz = b[2] + k8[2] * stepv;
+      st_row(a.T.bx, row, jb, nbx);
+      st_row(a.T.by, row, jb, nby);
+      st_row(a.T.bz, row, jb, nbz);
+      if (DT) {
+        const double bx = qc[Q_BEX] + nbx, by = qc[Q_BEY] + nby, bz = qc[Q_BEZ] + nbz;
+        o_b2 = bx * bx + by * by + bz * bz;
+      }
+    }
+    }
+    if (DT && ROLE == FIELD) sh.b2[slot][lane] = o_b2;
+    if (DT && ROLE == FLUID) {
+      // a fixed or reflecting side's ghost fill zeroes the momenta of the interior row next to it
+      const bool still = (r == M.x.lo && (a.dt_still & 1)) || (r == M.x.hi && (a.dt_still & 2)) ||
+                         (col.j == M.y.lo && (a.dt_still & 4)) || (col.j == M.y.hi && (a.dt_still & 8));
+      dt.rho = o_rho;
+      dt.te = o_te;
+      dt.mx = still ? 0.0 : o_mx;
+      dt.my = still ? 0.0 : o_my;
+      dt.dx = dx;
+      dt.rdx = rdx;
+      dt.cell = col.out && col.interior && r >= M.x.lo && r <= M.x.hi;
+      dt.pending = true;
     }
     return true;
   };
@@ -417,14 +509,28 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
   return rend;
 }
 
-template <int ROLE, int MODE, bool SAME>
+template <int ROLE, int MODE, bool SAME, bool DT>
 __device__ __forceinline__ void strip_rows(const StageArgs& a, const Column& col, Shared& sh, double stepv, int r,
                                            int rend) {
-  if (a.in_range) r = march<ROLE, MODE, true, SAME>(a, col, sh, stepv, r, rend);
-  if (r < rend) (void)march<ROLE, MODE, false, SAME>(a, col, sh, stepv, r, rend);
+  DtState dt;
+  if (a.in_range) r = march<ROLE, MODE, true, SAME, DT>(a, col, sh, stepv, r, rend, dt);
+  if (r < rend) (void)march<ROLE, MODE, false, SAME, DT>(a, col, sh, stepv, r, rend, dt);
+  if constexpr (DT) {
+    block_barrier();
+    if constexpr (ROLE == FLUID) {
+      const double2 d = sh.geom[5][threadIdx.x];
+      if (dt.pending) dt.finish(sh.b2[(rend - 1) & 1][threadIdx.x], a.k, d.x, d.y);
+      double m = dt.worst;
+      for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(m, off, 64);
+        m = m < o ? o : m;
+      }
+      if (threadIdx.x == 0) a.dt_partial[blockIdx.x] = m > 0.0 ? 1.0 / m : DBL_MAX;
+    }
+  }
 }
 
-template <int MODE, bool SAME>
+template <int MODE, bool SAME, bool DT>
 __global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
 k_mhd_stage_strip(StageArgs a, int R, int nstrips) {
   const Mesh& M = a.mesh;
@@ -442,8 +548,8 @@ k_mhd_stage_strip(StageArgs a, int R, int nstrips) {
   const double stepv = a.step_mult * (*a.step);
   const int r0 = strip * R, rend = min(r0 + R, M.nx);
   put_ygeom(sh, M.y, col.j, lane);   // both wavefronts write, and each reads, the same values
-  if (__builtin_amdgcn_readfirstlane(threadIdx.y) == 0) strip_rows<FLUID, MODE, SAME>(a, col, sh, stepv, r0, rend);
-  else strip_rows<FIELD, MODE, SAME>(a, col, sh, stepv, r0, rend);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.y) == 0) strip_rows<FLUID, MODE, SAME, DT>(a, col, sh, stepv, r0, rend);
+  else strip_rows<FIELD, MODE, SAME, DT>(a, col, sh, stepv, r0, rend);
 }
 
 }  // namespace
@@ -463,18 +569,27 @@ int mhd_strip_rows_default(int nx, int ny) {
   return best;
 }
 
+int mhd_strip_blocks(const Mesh& m, int R) {
+  return ((m.ny + OUT_COLS - 1) / OUT_COLS) * ((m.nx + R - 1) / R);
+}
+
 void launch_mhd_stage_strip(const StageArgs& a, int R, hipStream_t s) {
-  const int cols = (a.mesh.ny + OUT_COLS - 1) / OUT_COLS, nstrips = (a.mesh.nx + R - 1) / R;
-  const dim3 grid(cols * nstrips);
+  const int nstrips = (a.mesh.nx + R - 1) / R;
+  const dim3 grid(mhd_strip_blocks(a.mesh, R));
   const bool same = a.B.rho == a.S.rho;
-  auto go = [&](auto mode) {
-    constexpr int M = decltype(mode)::value;
-    if (same) hipLaunchKernelGGL((k_mhd_stage_strip<M, true>), grid, dim3(64, 2), 0, s, a, R, nstrips);
-    else hipLaunchKernelGGL((k_mhd_stage_strip<M, false>), grid, dim3(64, 2), 0, s, a, R, nstrips);
+  auto go = [&](auto mode, auto is_same, auto dt) {
+    hipLaunchKernelGGL((k_mhd_stage_strip<decltype(mode)::value, decltype(is_same)::value, decltype(dt)::value>), grid,
+                       dim3(64, 2), 0, s, a, R, nstrips);
   };
-  if (a.mode == STAGE_STORE_K) go(std::integral_constant<int, STAGE_STORE_K>{});
-  else if (a.mode == STAGE_RK4_FINAL) go(std::integral_constant<int, STAGE_RK4_FINAL>{});
-  else go(std::integral_constant<int, STAGE_PLAIN>{});
+  using Y = std::true_type;
+  using No = std::false_type;
+  const std::integral_constant<int, STAGE_PLAIN> plain{};
+  const std::integral_constant<int, STAGE_STORE_K> store{};
+  const std::integral_constant<int, STAGE_RK4_FINAL> final4{};
+  if (a.mode == STAGE_STORE_K) same ? go(store, Y{}, No{}) : go(store, No{}, No{});
+  else if (a.mode == STAGE_RK4_FINAL) a.dt_partial ? go(final4, No{}, Y{}) : go(final4, No{}, No{});
+  else if (a.dt_partial) same ? go(plain, Y{}, Y{}) : go(plain, No{}, Y{});
+  else same ? go(plain, Y{}, No{}) : go(plain, No{}, No{});
 }
 
 }  // namespace spruce

@@ -58,6 +58,19 @@ __device__ __forceinline__ double recip_in(double b) {
   return fma(y, fma(-b, y, 1.0), y);
 }
 
+// sqrt(x) correctly rounded for x in 2^-700 .. 2^700: Newton steps from v_rsq_f64 and two corrections
+// by the exact residual, the sequence of the compiler's own square root without its scaling and
+// its tests for 0 and infinity.
+__device__ __forceinline__ double sqrt_in(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = fma(-h, s, 0.5);
+  h = fma(h, r, h);
+  s = fma(s, r, s);
+  s = fma(fma(-s, s, x), h, s);
+  return fma(fma(-s, s, x), h, s);
+}
+
 // The hardware's minimum and maximum: std::min and std::max where neither operand is NaN, up to the
 // sign of a zero.  Written as instructions because the compiler's own form first canonicalises both
 // operands.
