@@ -287,18 +287,20 @@ __device__ __forceinline__ int tc_march(const TcStepArgs& a, const tcs::Lane& L,
     if (IN && __any(row_out<SAT>(prev, rp) || row_out<SAT>(cur, rc))) return rs;
     lo = xfaces<SAT, D>(g, prev, cur);
   }
-  Raw ahead = load_raw<SAT>(a, L, rs + 1);
-  for (int r = rs; r < rend; ++r) {
-    const Raw raw = ahead;
+  // Row r from row r+1's values (raw), with row r+2 asked for first; false when the march ends before
+  // it.  What row r leaves for the next is written to the second of each pair, so that two rows in
+  // turn swap the pairs and nothing is copied.
+  auto step = [&](int r, const Raw& raw, Raw& ahead, const Row& cur, Row& nxt, const XFaces& lo, XFaces& hi,
+                  const FaceGeom& g, FaceGeom& gn) -> bool {
     ahead = load_raw<SAT>(a, L, r + 2);
     const size_t row = (size_t)r * M.ny;
     uint32_t jb = 8u * (uint32_t)L.j;
     strip::lane_offset(jb);
     const double base = SEP ? strip::ld_row(a.te_base, row, jb) : cur.te;
-    const FaceGeom gn = strip::face_geom_row(M.x, r + 1);
-    const Row nxt = make_row<SAT, D>(a, L, r + 1, raw);
-    if (IN && __any(row_out<SAT>(nxt, raw))) return r;
-    const XFaces hi = xfaces<SAT, D>(gn, cur, nxt);
+    gn = strip::face_geom_row(M.x, r + 1);
+    nxt = make_row<SAT, D>(a, L, r + 1, raw);
+    if (IN && __any(row_out<SAT>(nxt, raw))) return false;
+    hi = xfaces<SAT, D>(gn, cur, nxt);
     // cell values at row r along x
     const double dx = g.d, rdx = g.rd;
     const bool in = cur.inx && L.iny;
@@ -331,15 +333,26 @@ __device__ __forceinline__ int tc_march(const TcStepArgs& a, const tcs::Lane& L,
       if (MODE == TC_STORE_K) strip::st_row(a.k_out, row, jb, dE);
       strip::st_row(a.te_out, row, jb, te);
     }
-    cur = nxt;
-    lo = hi;
-    g = gn;
+    return true;
+  };
+  Raw raw[2];
+  Row rows[2];
+  XFaces faces[2];
+  FaceGeom geom[2];
+  raw[0] = load_raw<SAT>(a, L, rs + 1);
+  rows[0] = cur;
+  faces[0] = lo;
+  geom[0] = g;
+  for (int r = rs; r < rend; r += 2) {
+    if (!step(r, raw[0], raw[1], rows[0], rows[1], faces[0], faces[1], geom[0], geom[1])) return r;
+    if (r + 1 >= rend) break;
+    if (!step(r + 1, raw[1], raw[0], rows[1], rows[0], faces[1], faces[0], geom[1], geom[0])) return r + 1;
   }
   return rend;
 }
 
 template <int MODE, bool SAT, bool SEP>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
 k_tc_strip(TcStepArgs a, int R, int nstrips, int total) {
   const Mesh& M = a.mesh;
   const int t = strip::xcd_tile(blockIdx.x, total);
@@ -478,13 +491,13 @@ void launch_tc_sat(const double* te_src, const double* n, const double* rho, con
 }
 
 int tc_strip_rows_default(int nx, int ny) {
-  // 4096 wavefronts (4 per SIMD) run at once and a strip costs its rows plus about five (three rows to
+  // 3072 wavefronts (3 per SIMD) run at once and a strip costs its rows plus about five (three rows to
   // start with, the launch): the height with the least rounds x cost, the taller one of equals
   const long tiles = (ny + 61) / 62;
   int best = 1;
   long least = 0;
   for (int R = 1; R <= 96; ++R) {
-    const long cost = (tiles * ((nx + R - 1) / R) + 4095) / 4096 * (R + 5);
+    const long cost = (tiles * ((nx + R - 1) / R) + 3071) / 3072 * (R + 5);
     if (R == 1 || cost <= least) { best = R; least = cost; }
   }
   return best;
