@@ -51,16 +51,14 @@ struct DBuf {
 };
 
 struct AxisBufs {
-  DBuf d, rd, h, hsq, rhsq, fden, rfden, gup, gdn;
+  static constexpr size_t FACE_WORDS = sizeof(FaceGeom) / sizeof(double);
+  DBuf all;                // the face table, then the nine arrays of an Axis, n values each
   std::vector<double> hd;  // host copy of the cell sizes
-  FaceGeom* face = nullptr;   // device
-  AxisBufs() = default;
-  AxisBufs(const AxisBufs&) = delete;
-  AxisBufs& operator=(const AxisBufs&) = delete;
-  ~AxisBufs() { if (face) (void)hipFree(face); }
   bool in_range = false;   // every length on the axis is in the range of the untested divisions
   Axis view(int n, int lo, int hi, int per) const {
-    return Axis{d.p, rd.p, h.p, hsq.p, rhsq.p, fden.p, rfden.p, gup.p, gdn.p, n, lo, hi, per, lo, hi, face};
+    const double* q = all.p + FACE_WORDS * n;
+    return Axis{q, q + n, q + 2 * n, q + 3 * n, q + 4 * n, q + 5 * n, q + 6 * n, q + 7 * n, q + 8 * n, n, lo, hi, per,
+                lo, hi, reinterpret_cast<const FaceGeom*>(all.p)};
   }
   // Precomputes the geometry the stencils divide by; every reciprocal is a correctly rounded
   // IEEE division on the host.
@@ -84,22 +82,18 @@ struct AxisBufs {
       if (cm2 >= 0 && cm2 < n && cm1 >= 0) vgu[c] = vh[cm2] + 2.0 * vh[cm1];
       if (cp1 >= 0 && cp1 < n) vgd[c] = vh[cp1] + 2.0 * vh[c];
     }
-    auto up = [&](DBuf& b, const std::vector<double>& v) {
-      b.alloc(n);
-      hip_check(hipMemcpy(b.p, v.data(), n * sizeof(double), hipMemcpyHostToDevice), "upload geometry");
-    };
-    up(d, vd); up(rd, vrd); up(h, vh); up(hsq, vhsq); up(rhsq, vrhsq); up(fden, vf); up(rfden, vrf);
-    up(gup, vgu); up(gdn, vgd);
     std::vector<FaceGeom> vface(n);
     for (int c = 0; c < n; ++c) {
       const int cm1 = per ? w(c - 1) : std::max(c - 1, 0), cp1 = per ? w(c + 1) : std::min(c + 1, n - 1);
       vface[c] = FaceGeom{vh[cm1], vh[c], vf[c], vrf[c], vgu[c], vf[cm1], vrf[cm1], vgd[c], vf[cp1], vrf[cp1], vd[c], vrd[c],
                           vhsq[c], vrhsq[c]};
     }
-    if (face) (void)hipFree(face);
-    face = nullptr;
-    hip_check(hipMalloc(&face, n * sizeof(FaceGeom)), "hipMalloc");
-    hip_check(hipMemcpy(face, vface.data(), n * sizeof(FaceGeom), hipMemcpyHostToDevice), "upload geometry");
+    std::vector<double> host(reinterpret_cast<const double*>(vface.data()),
+                             reinterpret_cast<const double*>(vface.data()) + FACE_WORDS * n);
+    for (const std::vector<double>* v : {&vd, &vrd, &vh, &vhsq, &vrhsq, &vf, &vrf, &vgu, &vgd})
+      host.insert(host.end(), v->begin(), v->end());
+    all.alloc(host.size());
+    hip_check(hipMemcpy(all.p, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice), "upload geometry");
   }
 };
 

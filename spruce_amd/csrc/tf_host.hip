@@ -68,6 +68,7 @@ void TfDomain::set_grid(const std::string& name, const double* p, int64_t count)
 
 TfShape parse_tf_shape(const std::string& v) {
   TfShape sh;
+  sh.automatic = false;
   if (v.rfind("strip", 0) == 0) {
     const int r = std::stoi(v.substr(5));
     require(r >= 4 && r <= 64 && r % 4 == 0, SPRUCE_E_ARG, "strip rows must be a multiple of 4 in [4, 64]");
@@ -149,6 +150,14 @@ void TfDomain::setup() {
   c.obs = desc.open_boundary_strength;
   c.rC = 1.0 / C_LIGHT; c.r6 = 1.0 / 6.0; c.r3 = 1.0 / 3.0;
   c.curl = remove_curl ? 0 : 1;
+  auto moderate = [](double m) { return m >= 0x1p-150 && m <= 0x1p+40; };
+  D.in_range = ax.in_range && ay.in_range && moderate(c.mi) && c.gm1 >= 0x1p-60 && c.gm1 <= 0x1p+10 ? 1 : 0;
+  for (int k = 0; k < 2; ++k) {
+    const std::vector<double>& g = host_grids[k == 0 ? "grav_x" : "grav_y"];
+    bool same = true;
+    for (int i = 1; same && i < nx; ++i) same = std::memcmp(&g[(size_t)i * ny], &g[0], ny * sizeof(double)) == 0;
+    D.row_mask[k] = same ? 0 : ~(uint64_t)0;
+  }
   c.em_dt = (!use_sub_cycling && !remove_curl) ? 1 : 0;          // ideal2F.cpp:195
   for (int k = 0; k < 4; ++k) {
     const std::vector<double>& d = k < 2 ? dx : dy;
@@ -201,7 +210,7 @@ void TfDomain::setup() {
   hip_check(hipMemcpy(dp, hp, 2 * sizeof(double*), hipMemcpyHostToDevice), "upload");
   launch_tf_populate(self->b, (const double* const*)dp, (const double* const*)(dp + 1), stream);
   launch_tf_ghost(self->b, TF_SEL_L, 0x3F, self->maxn, stream);
-  launch_tf_dt(self->b, stream);  // counter is 0: the first step size lands in history[0]
+  launch_tf_dt(self->b, false, stream);  // counter is 0: the first step size lands in history[0]
   hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
   (void)hipFree(dp);
   double h0 = 0.0;
@@ -298,6 +307,14 @@ void TfBatchRun::destroy_graph() {
 
 void TfBatchRun::rebuild(TfShape sh) {
   destroy_graph();
+  if (sh.automatic) {
+    std::vector<int> rows, tiles;
+    for (auto* d : members) {
+      rows.push_back(d->nx);
+      tiles.push_back((d->ny + 59) / 60);
+    }
+    sh.R = tf_strip_rows_default(rows.data(), tiles.data(), (int)rows.size());
+  }
   shape = sh;
   const int bx = sh.bx, by = sh.by;
   std::vector<TfDom> doms;
@@ -310,16 +327,18 @@ void TfBatchRun::rebuild(TfShape sh) {
     D.tiles_y = (d->nx + by - 1) / by;
     D.tile_base = base;
     const int nt = D.tiles_x * D.tiles_y;
-    if ((int)d->partial.n < nt) { d->partial.alloc(nt); d->dom.partial = d->partial.p; }
+    const int strips_x = sh.R > 0 ? (d->nx + sh.R - 1) / sh.R : 0;
+    const int ns = strips_x * ((d->ny + 59) / 60);   // 60 output columns per strip
+    if ((int)d->partial.n < std::max(nt, ns)) { d->partial.alloc(std::max(nt, ns)); d->dom.partial = d->partial.p; }
     D.partial = d->partial.p;
+    D.npartial = ns;
     D.history = d->history.p;
     D.hist_cap = (int)d->history.n;
     d->dom.tiles_x = D.tiles_x; d->dom.tiles_y = D.tiles_y;
     for (int t = 0; t < nt; ++t) tile_dom.push_back((int)k);
     base += nt;
     D.strip_base = sbase;
-    D.strips_x = sh.R > 0 ? (d->nx + sh.R - 1) / sh.R : 0;
-    const int ns = sh.R > 0 ? D.strips_x * ((d->ny + 59) / 60) : 0;   // 60 output columns per strip
+    D.strips_x = strips_x;
     for (int t = 0; t < ns; ++t) strip_dom.push_back((int)k);
     sbase += ns;
     doms.push_back(D);
@@ -347,25 +366,33 @@ void TfBatchRun::rebuild(TfShape sh) {
   b.strip_dom = d_strip_dom;
   b.nstrip_tiles = sbase;
   b.strip_rows = sh.R;
+  b.any_curl = 0;
+  b.stopping_sides = 0;
+  for (auto* d : members) {
+    if (d->dom.c.curl) b.any_curl = 1;
+    for (int k = 0; k < 4; ++k)
+      if (d->desc.bc[k] == SPRUCE_BC_FIXED || d->desc.bc[k] == SPRUCE_BC_REFLECT) b.stopping_sides = 1;
+  }
 }
 
 // One PlasmaDomain::advanceTime of every domain (evolution.cpp:59-124); no host interaction, so a
 // HIP graph can capture it.
 void TfBatchRun::enqueue_step(hipStream_t s) {
   const int ucnp = 1 << SPRUCE_BC_OPEN_UCNP;
-  auto stage = [&](int S, int B, int T, double mult, int mode, int kslot) {
-    clock.timed(s, "tf_stage", [&] { launch_tf_stage(b, S, B, T, mult, mode, kslot, s); });
+  const bool strips = b.strip_rows > 0;
+  auto stage = [&](int S, int B, int T, double mult, int mode, int kslot, bool last = false) {
+    clock.timed(s, "tf_stage", [&] { launch_tf_stage(b, S, B, T, mult, mode, kslot, last && strips, s); });
   };
   auto ghost = [&](int G, int kinds) {
     clock.timed(s, "tf_ghost", [&] { launch_tf_ghost(b, G, kinds, maxn, s); });
   };
   if (integrator == SPRUCE_EULER) {
-    stage(TF_SEL_L, TF_SEL_L, TF_SEL_W, 1.0, TF_STAGE_PLAIN, 0);
+    stage(TF_SEL_L, TF_SEL_L, TF_SEL_W, 1.0, TF_STAGE_PLAIN, 0, true);
     clock.timed(s, "tf_copy", [&] { launch_tf_copy(b, TF_SEL_W, TF_SEL_L, s); });
   } else if (integrator == SPRUCE_RK2) {
     stage(TF_SEL_L, TF_SEL_L, TF_SEL_W, 0.5, TF_STAGE_PLAIN, 0);
     if (any_ucnp) ghost(TF_SEL_W, ucnp);
-    stage(TF_SEL_W, TF_SEL_L, TF_SEL_L, 1.0, TF_STAGE_PLAIN, 0);
+    stage(TF_SEL_W, TF_SEL_L, TF_SEL_L, 1.0, TF_STAGE_PLAIN, 0, true);
   } else {
     // The live-grid ghost writes of the intermediate propagates (evolution.cpp:168-281) rewrite
     // the values the previous final propagate left there (the two-fluid derived step changes no
@@ -376,10 +403,10 @@ void TfBatchRun::enqueue_step(hipStream_t s) {
     if (any_ucnp) ghost(TF_SEL_W2, ucnp);
     stage(TF_SEL_W2, TF_SEL_L, TF_SEL_W, 1.0, TF_STAGE_STORE_K, 2);
     if (any_ucnp) ghost(TF_SEL_W, ucnp);
-    stage(TF_SEL_W, TF_SEL_L, TF_SEL_L, 1.0, TF_STAGE_RK4_FINAL, 0);
+    stage(TF_SEL_W, TF_SEL_L, TF_SEL_L, 1.0, TF_STAGE_RK4_FINAL, 0, true);
   }
   if (any_ucnp || any_other) ghost(TF_SEL_L, 0x3F);
-  clock.timed(s, "tf_dt", [&] { launch_tf_dt(b, s); });
+  clock.timed(s, "tf_dt", [&] { launch_tf_dt(b, strips, s); });
 }
 
 void TfBatchRun::run(int nsteps, bool use_graph, std::vector<std::vector<double>>* dts) {
@@ -397,9 +424,10 @@ void TfBatchRun::run(int nsteps, bool use_graph, std::vector<std::vector<double>
               uploaded[k].partial != d->partial.p;
   }
   if (realloc) rebuild(shape);
-  if (persistent && !(shape.R > 0 && shape.bx == 64 && shape.by == 4)) {
-    TfShape sh;                                      // the persistent form runs strips, 64x4 cell tiles
-    sh.R = shape.R > 0 ? shape.R : 4;
+  if (persistent && (shape.automatic || !(shape.R > 0 && shape.bx == 64 && shape.by == 4))) {
+    TfShape sh;                                      // the persistent form runs strips (rows a multiple
+    sh.automatic = false;                            // of 4), 64x4 cell tiles
+    sh.R = shape.R > 0 && !shape.automatic ? shape.R : 4;
     rebuild(sh);
   }
   launch_tf_reset_counters(b, s);
@@ -475,12 +503,14 @@ double TfBatchRun::autotune(int trial_steps, std::string* chosen) {
   for (auto& bxy : std::vector<std::pair<int, int>>{{64, 1}, {64, 2}, {64, 4}, {128, 1}, {128, 2}, {32, 2}, {32, 4},
                                                     {32, 8}, {16, 4}, {16, 8}}) {
     TfShape t;
+    t.automatic = false;
     t.bx = bxy.first;
     t.by = bxy.second;
     shapes.push_back(t);
   }
   for (int r : {4, 8, 16}) {
     TfShape t;
+    t.automatic = false;
     t.R = r;
     shapes.push_back(t);
   }

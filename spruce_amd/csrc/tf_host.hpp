@@ -13,12 +13,17 @@ namespace spruce {
 class TfBatchRun;
 
 // Launch shape of a batch: the stage kernel in strips of R rows (R > 0) or one thread per cell in
-// bx x by blocks; the other kernels always use the bx x by cell tiles.
+// bx x by blocks; the other kernels always use the bx x by cell tiles.  automatic: strips whose rows
+// follow from the members' sizes.
 struct TfShape {
   int bx = 64, by = 4, R = 0;
-  std::string str() const { return R > 0 ? "strip" + std::to_string(R) : std::to_string(bx) + "x" + std::to_string(by); }
+  bool automatic = true;
+  // "<columns>x<rows>", or "strip<rows>x60" (rows by output columns)
+  std::string str() const {
+    return R > 0 ? "strip" + std::to_string(R) + "x60" : std::to_string(bx) + "x" + std::to_string(by);
+  }
 };
-// "<columns>x<rows>" (64, 128, 192 or 256 threads) or "strip<rows>" (rows a multiple of 4, 4..64)
+// "<columns>x<rows>" (64, 128, 192 or 256 threads) or "strip<rows>", "strip<rows>x60" (rows a multiple of 4, 4..64)
 TfShape parse_tf_shape(const std::string& v);
 
 class TfDomain : public DomainBase {

@@ -10,6 +10,7 @@
 #include <type_traits>
 
 #include "arith.hpp"
+#include "range.hpp"
 #include "strip.hpp"
 #include <hip/hip_cooperative_groups.h>
 
@@ -325,21 +326,31 @@ __device__ void tf_ghost_side(const TfDom& D, const TfSet& G, int side, int kind
     for (int v : {TF_IMX, TF_IMY, TF_EMX, TF_EMY}) { G.v[v][c1] = 0.0; G.v[v][c2] = 0.0; G.v[v][c3] = 0.0; }
   } else if (kind == 5) {                                            // open_ucnp, :290-334
     const size_t ci = at(upper ? ax.hi : ax.lo);
+    // every value is read before the first is written, so that the reads overlap
+    constexpr int vars[11] = {TF_IRHO, TF_ERHO, TF_ITE, TF_ETE, TF_EX, TF_EY, TF_EZ, TF_IMX, TF_IMY, TF_EMX, TF_EMY};
+    double q[11];
+#pragma unroll
+    for (int k = 0; k < 11; ++k) q[k] = G.v[vars[k]][ci];
+#pragma unroll
     for (int g = 0; g < N_GHOST; ++g) {
       const size_t cb = at(upper ? ax.hi + 1 + g : g);
-      for (int v : {TF_IRHO, TF_ERHO, TF_ITE, TF_ETE, TF_EX, TF_EY, TF_EZ, TF_IMX, TF_IMY, TF_EMX, TF_EMY})
-        G.v[v][cb] = G.v[v][ci];
+#pragma unroll
+      for (int k = 0; k < 11; ++k) G.v[vars[k]][cb] = q[k];
     }
   }
 }
 
-__global__ void k_tf_ghost(TfBatch b, int Gsel, int kinds_mask, int xsides) {
+// One side per block row z (first + z).  The two sides of an axis touch disjoint cells and read disjoint
+// cells once the axis has at least 6 cells; on shorter ones the first of the two does both in order.
+__global__ void k_tf_ghost(TfBatch b, int Gsel, int kinds_mask, int first) {
   const int d = blockIdx.y;
   const TfDom& D = b.doms[d];
   const TfSet& G = pick(D, Gsel);
   const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int s0 = xsides ? 0 : 2;
-  for (int s = s0; s < s0 + 2; ++s) {
+  const int side = first + blockIdx.z;
+  const bool apart = (side < 2 ? D.mesh.nx : D.mesh.ny) >= 6;
+  if (!apart && (side & 1)) return;
+  for (int s = side; s <= (apart ? side : side + 1); ++s) {
     const int kind = D.bc[s];
     if (kind != 0 && kind != 4 && ((kinds_mask >> kind) & 1)) tf_ghost_side(D, G, s, kind, t);
   }
@@ -402,10 +413,10 @@ __global__ void k_tf_dt(TfBatch b) {
   if (threadIdx.x == 0 && threadIdx.y == 0) D.partial[blockIdx.x - D.tile_base] = v;
 }
 
-__global__ void k_tf_reduce(TfBatch b) {
+__global__ void k_tf_reduce(TfBatch b, int strips) {
   const TfDom& D = b.doms[blockIdx.x];
   double v = DBL_MAX;
-  const int n = D.tiles_x * D.tiles_y;
+  const int n = strips ? D.npartial : D.tiles_x * D.tiles_y;
   for (int k = threadIdx.x; k < n; k += blockDim.x) { const double o = D.partial[k]; v = (o < v) ? o : v; }
   for (int off = 32; off > 0; off >>= 1) { const double o = __shfl_xor(v, off, 64); v = (o < v) ? o : v; }
   __shared__ double part[16];
@@ -841,6 +852,499 @@ k_tf_stage_strip(TfBatch b, int Ssel, int Bsel, int Tsel, double mult, int mode,
   tf_stage_strip_tile(b, strip::xcd_tile(blockIdx.x, b.nstrip_tiles), Ssel, Bsel, Tsel, mult, mode, kslot, qs);
 }
 
+// ---------------------------------------------------------------------------------------------
+// Species-pair form of the strip stage (the production path of launch_tf_stage): a block of two
+// wavefronts owns a strip, one transporting the ions, the other the electrons.  The ions' wavefront
+// also updates the fields (the electrons' current comes over in LDS, the only thing they share), the
+// electrons' forms the step size, which reads nothing else.
+//
+// What bounds it: FP64 issue and the latency of a row's chain, as for the IdealMHD stage (mhd2.hip),
+// whose means it shares: range tests once per loaded value (range.hpp) instead of at each division,
+// rows fetched two ahead, geometry from LDS and through the scalar cache.  Per launch of the
+// 16-domain batch (1.64 million cells) and one 192x192 domain: see launch_tf_stage.
+// ---------------------------------------------------------------------------------------------
+enum Species { IONS = 0, ELECTRONS = 1 };
+enum { S_RHO = 0, S_MX, S_MY, S_TE };
+struct PairShared {
+  double2 geom[7][64];       // lower y-face of every column, cell size, Langmuir geometry
+  double current[2][2][64];  // the electrons' part of j_x, j_y of the row being finished, two slots
+  int out_of_range[2][2];
+};
+__device__ __forceinline__ void block_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ __forceinline__ bool is_minus_zero(double v) { return __builtin_amdgcn_class(v, 0x20); }
+__device__ __forceinline__ double row_const(const double* p, int i) {   // the same index in every lane
+  return reinterpret_cast<const __attribute__((address_space(4))) double*>(reinterpret_cast<uint64_t>(p))[i];
+}
+
+// A part of a domain's description at byte address p, the same in every lane, through the scalar cache
+// (nothing writes descriptions while kernels run).
+template <class T>
+__device__ __forceinline__ T ld_const(uint64_t p) {
+  static_assert(sizeof(T) % 8 == 0, "copied in 8-byte words");
+  const __attribute__((address_space(4))) uint64_t* src = reinterpret_cast<const __attribute__((address_space(4))) uint64_t*>(p);
+  uint64_t w[sizeof(T) / 8];
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 8; ++i) w[i] = src[i];
+  T r;
+  __builtin_memcpy(&r, w, sizeof(T));
+  return r;
+}
+// One domain as a row of the stage sees it: its arrays' addresses and constants are read again in every
+// row (a few wide scalar loads), because held over the whole march they would not fit the scalar
+// registers; the empty asm makes each row's address a new one.
+struct DomView {
+  uint64_t p;
+  int S, B, T;   // TfSetSel of the three sets
+  __device__ __forceinline__ DomView row() const {
+    DomView v = *this;
+    asm volatile("" : "+s"(v.p));
+    return v;
+  }
+  __device__ __forceinline__ double* set(int sel, int v) const {
+    return reinterpret_cast<double*>(ld_const<uint64_t>(p + (uint64_t)sel * sizeof(TfSet) + 8 * v));
+  }
+  __device__ __forceinline__ double* s(int v) const { return set(S, v); }
+  __device__ __forceinline__ double* b(int v) const { return set(B, v); }
+  __device__ __forceinline__ double* t(int v) const { return set(T, v); }
+  template <class X>
+  __device__ __forceinline__ X at(size_t offset) const { return ld_const<X>(p + offset); }
+  __device__ __forceinline__ double* ptr(size_t offset) const { return reinterpret_cast<double*>(ld_const<uint64_t>(p + offset)); }
+};
+#define TF_PTR(view, field) (view).ptr(offsetof(TfDom, field))
+
+// The inverse of Ideal2F::recomputeDT's first limit at one cell (ideal2F.cpp:169-198), the
+// operations of tf_dt_cell.  IN: rho, te and mom are in range and te is positive.
+template <bool IN>
+__device__ __forceinline__ double tf_dt_inverse(const TfConst& K, double erho, double ete, double emx, double emy, double kx3,
+                                                double kxv, double ky3, double kyv, double dx, double rdx, double dy,
+                                                double rdy) {
+  auto div = [](double a, double b) { return IN ? qdiv_in(a, b, recip_in(b)) : a / b; };
+  auto root = [](double a) { return IN ? sqrt_in(a) : sqrt(a); };
+  const double en = qdiv_t<IN>(erho, K.me, K.rme);
+  const double ep = ete * K.gm1;
+  const double etemp = div(ep, K_B * en);
+  double evx, evy;
+  if (IN) {
+    const double rr = recip_in(erho);
+    evx = qdiv_in(emx, erho, rr);
+    evy = qdiv_in(emy, erho, rr);
+  } else {
+    evx = emx / erho;
+    evy = emy / erho;
+  }
+  const double vth = root(qdiv_t<IN>(K_B * etemp, K.me, K.rme));
+  const double wpe = root(qdiv_t<IN>(4 * PI * en * E_CH * E_CH, K.me, K.rme));
+  const double vth2 = vth * vth;
+  const double wthx = root(kx3 * vth2), wthy = root(ky3 * vth2);
+  const double wLx = root(wpe * wpe + wthx * wthx), wLy = root(wpe * wpe + wthy * wthy);
+  const double vLx = div(wLx, kxv), vLy = div(wLy, kyv);
+  const double vmx = fabs(evx) + vLx, vmy = fabs(evy) + vLy;
+  return qdiv_t<IN>(vmx, dx, rdx) + qdiv_t<IN>(vmy, dy, rdy);
+}
+
+struct PairRow {
+  double q[4];
+  __device__ __forceinline__ bool out_of_range() const {
+    RangeTest t;
+    t.density(q[S_RHO]);
+    t.add(q[S_MX]);
+    t.add(q[S_MY]);
+    t.add(q[S_TE]);
+    return t.out();
+  }
+};
+struct PairColumn { int j; bool interior, out; int still; };   // still: a bit per side that stops the flow
+struct Flags { int first, in_range; };                          // two ints of the description
+struct PairDt { double worst = 0.0, em = DBL_MAX; };   // largest inverse, smallest light-crossing limit
+
+template <int SP, bool CURL, bool IN>
+__device__ __forceinline__ int pair_march(const DomView& dom, const Mesh& M, const PairColumn& col, PairShared& sh, double stp, int mode, int kslot, bool want_dt, int rs, int rend,
+                                          PairDt& dt) {
+  using namespace strip;
+  constexpr int V_RHO = SP == IONS ? TF_IRHO : TF_ERHO, V_MX = SP == IONS ? TF_IMX : TF_EMX,
+                V_MY = SP == IONS ? TF_IMY : TF_EMY, V_TE = SP == IONS ? TF_ITE : TF_ETE;
+  constexpr bool FLD = SP == IONS;           // this wavefront updates the fields
+  const int nx = M.nx, ny = M.ny, lane = threadIdx.x;
+  const size_t N = (size_t)nx * ny;
+  const uint32_t jcol = 8u * (uint32_t)col.j;
+  auto row_of = [&](int r) -> int { return M.x.per ? wrap_near(r, nx) : clampn(r, nx); };
+  auto post_test = [&](bool bad, int slot) {
+    const bool any = __any(bad);
+    if (lane == 0) sh.out_of_range[slot][SP] = any ? 1 : 0;
+  };
+  auto tested_out = [&](int slot) -> bool {
+    return __builtin_amdgcn_readfirstlane(sh.out_of_range[slot][0] | sh.out_of_range[slot][1]) != 0;
+  };
+  auto load = [&](const DomView& D, int i, PairRow& r) {
+    const size_t row = (size_t)i * ny;
+    uint32_t jb = jcol;
+    lane_offset(jb);
+    r.q[S_RHO] = ld_row(D.s(V_RHO), row, jb);
+    r.q[S_MX] = ld_row(D.s(V_MX), row, jb);
+    r.q[S_MY] = ld_row(D.s(V_MY), row, jb);
+    r.q[S_TE] = ld_row(D.s(V_TE), row, jb);
+  };
+  auto load_f = [&](const DomView& D, int i, double* f) {      // field values whose faces the curl terms take
+    const size_t row = (size_t)i * ny;
+    uint32_t jb = jcol;
+    lane_offset(jb);
+    f[TFF_BZ] = ld_row(D.s(TF_BZ), row, jb);
+    f[TFF_EZ] = ld_row(D.s(TF_EZ), row, jb);
+    f[TFF_BYT] = ld_row(TF_PTR(D, bey), row, jb) + ld_row(D.s(TF_BY), row, jb);
+    f[TFF_EY] = ld_row(D.s(TF_EY), row, jb);
+    f[TFF_BXT] = ld_row(TF_PTR(D, bex), row, jb) + ld_row(D.s(TF_BX), row, jb);
+    f[TFF_EX] = ld_row(D.s(TF_EX), row, jb);
+  };
+  auto f_out = [&](const double* f) {
+    RangeTest t;
+#pragma unroll
+    for (int k = 0; k < TFF_N; ++k) t.add(f[k]);
+    return t.out();
+  };
+  auto velocity = [&](const PairRow& r, double gm1, double* v, double& p) {
+    if (IN) {
+      const double rr = recip_in(r.q[S_RHO]);
+      v[0] = qdiv_in(r.q[S_MX], r.q[S_RHO], rr);
+      v[1] = qdiv_in(r.q[S_MY], r.q[S_RHO], rr);
+    } else {
+      v[0] = r.q[S_MX] / r.q[S_RHO];
+      v[1] = r.q[S_MY] / r.q[S_RHO];
+    }
+    p = r.q[S_TE] * gm1;
+  };
+
+  PairRow w[4], next;             // rows r-1 .. r+2, and row r+3 arriving
+  double v[2][2], p[2];           // velocities and pressure of rows r and r+1
+  double Px[4];                   // flux through row r's lower x-face
+  double xvf, xip, xfl[4];        // that face's velocity, pressure and fields
+  double f[2][TFF_N];             // fields of rows r and r+1
+  double gdx, grdx;
+  {
+    const DomView D = dom.row();
+    const double gm1 = D.at<double>(offsetof(TfDom, c.gm1));
+    load(D, row_of(rs - 2), w[3]);
+    load(D, row_of(rs - 1), w[0]);
+    load(D, row_of(rs), w[1]);
+    load(D, row_of(rs + 1), w[2]);
+    load(D, row_of(rs + 2), next);
+    double ft[TFF_N];
+    if constexpr (FLD && CURL) {
+      load_f(D, row_of(rs - 1), ft);
+      load_f(D, row_of(rs), f[0]);
+    }
+    if (IN) {
+      bool bad = w[3].out_of_range() || w[0].out_of_range() || w[1].out_of_range() || w[2].out_of_range();
+      if constexpr (FLD && CURL) bad = bad || f_out(ft) || f_out(f[0]);
+      post_test(bad, (rs + 1) & 1);
+      block_barrier();
+      if (tested_out((rs + 1) & 1)) return rs;
+    }
+    double vt[2], pt;
+    velocity(w[0], gm1, vt, pt);
+    velocity(w[1], gm1, v[0], p[0]);
+    const FaceGeom gx = face_geom_row(M.x, rs);
+    gdx = gx.d;
+    grdx = gx.rd;
+    xvf = interp<IN>(gx, vt[0], v[0][0]);
+    xip = interp<IN>(gx, pt, p[0]);
+    const FaceDir fd = face_dir(xvf, gx);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double d2;
+      Px[k] = face_flux<IN>(w[3].q[k], w[0].q[k], w[1].q[k], w[2].q[k], gx, fd, d2);
+    }
+    if constexpr (FLD && CURL) {
+      constexpr int xf[4] = {TFF_BZ, TFF_BYT, TFF_EZ, TFF_EY};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) xfl[k] = interp<IN>(gx, ft[xf[k]], f[0][xf[k]]);
+    }
+  }
+
+  auto step = [&](auto BC, int r) -> bool {
+    constexpr int Bi = decltype(BC)::value;
+    constexpr int SM = Bi % 4, S0 = (Bi + 1) % 4, S1 = (Bi + 2) % 4, S2 = (Bi + 3) % 4;
+    constexpr int D0 = Bi % 2, D1 = (Bi + 1) % 2;
+    if (r >= rend) return false;
+    const int slot = r & 1;
+    const DomView D = dom.row();
+    const TfConst K = D.at<TfConst>(offsetof(TfDom, c));
+    const double mass = SP == IONS ? K.mi : K.me, rmass = SP == IONS ? K.rmi : K.rme;
+    w[S2] = next;
+    load(D, row_of(r + 3), next);
+    if constexpr (FLD && CURL) load_f(D, row_of(r + 1), f[D1]);
+    const size_t row = (size_t)r * ny;
+    uint32_t jb = jcol;
+    lane_offset(jb);
+    double b[4];
+    b[0] = ld_row(D.b(V_RHO), row, jb); b[1] = ld_row(D.b(V_MX), row, jb);
+    b[2] = ld_row(D.b(V_MY), row, jb); b[3] = ld_row(D.b(V_TE), row, jb);
+    const double grx = ld_row(TF_PTR(D, gx), row & D.at<uint64_t>(offsetof(TfDom, row_mask)), jb),
+                 gry = ld_row(TF_PTR(D, gy), row & D.at<uint64_t>(offsetof(TfDom, row_mask) + 8), jb);
+    const double bz = ld_row(D.s(TF_BZ), row, jb), Ex = ld_row(D.s(TF_EX), row, jb), Ey = ld_row(D.s(TF_EY), row, jb);
+    double bf[6];
+    if constexpr (FLD) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) bf[k] = ld_row(D.b(TF_EX + k), row, jb);
+    }
+    const bool in = r >= M.x.lo && r <= M.x.hi && col.interior;   // derivatives are zero outside (derivs.cpp:229-233)
+    const FaceGeom gx = face_geom_row(M.x, r + 1);
+    const double dx = gdx, rdx = grdx;
+    gdx = gx.d;
+    grdx = gx.rd;
+    FaceGeom gy;
+    {
+      const double2 g0 = sh.geom[0][lane], g1 = sh.geom[1][lane], g2 = sh.geom[2][lane], g3 = sh.geom[3][lane],
+                    g4 = sh.geom[4][lane], g5 = sh.geom[5][lane];
+      gy = FaceGeom{g0.x, g0.y, g1.x, g1.y, g2.x, g2.y, g3.x, g3.y, g4.x, g4.y, g5.x, g5.y, 0.0, 0.0};
+    }
+    auto ddx = [&](double up, double lo) { return qdiv_t<IN>(up - lo, dx, rdx); };
+    auto ddy = [&](double lo) { return qdiv_t<IN>(shl1(lo) - lo, gy.d, gy.rd); };
+    // ---- y-faces of row r
+    const double vfy = interp<IN>(gy, shr1(v[D0][1]), v[D0][1]);
+    const double dpy = ddy(interp<IN>(gy, shr1(p[D0]), p[D0]));
+    const double dvy = ddy(vfy);
+    const FaceDir fdy = face_dir(vfy, gy);
+    double td[4], fly[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double qc = w[S0].q[k];
+      const double qm1 = shr1(qc);
+      const double qm2 = shr1(qm1);
+      const double qp1 = shl1(qc);
+      double d2;
+      td[k] = ddy(face_flux<IN>(qm2, qm1, qc, qp1, gy, fdy, d2));
+    }
+    if constexpr (FLD && CURL) {
+      constexpr int yf[4] = {TFF_BZ, TFF_BXT, TFF_EZ, TFF_EX};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) fly[k] = ddy(interp<IN>(gy, shr1(f[D0][yf[k]]), f[D0][yf[k]]));
+    }
+    if (IN) {
+      // a base of -0 keeps its sign only if the derivative is -0 too, which the untested limiter does
+      // not settle
+      bool bad = w[S2].out_of_range() || is_minus_zero(b[1]) || is_minus_zero(b[2]) || is_minus_zero(b[3]);
+      RangeTest t;
+      t.add(bz);
+      bad = bad || t.out();
+      if constexpr (FLD && CURL) bad = bad || f_out(f[D1]);
+      post_test(bad, slot);
+    }
+    // ---- upper x-face of row r from rows r-1 .. r+2
+    velocity(w[S1], K.gm1, v[D1], p[D1]);
+    double flx[4];
+    const double nvf = interp<IN>(gx, v[D0][0], v[D1][0]), nip = interp<IN>(gx, p[D0], p[D1]);
+    const double dpx = ddx(nip, xip), dvx = ddx(nvf, xvf);
+    xip = nip;
+    xvf = nvf;
+    const FaceDir fd = face_dir(nvf, gx);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double d2;
+      const double Pn = face_flux<IN>(w[SM].q[k], w[S0].q[k], w[S1].q[k], w[S2].q[k], gx, fd, d2);
+      const double tx = ddx(Pn, Px[k]);
+      td[k] = tx + td[k];
+      Px[k] = Pn;
+    }
+    if constexpr (FLD && CURL) {
+      constexpr int xf[4] = {TFF_BZ, TFF_BYT, TFF_EZ, TFF_EY};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const double nf = interp<IN>(gx, f[D0][xf[k]], f[D1][xf[k]]);
+        flx[k] = ddx(nf, xfl[k]);
+        xfl[k] = nf;
+      }
+    }
+    // ---- the cell (tf_rhs_cell)
+    const double rho = w[S0].q[S_RHO], vx = v[D0][0], vy = v[D0][1];
+    const double num = qdiv_t<IN>(rho, mass, rmass);
+    const double curx = num * E_CH * vx, cury = num * E_CH * vy;
+    if constexpr (!FLD) {
+      sh.current[slot][0][lane] = curx;
+      sh.current[slot][1][lane] = cury;
+    }
+    block_barrier();
+    if (IN && tested_out(slot)) return false;
+    const double vb0 = vy * bz, vb1 = (-vx) * bz;
+    const double eq = SP == IONS ? E_CH * num : -E_CH * num;
+    const double Fx = eq * (Ex + qdiv_t<IN>(vb0, C_L, K.rC)), Fy = eq * (Ey + qdiv_t<IN>(vb1, C_L, K.rC));
+    const double mask = in ? 1.0 : 0.0;                            // ideal2F.cpp:94
+    double k[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) td[q] = in ? td[q] : 0.0;
+    k[S_RHO] = -td[S_RHO] * mask;
+    k[S_MX] = (-td[S_MX] - (in ? dpx : 0.0) + rho * grx + Fx) * mask;
+    k[S_MY] = (-td[S_MY] - (in ? dpy : 0.0) + rho * gry + Fy) * mask;
+    k[S_TE] = (-td[S_TE] - p[D0] * (in ? dvx + dvy : 0.0)) * mask;
+    double kf[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if constexpr (FLD) {
+      const double jx = curx - sh.current[slot][0][lane], jy = cury - sh.current[slot][1][lane];   // ideal2F.cpp:128-129
+      if constexpr (CURL) {                                        // :75-80
+        const double dbz_x = in ? flx[0] : 0.0, dby_x = in ? flx[1] : 0.0, dEz_x = in ? flx[2] : 0.0, dEy_x = in ? flx[3] : 0.0;
+        const double dbz_y = in ? fly[0] : 0.0, dbx_y = in ? fly[1] : 0.0, dEz_y = in ? fly[2] : 0.0, dEx_y = in ? fly[3] : 0.0;
+        kf[0] = C_L * dbz_y - 4. * PI * jx;
+        kf[1] = -C_L * dbz_x - 4. * PI * jy;
+        kf[2] = C_L * (dby_x - dbx_y);
+        kf[3] = -C_L * dEz_y;
+        kf[4] = C_L * dEz_x;
+        kf[5] = C_L * (dEx_y - dEy_x);
+      } else {                                                     // :83-88
+        kf[0] = -4. * PI * jx;
+        kf[1] = -4. * PI * jy;
+      }
+#pragma unroll
+      for (int q = 0; q < 6; ++q) kf[q] *= mask;
+    }
+    constexpr int vars[4] = {V_RHO, V_MX, V_MY, V_TE};
+    if (col.out) {
+      if (mode == TF_STAGE_STORE_K) {
+        double* const kst = D.ptr(offsetof(TfDom, k) + 8 * (size_t)kslot);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) st_row(kst, vars[q] * N + row, jb, k[q]);
+        if constexpr (FLD) {
+#pragma unroll
+          for (int q = 0; q < 6; ++q) st_row(kst, (TF_EX + q) * N + row, jb, kf[q]);
+        }
+      } else if (mode == TF_STAGE_RK4_FINAL) {                     // evolution.cpp:119-121
+        double *const k0 = D.ptr(offsetof(TfDom, k)), *const k1 = D.ptr(offsetof(TfDom, k) + 8),
+                     *const k2 = D.ptr(offsetof(TfDom, k) + 16);
+        auto comb = [&](int var, double k4) {
+          return qdiv(ld_row(k0, var * N + row, jb) + k4, 6.0, K.r6) +
+                 qdiv(ld_row(k1, var * N + row, jb) + ld_row(k2, var * N + row, jb), 3.0, K.r3);
+        };
+#pragma unroll
+        for (int q = 0; q < 4; ++q) k[q] = comb(vars[q], k[q]);
+        if constexpr (FLD) {
+#pragma unroll
+          for (int q = 0; q < 6; ++q) kf[q] = comb(TF_EX + q, kf[q]);
+        }
+      }
+    }
+    double nv[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) nv[q] = b[q] + k[q] * stp;
+    // enforceMinimums (ideal2F.cpp:98-105)
+    nv[S_RHO] = smax(qdiv(nv[S_RHO], mass, rmass), K.nmin) * mass;
+    nv[S_TE] = smax(nv[S_TE], K.temin);
+    if (col.out) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) st_row(D.t(vars[q]), row, jb, nv[q]);
+      if constexpr (FLD) {
+#pragma unroll
+        for (int q = 0; q < 6; ++q) st_row(D.t(TF_EX + q), row, jb, bf[q] + kf[q] * stp);
+      }
+    }
+    if (!FLD && want_dt) {
+      // a fixed or reflecting side's ghost fill zeroes the momenta of the interior row next to it
+      const bool still = (r == M.x.lo && (col.still & 1)) || (r == M.x.hi && (col.still & 2)) ||
+                         (col.j == M.y.lo && (col.still & 4)) || (col.j == M.y.hi && (col.still & 8));
+      const bool cell = col.out && in;
+      const double emx = still ? 0.0 : nv[S_MX], emy = still ? 0.0 : nv[S_MY];
+      RangeTest t;
+      t.density(nv[S_RHO]);
+      t.add(nv[S_TE]);
+      t.add(emx);
+      t.add(emy);
+      const double2 kk = sh.geom[6][lane];
+      const double kx3 = row_const(TF_PTR(D, kx3), r), kxv = row_const(TF_PTR(D, kxv), r);
+      double s;
+      if (!IN || __any(cell && (t.out() || !(nv[S_TE] > 0.0))))
+        s = tf_dt_inverse<false>(K, nv[S_RHO], nv[S_TE], emx, emy, kx3, kxv, kk.x, kk.y, dx, rdx, gy.d, gy.rd);
+      else
+        s = tf_dt_inverse<true>(K, nv[S_RHO], nv[S_TE], emx, emy, kx3, kxv, kk.x, kk.y, dx, rdx, gy.d, gy.rd);
+      dt.worst = (cell && s > dt.worst) ? s : dt.worst;
+      if (K.em_dt && cell && s == s) {
+        const double dtem = qdiv(dx * gy.d / (dx + gy.d), C_L, K.rC);
+        dt.em = dtem < dt.em ? dtem : dt.em;
+      }
+    }
+    return true;
+  };
+
+  for (int r = rs; r < rend; r += 4) {
+    if (!step(std::integral_constant<int, 0>{}, r)) return r;
+    if (!step(std::integral_constant<int, 1>{}, r + 1)) return r + 1;
+    if (!step(std::integral_constant<int, 2>{}, r + 2)) return r + 2;
+    if (!step(std::integral_constant<int, 3>{}, r + 3)) return r + 3;
+  }
+  return rend;
+}
+
+template <int SP, bool ANYCURL>
+__device__ __forceinline__ void pair_strip(const DomView& D, const Mesh& M, const PairColumn& col, PairShared& sh,
+                                           double stp, int mode, int kslot, bool want_dt, int r, int rend, int part) {
+  PairDt dt;
+  const bool in_range = D.at<Flags>(offsetof(TfDom, npartial)).in_range != 0;
+  if (ANYCURL && D.at<Flags>(offsetof(TfDom, c.curl)).first != 0) {
+    if (in_range) r = pair_march<SP, true, true>(D, M, col, sh, stp, mode, kslot, want_dt, r, rend, dt);
+    if (r < rend) (void)pair_march<SP, true, false>(D, M, col, sh, stp, mode, kslot, want_dt, r, rend, dt);
+  } else {
+    if (in_range) r = pair_march<SP, false, true>(D, M, col, sh, stp, mode, kslot, want_dt, r, rend, dt);
+    if (r < rend) (void)pair_march<SP, false, false>(D, M, col, sh, stp, mode, kslot, want_dt, r, rend, dt);
+  }
+  if (SP == ELECTRONS && want_dt) {
+    // 1/x falls as x grows, so the smallest step size is 1 over the largest inverse; NaN is dropped, as
+    // std::min drops it
+    double m = dt.worst, e = dt.em;
+    for (int off = 32; off > 0; off >>= 1) {
+      const double o = __shfl_xor(m, off, 64), q = __shfl_xor(e, off, 64);
+      m = m < o ? o : m;
+      e = q < e ? q : e;
+    }
+    const double v = m > 0.0 ? 1. / m : DBL_MAX;
+    if (threadIdx.x == 0) TF_PTR(D, partial)[part] = e < v ? e : v;
+  }
+}
+
+// ANYCURL: some domain of the batch has the Maxwell curl terms (their faces take 50 more registers).
+template <bool ANYCURL>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(ANYCURL ? 2 : 3)))
+k_tf_stage_pair(TfBatch b, int Ssel, int Bsel, int Tsel, double mult, int mode, int kslot, int want_dt) {
+  using namespace strip;
+  __shared__ PairShared sh;
+  const int t = xcd_tile(blockIdx.x, b.nstrip_tiles);
+  // the domain is the same in every lane: its description stays in scalar registers
+  const int d = __builtin_amdgcn_readfirstlane(b.strip_dom[t]);
+  const DomView D{reinterpret_cast<uint64_t>(b.doms + d), Ssel, Bsel, Tsel};
+  const Flags strips = D.at<Flags>(offsetof(TfDom, strip_base));   // strip_base, strips_x
+  const int lt = t - strips.first;
+  const int tile = lt / strips.in_range, sidx = lt - tile * strips.in_range;
+  const Mesh M = D.at<Mesh>(offsetof(TfDom, mesh));
+  const int lane = threadIdx.x;
+  const int jraw = tile * OUT_COLS + lane - 2;
+  PairColumn col;
+  bool valid = true;
+  if (M.y.per) col.j = wrapn(jraw, M.ny);
+  else { valid = jraw >= 0 && jraw < M.ny; col.j = clampn(jraw, M.ny); }
+  col.out = lane >= 2 && lane < 62 && jraw >= 0 && jraw < M.ny;
+  col.interior = valid && col.j >= M.y.lo && col.j <= M.y.hi;
+  {   // both wavefronts write, and each reads, the same values
+    const FaceGeom g = face_geom(M.y, col.j);
+    sh.geom[0][lane] = double2{g.hlo, g.hup};
+    sh.geom[1][lane] = double2{g.den, g.rden};
+    sh.geom[2][lane] = double2{g.gup, g.denm};
+    sh.geom[3][lane] = double2{g.rdenm, g.gdn};
+    sh.geom[4][lane] = double2{g.denp, g.rdenp};
+    sh.geom[5][lane] = double2{g.d, g.rd};
+    sh.geom[6][lane] = double2{TF_PTR(D, ky3)[col.j], TF_PTR(D, kyv)[col.j]};
+    struct Kinds { int k[4]; };
+    const Kinds bc = D.at<Kinds>(offsetof(TfDom, bc));
+    col.still = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (bc.k[k] == 2 || bc.k[k] == 3) col.still |= 1 << k;
+  }
+  const double stp = mult * (*TF_PTR(D, step));
+  const int r0 = sidx * b.strip_rows, rend = min(r0 + b.strip_rows, M.nx);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.y) == 0)
+    pair_strip<IONS, ANYCURL>(D, M, col, sh, stp, mode, kslot, want_dt != 0, r0, rend, lt);
+  else
+    pair_strip<ELECTRONS, ANYCURL>(D, M, col, sh, stp, mode, kslot, want_dt != 0, r0, rend, lt);
+}
+
 // ---- persistent form: every phase of nsteps steps of the whole batch in one cooperative launch,
 // one 64-lane wavefront per block, phases separated by grid barriers --------------------------
 
@@ -954,21 +1458,46 @@ k_tf_persistent(TfBatch b, int nsteps, int integrator, int ucnp_mask, int final_
 }
 }  // namespace
 
-void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, hipStream_t s) {
-  if (b.strip_rows > 0)
-    hipLaunchKernelGGL(k_tf_stage_strip, dim3(b.nstrip_tiles), dim3(64), 0, s, b, S, B, T, mult, mode, kslot);
+int tf_strip_rows_default(const int* rows, const int* tiles, int n) {
+  // 1024 blocks (2 wavefronts per SIMD; half as many again without curl terms) run at once and a strip
+  // costs its rows plus about three: the height with the least rounds x cost, the taller of equals
+  int best = 1;
+  long least = 0;
+  for (int R = 1; R <= 64; ++R) {
+    long blocks = 0;
+    for (int k = 0; k < n; ++k) blocks += (long)tiles[k] * ((rows[k] + R - 1) / R);
+    const long cost = (blocks + 1535) / 1536 * (R + 3);
+    if (R == 1 || cost <= least) { best = R; least = cost; }
+  }
+  return best;
+}
+
+void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, bool dt, hipStream_t s) {
+  const int want_dt = dt ? 1 : 0;
+  if (b.strip_rows > 0 && b.any_curl)
+    hipLaunchKernelGGL(k_tf_stage_pair<true>, dim3(b.nstrip_tiles), dim3(64, 2), 0, s, b, S, B, T, mult, mode, kslot, want_dt);
+  else if (b.strip_rows > 0)
+    hipLaunchKernelGGL(k_tf_stage_pair<false>, dim3(b.nstrip_tiles), dim3(64, 2), 0, s, b, S, B, T, mult, mode, kslot, want_dt);
   else
     hipLaunchKernelGGL(k_tf_stage, dim3(b.ntiles), dim3(b.bx, b.by), 0, s, b, S, B, T, mult, mode, kslot);
 }
 
 void launch_tf_ghost(const TfBatch& b, int G, int kinds_mask, int maxn, hipStream_t s) {
-  hipLaunchKernelGGL(k_tf_ghost, dim3((maxn + 127) / 128, b.ndom), dim3(128), 0, s, b, G, kinds_mask, 1);
-  hipLaunchKernelGGL(k_tf_ghost, dim3((maxn + 127) / 128, b.ndom), dim3(128), 0, s, b, G, kinds_mask, 0);
+  // Fixed and reflecting sides also zero momenta of the interior row next to them, which an open side
+  // of the other axis reads: x sides first, then y sides.  The other kinds read interior cells only
+  // and write ghost cells of their own, so all four sides go at once.
+  const unsigned lines = (maxn + 127) / 128;
+  if (kinds_mask & ((1 << 2) | (1 << 3)) && b.stopping_sides) {
+    hipLaunchKernelGGL(k_tf_ghost, dim3(lines, b.ndom, 2), dim3(128), 0, s, b, G, kinds_mask, 0);
+    hipLaunchKernelGGL(k_tf_ghost, dim3(lines, b.ndom, 2), dim3(128), 0, s, b, G, kinds_mask, 2);
+  } else {
+    hipLaunchKernelGGL(k_tf_ghost, dim3(lines, b.ndom, 4), dim3(128), 0, s, b, G, kinds_mask, 0);
+  }
 }
 
-void launch_tf_dt(const TfBatch& b, hipStream_t s) {
-  hipLaunchKernelGGL(k_tf_dt, dim3(b.ntiles), dim3(b.bx, b.by), 0, s, b);
-  hipLaunchKernelGGL(k_tf_reduce, dim3(b.ndom), dim3(256), 0, s, b);
+void launch_tf_dt(const TfBatch& b, bool partials, hipStream_t s) {
+  if (!partials) hipLaunchKernelGGL(k_tf_dt, dim3(b.ntiles), dim3(b.bx, b.by), 0, s, b);
+  hipLaunchKernelGGL(k_tf_reduce, dim3(b.ndom), dim3(256), 0, s, b, partials ? 1 : 0);
 }
 
 void launch_tf_populate(const TfBatch& b, const double* const* itemp, const double* const* etemp, hipStream_t s) {

@@ -27,8 +27,9 @@ struct TfConst {
 };
 
 // One domain as the batched kernels see it (all pointers are device memory).
+// Parts of it are read in 8-byte words: pairs of ints keep their order.
 struct TfDom {
-  TfSet L, W, W2;          // live and stage sets
+  TfSet L, W, W2;          // live and stage sets, first and in TfSetSel's order
   double* k[3];            // RK4 k1..k3 (14 fields each)
   const double *bex, *bey, *gx, *gy;
   const double* kx3;       // per row: (k_x)^2 * 3 with k_x = 2 pi / (2 d_x)   (ideal2F.cpp:175-182)
@@ -42,10 +43,13 @@ struct TfDom {
   double* step;            // device step size of this domain
   double* history;         // step sizes, indexed by *counter
   int* counter;
-  int hist_cap;            // doubles history holds; later step sizes are not stored
-  double* partial;         // one dt minimum per tile
-  int tile_base, tiles_x, tiles_y;
+  double* partial;         // one dt minimum per tile, or per strip where the stage forms them
+  int npartial;
+  int in_range;            // the mesh, masses and gamma allow the untested divisions (range.hpp)
+  uint64_t row_mask[2];    // grav_x, grav_y: all bits set, or 0 where every row equals row 0
   int strip_base, strips_x;  // strip kernel: first strip tile of this domain, strips per column tile
+  int tile_base, tiles_x, tiles_y;
+  int hist_cap;            // doubles history holds; later step sizes are not stored
 };
 
 // tile -> domain map and block shape shared by every launch of a batch
@@ -57,17 +61,23 @@ struct TfBatch {
   const int* strip_dom;    // device: domain of each strip tile (strip stage kernel)
   int nstrip_tiles;
   int strip_rows;          // rows per strip of the stage kernel; 0: one thread per cell
+  int any_curl;            // some domain has the Maxwell curl terms
+  int stopping_sides;      // some domain has a fixed or reflecting side
 };
 
 enum TfStage { TF_STAGE_PLAIN = 0, TF_STAGE_STORE_K = 1, TF_STAGE_RK4_FINAL = 2 };
 enum TfSetSel { TF_SEL_L = 0, TF_SEL_W = 1, TF_SEL_W2 = 2 };
 
-// T = minimums(B + mult*step * k(S)) for every domain of the batch.
-void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, hipStream_t s);
+// T = minimums(B + mult*step * k(S)) for every domain of the batch.  dt (strips only): the stage also
+// writes one minimum of T's per-cell step size per strip, as it is after a ghost fill.
+void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, bool dt, hipStream_t s);
+// rows per strip for these domains (numbers of rows and of 60-column tiles)
+int tf_strip_rows_default(const int* rows, const int* tiles, int n);
 // ghost fill of set G of every domain; kinds_mask selects which boundary kinds act (bit per kind).
 void launch_tf_ghost(const TfBatch& b, int G, int kinds_mask, int maxn, hipStream_t s);
-// per-tile dt minima of the live sets, then one step size per domain.
-void launch_tf_dt(const TfBatch& b, hipStream_t s);
+// per-tile dt minima of the live sets (partials: the last stage has left them per strip), then one step
+// size per domain.
+void launch_tf_dt(const TfBatch& b, bool partials, hipStream_t s);
 void launch_tf_populate(const TfBatch& b, const double* const* itemp, const double* const* etemp, hipStream_t s);
 // variable `which` (TF_DERIVED order of tf_host.hip) of the live set of domain d, and its RHS
 // (14 grids, evolved order); nx, ny are that domain's sizes.

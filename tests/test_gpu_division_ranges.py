@@ -42,13 +42,13 @@ def plant(st, what):
         g["be_x"] = np.full((st.xdim, st.ydim), 1e-60)
 
 
-def check(st, cfg, options, steps=3):
+def check(st, cfg, options, steps=3, names=EVOLVED):
     spec = spec_from_files(cfg, st)
     gpu, ora = GpuDomain(spec, options), OracleDomain(spec)
     try:
         a, b = gpu.step(steps), ora.step(steps)
         assert np.array_equal(a.view(np.int64), b.view(np.int64)), (a, b)
-        for v in EVOLVED:
+        for v in names:
             x, y = gpu.grid(v), ora.grid(v)
             assert np.array_equal(x.view(np.int64), y.view(np.int64)) or np.array_equal(x, y, equal_nan=True), \
                 (v, np.argwhere(x != y)[:4])
@@ -106,3 +106,26 @@ def test_conduction_out_of_range(sat, integ, what):
         check(st, cfg, {"tc_kernel": "strip", "tc_rows": 4}, steps=2)
     finally:
         set_pow_mode(0)
+
+
+@pytest.mark.parametrize("curl", [False, True])
+@pytest.mark.parametrize("what,nx,ny,bc", [("minus_zero", 21, 62, "open_ucnp"), ("tiny", 23, 121, "open_ucnp"),
+                                           ("none", 7, 59, "fixed"), ("none", 16, 120, "reflect"), ("mesh", 14, 61, "periodic")])
+def test_two_fluid(curl, what, nx, ny, bc):
+    """Both species' wavefronts stop together where either finds a value out of range, or a base of -0."""
+    st = W.ucnp_state(nx, ny, seed=nx, v_noise=2e4, e_noise=1e-3)
+    g, i = st.grids, nx // 2
+    if what == "minus_zero":
+        for k in ("i_mom_x", "e_mom_y"):
+            g[k][i:, :] = -0.0
+    elif what == "tiny":
+        g["e_mom_x"][i:i + 2, :] = 1e-70
+        g["i_mom_y"][:, ny // 2:] = 1e-65
+    elif what == "mesh":
+        for k in ("d_x", "d_y", "pos_x", "pos_y"):
+            g[k] = g[k] * 1e-15
+    cfg = W.ucnp_config(steps=4, integrator="rk2", remove_curl_terms=not curl, bc=(bc,) * 4)
+    names = ("i_rho", "e_rho", "i_mom_x", "i_mom_y", "e_mom_x", "e_mom_y", "i_thermal_energy", "e_thermal_energy", "E_x", "E_y",
+             "E_z", "bi_x", "bi_y", "bi_z")
+    check(st, cfg, {"block": "strip4"}, steps=3, names=names)
+    check(st, cfg, {}, steps=3, names=names)
