@@ -102,8 +102,18 @@ __host__ __device__ inline void adj_face_slots(const MhdSet& S, const MhdStatic&
   const double den = ax.fden[c], rden = ax.rfden[c];
   const double wlo = hup * rden, wup = hlo * rden;   // d interp / d q_lower, d interp / d q_upper
   auto interp = [&](double a, double b) { return qdiv(a * hup + b * hlo, den, rden); };
-  const double r1 = S.rho[i1], r2 = S.rho[i2];
-  const double m1[3] = {S.mx[i1], S.my[i1], S.mz[i1]}, m2[3] = {S.mx[i2], S.my[i2], S.mz[i2]};
+  const double* src[T_N] = {S.rho, S.mx, S.my, S.mz, S.te, S.bx, st.bex, S.by, st.bey, S.bz, st.bez};
+  // every value is loaded before the first is used: the branches of the divisions below would each
+  // hold the loads behind them back
+  double u[T_N][4];
+  for (int q = 0; q < T_N; ++q) {
+    u[q][0] = src[q][i0];
+    u[q][1] = src[q][i1];
+    u[q][2] = src[q][i2];
+    u[q][3] = src[q][i3];
+  }
+  const double r1 = u[0][1], r2 = u[0][2];
+  const double m1[3] = {u[1][1], u[2][1], u[3][1]}, m2[3] = {u[1][2], u[2][2], u[3][2]};
   const double v1[3] = {m1[0] / r1, m1[1] / r1, m1[2] / r1};
   const double v2[3] = {m2[0] / r2, m2[1] / r2, m2[2] / r2};
   const double vf = interp(v1[AX], v2[AX]);
@@ -112,11 +122,10 @@ __host__ __device__ inline void adj_face_slots(const MhdSet& S, const MhdStatic&
   const int ce = pos ? cm1 : cp1;
   const double eden = ax.fden[ce], reden = ax.rfden[ce];
   const double t = g * reden;                        // d d1 / d b; d d1 / d a = 1 - t
-  const double* src[T_N] = {S.rho, S.mx, S.my, S.mz, S.te, S.bx, st.bex, S.by, st.bey, S.bz, st.bez};
   const int var_of[T_N] = {AV_RHO, AV_MX, AV_MY, AV_MZ, AV_TE, AV_BX, -1, AV_BY, -1, AV_BZ, -1};
   double g_vf = 0.0;
   for (int q = 0; q < T_N; ++q) {
-    const double q0 = src[q][i0], q1 = src[q][i1], q2 = src[q][i2], q3 = src[q][i3];
+    const double q0 = u[q][0], q1 = u[q][1], q2 = u[q][2], q3 = u[q][3];
     const double d2 = interp(q1, q2);
     const double a = pos ? q0 : q3, b = pos ? q1 : q2;
     const double d1 = a + qdiv((b - a) * g, eden, reden);

@@ -7,6 +7,7 @@
 #include "adj_cell.hpp"
 #include "adjoint.hpp"
 #include "arith.hpp"
+#include "strip.hpp"
 
 namespace spruce {
 namespace {
@@ -126,34 +127,32 @@ __global__ void __launch_bounds__(256) k_adj_rhs_cells(MhdSet S, MhdStatic st, M
   for (int q = 0; q < ADJ_NCOEF; ++q) { cx[q * N + c] = fx[q]; cy[q * N + c] = fy[q]; }
 }
 
-// The face scatter without a global atomic per contribution.  x faces: one thread per column
-// marches a strip of FX_ROWS faces down the rows; a face adds to the rows f-2 .. f+1 of its column,
-// so the thread keeps those four rows' adjoint in registers and writes a row once no later face of
-// the strip can reach it: plainly where no other strip reaches the row either (rows fs+1 ..
-// fe-3 of the strip [fs, fe)), atomically otherwise.  y faces: a 64 x 4 block sums its faces'
-// contributions per row in LDS and writes each cell once, plainly for the cells only its own faces
-// reach (columns j0+1 .. j0+61), atomically for the rest.  The x and y launches run one after the
-// other, so no cell is written plainly by two threads at once.
-constexpr int FX_ROWS = 16;
-
-__global__ void __launch_bounds__(64) k_adj_faces_x(MhdSet S, MhdStatic st, MhdConst K, Mesh M, const double* cx,
-                                                    double* lam_S) {
-  const int j = blockIdx.x * 64 + threadIdx.x;
+// The face scatter, x and y faces in one launch of one-wavefront blocks: the first x_blocks blocks take
+// the x faces, the others the y faces.
+//
+// x faces: one thread per column takes `rows` consecutive faces; a face adds to the rows f-2 .. f+1 of its
+// column, so the thread keeps those four rows' adjoint in registers and adds a row once no later face of
+// its own can reach it.  y faces: a wavefront takes 64 consecutive faces of a row, one per lane; a cell's
+// four faces lie in neighbouring lanes, whose contributions are exchanged by lane shifts, so that lanes
+// 1 .. 61 hold complete sums of 61 cells and neighbouring wavefronts share no cell.  What bounds both is the
+// latency of one wavefront's chain of loads and divisions; at 2048x2048 the two read and write 3.0 GB at
+// 2.6 TB/s.
+__device__ __forceinline__ void adj_faces_x(const MhdSet& S, const MhdStatic& st, const MhdConst& K, const Mesh& M,
+                                            const double* cx, double* lam_S, int block, int rows) {
+  const int cols = (M.ny + 63) / 64, strip = block / cols;
+  const int j = (block - strip * cols) * 64 + threadIdx.x;
   if (j >= M.ny) return;
   const Axis& ax = M.x;
   const size_t N = (size_t)M.nx * M.ny;
-  const int fs = blockIdx.y * FX_ROWS, fe = min(fs + FX_ROWS, M.nx);
+  const int fs = strip * rows, fe = min(fs + rows, M.nx);
   double acc[4][8];
   for (int a = 0; a < 4; ++a)
     for (int v = 0; v < 8; ++v) acc[a][v] = 0.0;
-  auto flush = [&](int row, const double* a8, bool plain) {
+  auto flush = [&](int row, const double* a8) {
     if (!ax.per && (row < 0 || row >= ax.n)) return;
     const size_t c = (size_t)wrapi(row, ax.n, ax.per) * M.ny + j;
-    for (int v = 0; v < 8; ++v) {
-      if (a8[v] == 0.0) continue;
-      if (plain) lam_S[v * N + c] += a8[v];
-      else atomicAdd(&lam_S[v * N + c], a8[v]);
-    }
+    for (int v = 0; v < 8; ++v)
+      if (a8[v] != 0.0) atomicAdd(&lam_S[v * N + c], a8[v]);
   };
   for (int f = fs; f < fe; ++f) {
     if (ax.per || (f >= ax.lo && f <= ax.hi + 1)) {     // faces of interior cells only
@@ -167,27 +166,33 @@ __global__ void __launch_bounds__(64) k_adj_faces_x(MhdSet S, MhdStatic st, MhdC
       }
       if (any) adj_face_slots<0>(S, st, K, M, f, j, fa, [&](int slot, int v, double val) { acc[slot][v] += val; });
     }
-    // row f-2 is complete: later faces of the strip reach rows f-1 and above
-    flush(f - 2, acc[0], f - 3 >= fs);
+    flush(f - 2, acc[0]);   // complete as far as this strip goes: its later faces reach rows f-1 and above
     for (int a = 0; a < 3; ++a)
       for (int v = 0; v < 8; ++v) acc[a][v] = acc[a + 1][v];
     for (int v = 0; v < 8; ++v) acc[3][v] = 0.0;
   }
-  for (int a = 0; a < 3; ++a) flush(fe - 2 + a, acc[a], false);   // rows the next strip reaches too
+  for (int a = 0; a < 3; ++a) flush(fe - 2 + a, acc[a]);
 }
 
-constexpr int FY_W = 64 + 3;   // cells j0-2 .. j0+64 of a row
+constexpr int FY_CELLS = 61;   // cells a wavefront of 64 y faces completes
 
-__global__ void __launch_bounds__(256) k_adj_faces_y(MhdSet S, MhdStatic st, MhdConst K, Mesh M, const double* cy,
-                                                     double* lam_S) {
-  __shared__ double acc[4][8][FY_W];
-  const int li = threadIdx.y, lj = threadIdx.x;
-  for (int t = li * 64 + lj; t < 4 * 8 * FY_W; t += 256) (&acc[0][0][0])[t] = 0.0;
-  __syncthreads();
+template <bool SHARED>
+__device__ __forceinline__ void adj_faces_y(const MhdSet& S, const MhdStatic& st, const MhdConst& K, const Mesh& M,
+                                            const double* cy, double* lam_S, int block) {
   const Axis& ax = M.y;
   const size_t N = (size_t)M.nx * M.ny;
-  const int i = blockIdx.y * 4 + li, j0 = blockIdx.x * 64, j = j0 + lj;
-  if (i < M.nx && j < M.ny && (ax.per || (j >= ax.lo && j <= ax.hi + 1))) {
+  const int tiles = (M.ny + FY_CELLS - 1) / FY_CELLS;
+  const int i = block / tiles, lane = threadIdx.x, base = (block - i * tiles) * FY_CELLS;
+  const int ncell = min(FY_CELLS, M.ny - base);
+  const bool own = lane >= 1 && lane <= ncell;
+  const size_t co = (size_t)i * M.ny + (own ? base + lane - 1 : base);
+  double lam[8], acc[4][8];
+  if (!SHARED)
+    for (int v = 0; v < 8; ++v) lam[v] = lam_S[v * N + co];
+  for (int a = 0; a < 4; ++a)
+    for (int v = 0; v < 8; ++v) acc[a][v] = 0.0;
+  const int j = wrapi(base - 1 + lane, ax.n, ax.per);     // the lane's face: between cells j-1 and j
+  if (lane < ncell + 3 && (ax.per || (j >= ax.lo && j <= ax.hi + 1))) {
     const int fl = wrapi(j - 1, ax.n, ax.per);
     const size_t cu = (size_t)i * M.ny + j, cl = (size_t)i * M.ny + fl;
     double fa[ADJ_NCOEF];
@@ -196,23 +201,32 @@ __global__ void __launch_bounds__(256) k_adj_faces_y(MhdSet S, MhdStatic st, Mhd
       fa[q] = cy[q * N + cl] - cy[q * N + cu];
       any = any || fa[q] != 0.0;
     }
-    if (any)
-      adj_face_slots<1>(S, st, K, M, i, j, fa,
-                        [&](int slot, int v, double val) { atomicAdd(&acc[li][v][lj + slot], val); });
+    if (any) adj_face_slots<1>(S, st, K, M, i, j, fa, [&](int slot, int v, double val) { acc[slot][v] += val; });
   }
-  __syncthreads();
-  for (int t = li * 64 + lj; t < 4 * 8 * FY_W; t += 256) {
-    const int r = t / (8 * FY_W), rem = t - r * (8 * FY_W), v = rem / FY_W, col = rem - v * FY_W;
-    const double val = acc[r][v][col];
-    const int ii = blockIdx.y * 4 + r;
-    if (val == 0.0 || ii >= M.nx) continue;
-    const int jj = j0 - 2 + col;
-    if (!ax.per && (jj < 0 || jj >= ax.n)) continue;
-    const size_t c = (size_t)ii * M.ny + wrapi(jj, ax.n, ax.per);
-    // owned: the faces jj-1 .. jj+2 are all lanes of this block (none wraps round a periodic axis)
-    if (col >= 3 && col <= 63 && jj + 2 < ax.n) lam_S[v * N + c] += val;
-    else atomicAdd(&lam_S[v * N + c], val);
+  // cell j: slot 2 of its own face, slot 1 of face j+1, slot 0 of face j+2, slot 3 of face j-1
+  for (int v = 0; v < 8; ++v) {
+    const double t = acc[2][v] + strip::shl1(acc[1][v]) + strip::shl1(strip::shl1(acc[0][v])) + strip::shr1(acc[3][v]);
+    if (!own) continue;
+    if (SHARED) atomicAdd(&lam_S[v * N + co], t);
+    else lam_S[v * N + co] = lam[v] + t;
   }
+}
+
+__global__ void __launch_bounds__(64) k_adj_faces(MhdSet S, MhdStatic st, MhdConst K, Mesh M, const double* cx,
+                                                  const double* cy, double* lam_S, int x_blocks, int rows) {
+  const int b = blockIdx.x;
+  if (b < x_blocks) adj_faces_x(S, st, K, M, cx, lam_S, b, rows);
+  else adj_faces_y<true>(S, st, K, M, cy, lam_S, b - x_blocks);
+}
+
+__global__ void __launch_bounds__(64) k_adj_faces_x(MhdSet S, MhdStatic st, MhdConst K, Mesh M, const double* cx,
+                                                    double* lam_S, int rows) {
+  adj_faces_x(S, st, K, M, cx, lam_S, blockIdx.x, rows);
+}
+
+__global__ void __launch_bounds__(64) k_adj_faces_y(MhdSet S, MhdStatic st, MhdConst K, Mesh M, const double* cy,
+                                                    double* lam_S) {
+  adj_faces_y<false>(S, st, K, M, cy, lam_S, blockIdx.x);
 }
 
 // per-block (min dt, index) over the interior, std::min semantics (NaN never selected)
@@ -332,11 +346,24 @@ void launch_adj_stage_cells(MhdSet B, const double* kv, const double* step, doub
 
 void launch_adj_faces(MhdSet S, MhdStatic st, MhdConst k, Mesh mesh, const double* cx, const double* cy,
                       double* lam_S, hipStream_t s) {
-  const unsigned cols = (unsigned)((mesh.ny + 63) / 64);
-  hipLaunchKernelGGL(k_adj_faces_x, dim3(cols, (unsigned)((mesh.nx + FX_ROWS - 1) / FX_ROWS)), dim3(64), 0, s, S, st,
-                     k, mesh, cx, lam_S);
-  hipLaunchKernelGGL(k_adj_faces_y, dim3(cols, (unsigned)((mesh.nx + 3) / 4)), dim3(64, 4), 0, s, S, st, k, mesh, cy,
-                     lam_S);
+  // A wavefront needs 5 us for one face per lane and 300 registers, so one fits on a SIMD.  Small grids: x
+  // and y together fill the 1024 SIMDs better than two launches that each leave most of them idle, and the
+  // strips are as short as one residency allows (measured, both axes, us: 128x128 12.5, 192x192 22.5,
+  // 256x256 25.4, 320x320 39 in one launch against 30, 33, 36, 43 in two).  Large grids: two launches, where
+  // the y faces need no atomics (512x512 89 against 96, 2048x2048 1157 against 1477).  Strips of 16 rows, as
+  // many as a quarter of a residency at 256x256, took 142 us there for the x faces alone.
+  const int cols = (mesh.ny + 63) / 64, tiles = (mesh.ny + FY_CELLS - 1) / FY_CELLS;
+  const int y_blocks = tiles * mesh.nx;
+  const auto x_blocks = [&](int rows) { return cols * ((mesh.nx + rows - 1) / rows); };
+  if (y_blocks <= 2048) {
+    const int rows = x_blocks(1) + y_blocks <= 1024 ? 1 : 3;
+    hipLaunchKernelGGL(k_adj_faces, dim3((unsigned)(x_blocks(rows) + y_blocks)), dim3(64), 0, s, S, st, k, mesh, cx, cy,
+                       lam_S, x_blocks(rows), rows);
+  } else {
+    const int rows = 2;
+    hipLaunchKernelGGL(k_adj_faces_x, dim3((unsigned)x_blocks(rows)), dim3(64), 0, s, S, st, k, mesh, cx, lam_S, rows);
+    hipLaunchKernelGGL(k_adj_faces_y, dim3((unsigned)y_blocks), dim3(64), 0, s, S, st, k, mesh, cy, lam_S);
+  }
 }
 
 void launch_adj_dt(MhdSet L, MhdStatic st, MhdConst k, Mesh mesh, double eps, const double* p1, const double* p2,
