@@ -827,16 +827,8 @@ class Domain : public DomainBase {
     rhs_staged(noalloc_scratch(device), out);
   }
 
-  static void copy_set(SetBufs& from, SetBufs& to, size_t N, hipStream_t s) {
-    auto a = from.all(), b = to.all();
-    for (size_t k = 0; k < a.size(); ++k)
-      hip_check(hipMemcpyAsync(b[k]->p, a[k]->p, N * 8, hipMemcpyDeviceToDevice, s), "copy set");
-  }
   static void copy_set(const MhdSet& from, const MhdSet& to, size_t N, hipStream_t s) {
-    const double* a[10] = {from.rho, from.n, from.mx, from.my, from.mz, from.te, from.bx, from.by, from.bz, from.rho_pre};
-    double* b[10] = {to.rho, to.n, to.mx, to.my, to.mz, to.te, to.bx, to.by, to.bz, to.rho_pre};
-    for (int k = 0; k < 10; ++k)
-      hip_check(hipMemcpyAsync(b[k], a[k], N * 8, hipMemcpyDeviceToDevice, s), "copy set");
+    launch_copy_set(from, to, N, s);
   }
   // a set of 10 grids laid out one after another from p
   static MhdSet set_at(double* p, size_t N) {

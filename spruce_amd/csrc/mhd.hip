@@ -95,6 +95,20 @@ __global__ void __launch_bounds__(256) k_mhd_stage(StageArgs a) {
   stage_finish(a, N, c, k);
 }
 
+// One launch for the ten grids of a set: as ten copies a set cost 10 x (3.2 us + the gap between two), two
+// thirds of it launches at 384x512 (15.7 MB), and the gradient makes up to nine such copies per step.
+__global__ void __launch_bounds__(256) k_copy_set(MhdSet from, MhdSet to, size_t N) {
+  const double* a[10] = {from.rho, from.n, from.mx, from.my, from.mz, from.te, from.bx, from.by, from.bz, from.rho_pre};
+  double* b[10] = {to.rho, to.n, to.mx, to.my, to.mz, to.te, to.bx, to.by, to.bz, to.rho_pre};
+  const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (c >= N) return;
+  double v[10];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) v[k] = a[k][c];
+#pragma unroll
+  for (int k = 0; k < 10; ++k) b[k][c] = v[k];
+}
+
 // populateVariablesFromState up to the ghost fill (equationset.cpp:96-104; idealmhd.cpp:226-252).
 __global__ void __launch_bounds__(256) k_mhd_populate(MhdSet L, const double* temp, MhdConst K, int nx, int ny) {
   const size_t N = (size_t)nx * ny;
@@ -378,6 +392,10 @@ __global__ void k_gather_scalars(const double* scal, int n, const double* step, 
 void launch_mhd_stage(const StageArgs& a, hipStream_t s) {
   dim3 b(64, 4);
   hipLaunchKernelGGL(k_mhd_stage, grid2d(a.mesh.nx, a.mesh.ny, b), b, 0, s, a);
+}
+
+void launch_copy_set(MhdSet from, MhdSet to, size_t N, hipStream_t s) {
+  hipLaunchKernelGGL(k_copy_set, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, from, to, N);
 }
 
 void launch_mhd_populate(MhdSet L, const double* temp, MhdConst k, int nx, int ny, hipStream_t s) {

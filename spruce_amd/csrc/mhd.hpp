@@ -116,6 +116,8 @@ void launch_mhd_stage_strip(const StageArgs& a, int R, hipStream_t s);
 int mhd_strip_rows_default(int nx, int ny);
 // blocks (and dt_partial entries) of a launch
 int mhd_strip_blocks(const Mesh& m, int R);
+// to = from, all ten grids
+void launch_copy_set(MhdSet from, MhdSet to, size_t N, hipStream_t s);
 void launch_mhd_populate(MhdSet L, const double* temp, MhdConst k, int nx, int ny, hipStream_t s);
 // Ghost fill of the sides whose kinds[] entry is non-zero; s1/s2 are the open-boundary decay
 // factors of each side (evolution.cpp:166-167), computed on the host with the C library's pow.
