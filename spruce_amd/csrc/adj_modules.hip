@@ -488,10 +488,10 @@ __global__ void __launch_bounds__(64) k_adj_tc_strip(TcStepArgs a, const double*
   const double wc = L.hc * L.rfd, wn = L.hn * L.rfd;   // d(upper y-face)/d(own value, next lane's)
   const int r0 = sidx * R, r1 = min(r0 + R, M.nx);
   tcs::Raw rw = tcs::load_raw<false>(a, L, r0 - 2);
-  const tcs::Row first = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r0 - 2, rw);
+  const tcs::Row first = tcs::make_row<tcs::DIV_PRODUCT>(a, L, r0 - 2, rw);
   rw = tcs::load_raw<false>(a, L, r0 - 1);
-  tcs::Row cur = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r0 - 1, rw);
-  tcs::XFaces lo = tcs::xfaces<false, tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, cur.i), first, cur);
+  tcs::Row cur = tcs::make_row<tcs::DIV_PRODUCT>(a, L, r0 - 1, rw);
+  tcs::XFaces lo = tcs::xfaces<tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, cur.i), first, cur);
   double cn = rw.n;
   tcs::Raw ahead = tcs::load_raw<false>(a, L, r0);
   // adjoints of the previous row (p*) and of the face between it and the current row (f*): T, gy
@@ -504,8 +504,8 @@ __global__ void __launch_bounds__(64) k_adj_tc_strip(TcStepArgs a, const double*
   for (int r = r0 - 1; r <= r1; ++r) {
     const tcs::Raw raw = ahead;
     if (r < r1) ahead = tcs::load_raw<false>(a, L, r + 2);
-    const tcs::Row nxt = tcs::make_row<false, tcs::DIV_PRODUCT>(a, L, r + 1, raw);
-    const tcs::XFaces hi = tcs::xfaces<false, tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, nxt.i), cur, nxt);
+    const tcs::Row nxt = tcs::make_row<tcs::DIV_PRODUCT>(a, L, r + 1, raw);
+    const tcs::XFaces hi = tcs::xfaces<tcs::DIV_PRODUCT>(strip::face_geom_row(M.x, nxt.i), cur, nxt);
     // the cell of row r, as the forward forms it
     const int i = cur.i;
     const double rdx = M.x.rd[i];

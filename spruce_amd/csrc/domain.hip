@@ -469,7 +469,6 @@ class Domain : public DomainBase {
     upload(scratch, host_grids["temp"]);
 
     if (strip_rows == 0) strip_rows = mhd_strip_rows_default(nx, ny);
-    if (tc_rows == 0) tc_rows = tc_strip_rows_default(nx, ny);
     if (tc_kernel < 0) tc_kernel = 0;   // the strips are the faster form at every size
     fuse_dt = !any_moc;
     for (auto& m : mods) fuse_dt = fuse_dt && !m->acts_after_integrator();
@@ -946,6 +945,7 @@ struct TcModule : GpuModule {
   std::string integ = "euler";
   bool inactive = false;
   DBuf ta, tb, tc, k1, k2, k3, rx, ry, coef, dbxx, dbxy, dbyx, dbyy;
+  int strip_rows = 0;      // rows per strip of the update unless the option tc_rows names them
   bool to_file = false;           // output_to_file: the average heating rate and the saturation factor
   double msf = 1.0;               // ms_electron_heating_fraction (thermalconduction.hpp:34)
   DBuf avg, sat;
@@ -1006,6 +1006,7 @@ struct TcModule : GpuModule {
     dbxx.alloc(d.N); dbxy.alloc(d.N); dbyx.alloc(d.N); dbyy.alloc(d.N);
     if (integ == "rk4") { k1.alloc(d.N); k2.alloc(d.N); k3.alloc(d.N); }
     if (p.saturation) { rx.alloc(d.N); ry.alloc(d.N); coef.alloc(d.N); }
+    strip_rows = tc_strip_rows_default(d.nx, d.ny, p.saturation);
     if (to_file) { alloc_zero(avg, d.N, d.stream); alloc_zero(sat, d.N, d.stream); }
   }
   void file_output(OutList& o) override {  // thermalconduction.cpp:229-239
@@ -1032,7 +1033,8 @@ struct TcModule : GpuModule {
   }
   void step(Domain& d, const double* src, const double* base, double* out, double mult, int mode, double* kout,
             double h) {
-    if (p.saturation)
+    const bool strips = d.tc_kernel != 1;     // which form the saturated flux themselves
+    if (p.saturation && !strips)
       d.timed("tc_sat", [&] {
         launch_tc_sat(src, d.L.n.p, d.L.rho.p, d.bhx.p, d.bhy.p, p, d.kc, d.mesh, rx.p, ry.p, coef.p, d.stream);
       });
@@ -1043,7 +1045,8 @@ struct TcModule : GpuModule {
     a.dbxx = dbxx.p; a.dbxy = dbxy.p; a.dbyx = dbyx.p; a.dbyy = dbyy.p;
     a.mesh = d.mesh;
     a.in_range = d.in_range ? 1 : 0;
-    a.rows = d.tc_kernel == 1 ? 0 : d.tc_rows;
+    a.rho = d.L.rho.p;
+    a.rows = !strips ? 0 : d.tc_rows ? d.tc_rows : strip_rows;
     d.timed("tc_step", [&] { launch_tc_step(a, d.stream); });
   }
   void iterate(Domain& d, double dt) override {  // thermalconduction.cpp:91-156

@@ -84,17 +84,27 @@ __global__ void __launch_bounds__(256) k_bhat_derivs(const double* bhx, const do
 
 // Field-aligned conductive flux at an interior cell and its saturated magnitude
 // (thermalconduction.cpp:198-232).
+// IN: T and rho in range (range.hpp), so that T^2.5 and (T K_B)^1.5 need no operand tests.
 struct SatFlux { double fx, fy, fm, sfm; };
+template <bool IN = false>
 __device__ __forceinline__ SatFlux sat_flux(double T, double gx, double gy, double rho, double bx, double by,
                                             double dx, double dy, const TcParams& p, const MhdConst& K) {
   const double kmax = qdiv(dx * dy * K_B * qdiv(rho, K.m, K.rm), p.dsm, 1.0 / p.dsm);
-  const double kap = smin(pow_2p5(T) * p.k0, kmax);
+  double t15 = 0.0, t25, k15, k25 = 0.0;
+  if (IN) {
+    pow_1p5_2p5_in(T, t15, t25);
+    pow_1p5_2p5_in(T * K_B, k15, k25);
+  } else {
+    t25 = pow_2p5(T);
+    k15 = pow_1p5(T * K_B);
+  }
+  const double kap = smin(t25 * p.k0, kmax);
   const double cfx = (-kap) * gx, cfy = (-kap) * gy;
   const double fmag = cfx * bx + cfy * by;
   SatFlux s;
   s.fx = fmag * bx;
   s.fy = fmag * by;
-  const double sat = qdiv(rho, K.m, K.rm) * p.c_sat * pow_1p5(T * K_B) / p.sqrt_me;
+  const double sat = qdiv(rho, K.m, K.rm) * p.c_sat * k15 / p.sqrt_me;
   s.fm = sqrt(s.fx * s.fx + s.fy * s.fy);
   const double scale = sat / sqrt(sat * sat + s.fm * s.fm);
   const double sx = s.fx * scale, sy = s.fy * scale;
@@ -266,58 +276,47 @@ __global__ void __launch_bounds__(256) k_tc_step(TcStepArgs a) {
 // each of ~20 divisions and both powers share one square root, so a row is about 250 VALU
 // instructions in one run instead of 400 in twenty pieces (1.78e7 against 2.79e7 a launch), and the
 // row's geometry comes through the scalar cache, so that nothing waits for the row being fetched but
-// its use.  Measured per subcycle: 2048x2048 79.5 -> 52.7 us, 512x1024 17.5 (one thread per cell) ->
-// 13.5 us, 133x197 7.7 -> 7.2 us.  109 VGPRs, four wavefronts per SIMD.
+// its use.  Measured per subcycle: 2048x2048 79.5 -> 51.8 us, 512x1024 17.5 (one thread per cell) ->
+// 12.3 us, 133x197 7.7 -> 7.2 us.  160 VGPRs, three wavefronts per SIMD: at four (128) the two register
+// sets of a pair of rows spill.
+//
+// With flux saturation the march also forms the saturated flux and coefficient of each row, from the
+// temperature gradient it has there, and writes a row once the next row's coefficient is known: its cells
+// reach two rows and two lanes to each side, so lane l holds column 60*tile + l - 2 and lanes 2..61 write.
+// As a kernel of its own, which formed temperatures and gradients again, the coefficient took 24.5 us
+// per update at 700x1301 beside the update's 19.3; together they take 28.5.  VALU-bound; 213 VGPRs, two
+// wavefronts per SIMD (three spill).
 //
 // Rows rs .. rend-1.  D = DIV_IN: the geometric divisions and the powers without their operand tests;
 // every row is tested once it is formed, and the march stops before the first row whose stencil holds
 // a value out of range.  Returns the row it stopped at (rend when done).
+struct SatRow { double te, dE, fx, fy, coef, clo; };   // a row waiting for the next; clo: its lower x-face's coefficient
+
 template <int MODE, bool SAT, bool SEP, int D>
 __device__ __forceinline__ int tc_march(const TcStepArgs& a, const tcs::Lane& L, int rs, int rend) {
   using namespace tcs;
   const Mesh& M = a.mesh;
   constexpr bool IN = D == DIV_IN;
+  constexpr int LAG = SAT ? 1 : 0;          // rows between the one formed and the one written
+  const int lane = threadIdx.x;
+  const int first = rs - LAG, last = rend + LAG;
   Row cur;
-  FaceGeom g = strip::face_geom_row(M.x, rs);
+  FaceGeom g = strip::face_geom_row(M.x, first);
   XFaces lo;
   {
-    const Raw rp = load_raw<SAT>(a, L, rs - 1), rc = load_raw<SAT>(a, L, rs);
-    const Row prev = make_row<SAT, D>(a, L, rs - 1, rp);
-    cur = make_row<SAT, D>(a, L, rs, rc);
+    const Raw rp = load_raw<SAT>(a, L, first - 1), rc = load_raw<SAT>(a, L, first);
+    const Row prev = make_row<D>(a, L, first - 1, rp);
+    cur = make_row<D>(a, L, first, rc);
     if (IN && __any(row_out<SAT>(prev, rp) || row_out<SAT>(cur, rc))) return rs;
-    lo = xfaces<SAT, D>(g, prev, cur);
+    lo = xfaces<D>(g, prev, cur);
   }
-  // Row r from row r+1's values (raw), with row r+2 asked for first; false when the march ends before
-  // it.  What row r leaves for the next is written to the second of each pair, so that two rows in
-  // turn swap the pairs and nothing is copied.
-  auto step = [&](int r, const Raw& raw, Raw& ahead, const Row& cur, Row& nxt, const XFaces& lo, XFaces& hi,
-                  const FaceGeom& g, FaceGeom& gn) -> bool {
-    ahead = load_raw<SAT>(a, L, r + 2);
+  // writes row r from its energy derivative
+  auto write = [&](int r, double te, double dE) {
     const size_t row = (size_t)r * M.ny;
     uint32_t jb = 8u * (uint32_t)L.j;
     strip::lane_offset(jb);
-    const double base = SEP ? strip::ld_row(a.te_base, row, jb) : cur.te;
-    gn = strip::face_geom_row(M.x, r + 1);
-    nxt = make_row<SAT, D>(a, L, r + 1, raw);
-    if (IN && __any(row_out<SAT>(nxt, raw))) return false;
-    hi = xfaces<SAT, D>(gn, cur, nxt);
-    // cell values at row r along x
-    const double dx = g.d, rdx = g.rd;
-    const bool in = cur.inx && L.iny;
-    const double gx = qd<D>(hi.T - lo.T, dx, rdx);
-    // dtemp_dx is zero outside the interior; its y-derivative takes the neighbouring lanes' values
-    const double dgx_y = yderiv<D>(L, yface<D>(L, in ? gx : 0.0));
-    const double s0 = qd<D>(hi.T - 2.0 * cur.T + lo.T, g.hsq, g.rhsq);
-    const double dgy_x = qd<D>(hi.gy - lo.gy, dx, rdx);
-    const double dbxx = qd<D>(hi.bx - lo.bx, dx, rdx);
-    const double dbyx = qd<D>(hi.by - lo.by, dx, rdx);
-    double dE = tcc::tc_combine<double, IN>(cur.T, gx, cur.gy, s0, cur.s1, dgx_y, dgy_x, cur.bx, cur.by, dbxx, cur.dbxy,
-                                            dbyx, cur.dbyy, a.p.k0);
-    if (SAT) {                                                  // thermalconduction.cpp:171-174, 255-271
-      const double dcx = qd<D>(hi.coef - lo.coef, dx, rdx);
-      const double add = -1.0 * (dcx * strip::ld_row(a.rx, row, jb) + cur.dcy * strip::ld_row(a.ry, row, jb));
-      dE = cur.coef * dE + add;
-    }
+    const double base = SEP ? strip::ld_row(a.te_base, row, jb) : te;
+    const bool in = r >= M.x.lo && r <= M.x.hi && L.iny;
     dE = in ? dE : 0.0;   // every derivative is zero outside the interior
     double v;
     if (MODE == TC_RK4_FINAL) {
@@ -328,38 +327,94 @@ __device__ __forceinline__ int tc_march(const TcStepArgs& a, const tcs::Lane& L,
       v = base + 1.0 * (a.mult * a.h) * dE;
     }
     // mask = 0 there: te + 0*dE
-    const double te = smax(in ? v : base + 0.0, a.k.temin);
+    const double out = smax(in ? v : base + 0.0, a.k.temin);
     if (L.out) {
       if (MODE == TC_STORE_K) strip::st_row(a.k_out, row, jb, dE);
-      strip::st_row(a.te_out, row, jb, te);
+      strip::st_row(a.te_out, row, jb, out);
     }
+  };
+  // Row r from row r+1's values (raw), with row r+2 asked for first; false when the march ends before
+  // it.  What row r leaves for the next is written to the second of each pair, so that two rows in
+  // turn swap the pairs and nothing is copied.
+  auto step = [&](int r, const Raw& rc, const Raw& raw, Raw& ahead, const Row& cur, Row& nxt, const XFaces& lo,
+                  XFaces& hi, const FaceGeom& g, FaceGeom& gn, const SatRow& sp, SatRow& sn, double dx_p,
+                  double rdx_p) -> bool {
+    ahead = load_raw<SAT>(a, L, r + 2);
+    gn = strip::face_geom_row(M.x, r + 1);
+    nxt = make_row<D>(a, L, r + 1, raw);
+    if (IN && __any(row_out<SAT>(nxt, raw))) return false;
+    hi = xfaces<D>(gn, cur, nxt);
+    // cell values at row r along x
+    const double dx = g.d, rdx = g.rd;
+    const bool in = cur.inx && L.iny;
+    const double gx = qd<D>(hi.T - lo.T, dx, rdx);
+    // dtemp_dx is zero outside the interior; its y-derivative takes the neighbouring lanes' values
+    const double dgx_y = yderiv<D>(L, yface<D>(L, in ? gx : 0.0));
+    const double s0 = qd<D>(hi.T - 2.0 * cur.T + lo.T, g.hsq, g.rhsq);
+    const double dgy_x = qd<D>(hi.gy - lo.gy, dx, rdx);
+    const double dbxx = qd<D>(hi.bx - lo.bx, dx, rdx);
+    const double dbyx = qd<D>(hi.by - lo.by, dx, rdx);
+    const double dE = tcc::tc_combine<double, IN>(cur.T, gx, cur.gy, s0, cur.s1, dgx_y, dgy_x, cur.bx, cur.by, dbxx,
+                                                  cur.dbxy, dbyx, cur.dbyy, a.p.k0);
+    if (!SAT) {
+      write(r, cur.te, dE);
+      return true;
+    }
+    const SatFlux f = sat_flux<IN>(cur.T, gx, cur.gy, rc.rho, cur.bx, cur.by, dx, L.dy, a.p, a.k);
+    sn.te = cur.te;
+    sn.dE = dE;
+    sn.fx = f.fx;
+    sn.fy = f.fy;
+    sn.coef = in && f.fm != 0.0 ? f.sfm / f.fm : 1.0;           // thermalconduction.cpp:264-268
+    if (IN) {
+      RangeTest t;
+      t.add(sn.coef);
+      if (__any(t.out() && lane >= 1 && lane <= 62)) return false;
+    }
+    // row r-1, whose upper x-face the coefficient now has (thermalconduction.cpp:171-174, 255-271)
+    sn.clo = qd<D>(sp.coef * g.hup + sn.coef * g.hlo, g.den, g.rden);
+    if (r <= rs) return true;
+    const double dcx = qd<D>(sn.clo - sp.clo, dx_p, rdx_p);
+    const double dcy = yderiv<D>(L, yface<D>(L, sp.coef));
+    const double add = -1.0 * (dcx * sp.fx + dcy * sp.fy);
+    write(r - 1, sp.te, sp.coef * sp.dE + add);
     return true;
   };
-  Raw raw[2];
+  Raw raw[2], rowraw = {};
   Row rows[2];
   XFaces faces[2];
   FaceGeom geom[2];
-  raw[0] = load_raw<SAT>(a, L, rs + 1);
+  SatRow sat[2] = {};
+  raw[0] = load_raw<SAT>(a, L, first + 1);
+  if (SAT) raw[1] = load_raw<SAT>(a, L, first);     // its density is the first row's
   rows[0] = cur;
   faces[0] = lo;
   geom[0] = g;
-  for (int r = rs; r < rend; r += 2) {
-    if (!step(r, raw[0], raw[1], rows[0], rows[1], faces[0], faces[1], geom[0], geom[1])) return r;
-    if (r + 1 >= rend) break;
-    if (!step(r + 1, raw[1], raw[0], rows[1], rows[0], faces[1], faces[0], geom[1], geom[0])) return r + 1;
+  geom[1] = g;
+  for (int r = first; r < last; r += 2) {
+    rowraw.rho = raw[1].rho;
+    double d = geom[1].d, rd = geom[1].rd;
+    if (!step(r, rowraw, raw[0], raw[1], rows[0], rows[1], faces[0], faces[1], geom[0], geom[1], sat[0], sat[1], d, rd))
+      return max(r - LAG, rs);
+    if (r + 1 >= last) break;
+    rowraw.rho = raw[0].rho;
+    d = geom[0].d, rd = geom[0].rd;
+    if (!step(r + 1, rowraw, raw[1], raw[0], rows[1], rows[0], faces[1], faces[0], geom[1], geom[0], sat[1], sat[0], d, rd))
+      return max(r + 1 - LAG, rs);
   }
   return rend;
 }
 
 template <int MODE, bool SAT, bool SEP>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3)))
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(SAT ? 2 : 3)))
 k_tc_strip(TcStepArgs a, int R, int nstrips, int total) {
   const Mesh& M = a.mesh;
   const int t = strip::xcd_tile(blockIdx.x, total);
   const int tile = t / nstrips, sidx = t - tile * nstrips;
-  const int lane = threadIdx.x, jc = tile * 62 + lane - 1;
+  constexpr int HALO = SAT ? 2 : 1;
+  const int lane = threadIdx.x, jc = tile * (64 - 2 * HALO) + lane - HALO;
   tcs::Lane L = tcs::lane_at(M, jc);
-  L.out = lane >= 1 && lane <= 62 && jc < M.ny;
+  L.out = lane >= HALO && lane < 64 - HALO && jc < M.ny;
   const int r0 = sidx * R, r1 = min(r0 + R, M.nx);
   int r = r0;
   if (a.in_range) r = tc_march<MODE, SAT, SEP, tcs::DIV_IN>(a, L, r, r1);
@@ -490,14 +545,16 @@ void launch_tc_sat(const double* te_src, const double* n, const double* rho, con
                      coef);
 }
 
-int tc_strip_rows_default(int nx, int ny) {
-  // 3072 wavefronts (3 per SIMD) run at once and a strip costs its rows plus about five (three rows to
-  // start with, the launch): the height with the least rounds x cost, the taller one of equals
-  const long tiles = (ny + 61) / 62;
+int tc_strip_rows_default(int nx, int ny, bool saturation) {
+  // 3072 wavefronts (3 per SIMD, 2 with saturation) run at once and a strip costs its rows plus about five
+  // (three rows to start with, the launch; two rows more with saturation): the height with the least
+  // rounds x cost, the taller one of equals
+  const int cols = saturation ? 60 : 62, waves = saturation ? 2048 : 3072, extra = saturation ? 7 : 5;
+  const long tiles = (ny + cols - 1) / cols;
   int best = 1;
   long least = 0;
   for (int R = 1; R <= 96; ++R) {
-    const long cost = (tiles * ((nx + R - 1) / R) + 3071) / 3072 * (R + 5);
+    const long cost = (tiles * ((nx + R - 1) / R) + waves - 1) / waves * (R + extra);
     if (R == 1 || cost <= least) { best = R; least = cost; }
   }
   return best;
@@ -505,7 +562,8 @@ int tc_strip_rows_default(int nx, int ny) {
 
 template <int MODE, bool SAT>
 static void launch_tc_strip_m(const TcStepArgs& a, int R, hipStream_t s) {
-  const int tiles = (a.mesh.ny + 61) / 62, nstrips = (a.mesh.nx + R - 1) / R, total = tiles * nstrips;
+  constexpr int COLS = SAT ? 60 : 62;
+  const int tiles = (a.mesh.ny + COLS - 1) / COLS, nstrips = (a.mesh.nx + R - 1) / R, total = tiles * nstrips;
   if (a.te_base != a.te_src)
     hipLaunchKernelGGL((k_tc_strip<MODE, SAT, true>), dim3(total), dim3(64), 0, s, a, R, nstrips, total);
   else

@@ -45,6 +45,7 @@ struct TcStepArgs {
   const double* k1;
   const double* k2;
   const double* k3;
+  const double* rho;      // flux saturation, strip form
   const double* dbxx;     // derivatives of the frozen b_hat (d b_hat_x/dx, d b_hat_x/dy, d b_hat_y/dx,
   const double* dbxy;     // d b_hat_y/dy), computed once per step
   const double* dbyx;
@@ -74,7 +75,7 @@ void launch_tc_sat(const double* te_src, const double* n, const double* rho, con
 // when a.rows is 0 (the b_hat derivative grids are then read, else they are formed in the kernel).
 void launch_tc_step(const TcStepArgs& a, hipStream_t s);
 // rows per strip of the strip form, chosen from the grid size
-int tc_strip_rows_default(int nx, int ny);
+int tc_strip_rows_default(int nx, int ny, bool saturation);
 // RL subcycle count inputs: out[0] = max losses, out[1] = min |te / losses| (radiativelosses.cpp:200-205).
 void launch_rl_pre(MhdSet L, const double* dt_grid, RlParams p, MhdConst k, Mesh mesh, double* partial, int nblocks,
                    double* out, hipStream_t s);

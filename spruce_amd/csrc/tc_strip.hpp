@@ -32,12 +32,11 @@ __device__ __forceinline__ double qd(double a, double b, double rb) {
 // one row of the strip at this lane: cell values and the quantities that need only y-neighbours
 struct Row {
   double T, te, gy, s1, bx, by, dbxy, dbyy;
-  double coef, dcy;          // flux saturation: coefficient and its y-derivative
   int i;                     // wrapped row index (clamped into [0, nx) when the row lies outside)
   bool val, inx;             // row exists; row inside the interior bounds
 };
-struct Raw { double te, n, bx, by, coef; };
-struct XFaces { double T, gy, bx, by, coef; };
+struct Raw { double te, n, bx, by, rho; };   // rho: flux saturation only
+struct XFaces { double T, gy, bx, by; };
 
 struct Lane {
   int j;                     // wrapped column (clamped into [0, ny) when it lies outside)
@@ -98,11 +97,11 @@ __device__ __forceinline__ Raw load_raw(const TcStepArgs& a, const Lane& L, int 
   r.n = strip::ld_row(a.n, row, jb);
   r.bx = strip::ld_row(a.bhx, row, jb);
   r.by = strip::ld_row(a.bhy, row, jb);
-  r.coef = SAT ? strip::ld_row(a.coef, row, jb) : 0.0;
+  r.rho = SAT ? strip::ld_row(a.rho, row, jb) : 0.0;
   return r;
 }
 
-template <bool SAT, int D>
+template <int D>
 __device__ __forceinline__ Row make_row(const TcStepArgs& a, const Lane& L, int k, const Raw& r) {
   const Mesh& M = a.mesh;
   Row w;
@@ -120,10 +119,6 @@ __device__ __forceinline__ Row make_row(const TcStepArgs& a, const Lane& L, int 
   w.s1 = qd<D>(fT - 2.0 * w.T + fTlo, L.hsq, L.rhsq);      // secondDerivative1D (derivs.cpp:450)
   w.dbxy = yderiv<D>(L, yface<D>(L, w.bx));
   w.dbyy = yderiv<D>(L, yface<D>(L, w.by));
-  if (SAT) {
-    w.coef = r.coef;
-    w.dcy = yderiv<D>(L, yface<D>(L, w.coef));
-  }
   return w;
 }
 
@@ -133,19 +128,18 @@ __device__ __forceinline__ bool row_out(const Row& w, const Raw& r) {
   RangeTest t;
   t.add(w.bx);
   t.add(w.by);
-  if (SAT) t.add(w.coef);
+  if (SAT) t.density(r.rho);
   return t.out() || !(w.T >= 0x1p-100 && w.T <= 0x1p+100) || !(r.n >= 0x1p-100 && r.n <= 0x1p+150);
 }
 
 // boundaryInterpolate across the x-face between rows A (lower) and B (upper), whose geometry is g
-template <bool SAT, int D>
+template <int D>
 __device__ __forceinline__ XFaces xfaces(const FaceGeom& g, const Row& A, const Row& B) {
   XFaces f;
   f.T = qd<D>(A.T * g.hup + B.T * g.hlo, g.den, g.rden);
   f.gy = qd<D>(A.gy * g.hup + B.gy * g.hlo, g.den, g.rden);
   f.bx = qd<D>(A.bx * g.hup + B.bx * g.hlo, g.den, g.rden);
   f.by = qd<D>(A.by * g.hup + B.by * g.hlo, g.den, g.rden);
-  if (SAT) f.coef = qd<D>(A.coef * g.hup + B.coef * g.hlo, g.den, g.rden);
   return f;
 }
 
