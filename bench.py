@@ -71,9 +71,9 @@ def kernel_bytes_per_cell(name: str, integrator: str):
     table = {
         "mhd_stage": stage_bytes_per_cell(integrator),
         "tc_step": 40.0,          # one Euler conduction subcycle: te, n, b_hat_x, b_hat_y read, te written
-        "rl_iterate": 24.0,       # all radiative subcycles of a step: te, n read, te written
+        "rl_iterate": 48.0,       # all radiative subcycles of a step and the minimums: te, n, rho read and written
         "mhd_dt": 88.0,           # 8 evolved + be_x/y/z read
-        "bhat": 64.0,             # be_x/y/z, bi_x/y/z read, b_hat_x/y written
+        "step_pre": 88.0,         # be_x/y/z, bi_x/y/z, te, n, rho read, b_hat_x/y written
         "propagate_live": 48.0,   # rho, te read; n, rho, te written
     }
     return table.get(name)

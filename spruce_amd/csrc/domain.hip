@@ -88,8 +88,9 @@ struct SetBufs {
 };
 
 
-// One Module of the reference plugin API (module.hpp:15-58) on the GPU.  pre_launch() enqueues the
-// reductions its subcycle count needs; pre_finish() turns their results into the count on the host
+// One Module of the reference plugin API (module.hpp:15-58) on the GPU.  pre_fill() enters the
+// reductions its subcycle count needs into the step's one pass over the live grids, pre_launch()
+// enqueues what else it needs before the subcycles; pre_finish() turns their results into the count on the host
 // after the domain's one synchronisation per step; iterate() enqueues the subcycles and the live
 // propagate that ends every reference iterateModule.
 struct GpuModule {
@@ -97,12 +98,14 @@ struct GpuModule {
   int nsub = -1;
   virtual ~GpuModule() = default;
   virtual void setup(Domain& d) = 0;
-  virtual void pre_launch(Domain& d, double* scal) = 0;
+  // false when the arguments already hold another module of this kind
+  virtual bool pre_fill(Domain&, StepPreArgs&, double* /*partial*/) { return true; }
+  virtual void pre_launch(Domain&) {}
   virtual void pre_finish(double dt, const double* scal) = 0;
   virtual void iterate(Domain& d, double dt) = 0;
   virtual bool needs_bhat() const { return false; }
   virtual bool needs_dt_grid() const { return false; }
-  // false when pre_launch/pre_finish do nothing (no subcycle-count reduction to read back)
+  // false when pre_fill/pre_finish do nothing (no subcycle-count reduction to read back)
   virtual bool needs_pre_scalars() const { return true; }
   // iterate() has work to do
   virtual bool iterates() const { return true; }
@@ -320,7 +323,7 @@ class Domain : public DomainBase {
   }
 
   std::vector<std::unique_ptr<GpuModule>> mods;
-  DBuf bhx, bhy, dtgrid, mod_partial, mod_scal;
+  DBuf bhx, bhy, dtgrid, mod_partial;
   std::vector<int32_t> sub_hist;
   bool need_dt_grid = false;
 
@@ -496,8 +499,7 @@ class Domain : public DomainBase {
     if (!mods.empty()) {
       bhx.alloc(N);
       bhy.alloc(N);
-      mod_partial.alloc(2 * (size_t)solar_blocks(mesh));
-      mod_scal.alloc(2 * mods.size());
+      mod_partial.alloc(2 * (size_t)solar_blocks(mesh) * mods.size());
       hip_check(hipHostMalloc((void**)&hscal, (2 * mods.size() + 2) * sizeof(double)), "hipHostMalloc");
       for (auto& m : mods) {
         m->setup(*this);
@@ -555,6 +557,9 @@ class Domain : public DomainBase {
   // iterateModule ends (e.g. thermalconduction.cpp:154-155).
   void propagate_live() {
     timed("propagate_live", [&] { launch_propagate_live(L.view(), kc, nx, ny, any_open ? 1 : 0, stream); });
+    finish_propagate();
+  }
+  void finish_propagate() {   // the rest of propagate_live() once minimums and derived variables are done
     ghost(L, kinds_all, GHOST_NORMAL);
     moc_limit(L.view());
   }
@@ -563,22 +568,46 @@ class Domain : public DomainBase {
   void run_modules(int s) {
     bool bh = false;
     for (auto& m : mods) bh = bh || m->needs_bhat();
-    if (bh) timed("bhat", [&] { launch_bhat(L.view(), stat(), mesh, bhx.p, bhy.p, stream); });
     bool host = false;
     for (auto& m : mods) host = host || m->needs_pre_scalars() || m->needs_host_dt();
-    for (size_t k = 0; k < mods.size(); ++k) mods[k]->pre_launch(*this, mod_scal.p + 2 * k);
+    StepPreArgs pre{};
+    const auto launch_pre = [&] {
+      if (pre.bhx || pre.tc_partial || pre.rl_partial) timed("step_pre", [&] { launch_step_pre(pre, stream); });
+    };
+    const auto begin_pre = [&] {
+      pre = StepPreArgs{};
+      pre.L = L.view();
+      pre.st = stat();
+      pre.k = kc;
+      pre.mesh = mesh;
+      if (bh) { pre.bhx = bhx.p; pre.bhy = bhy.p; }
+    };
+    begin_pre();
+    const int nblocks = solar_blocks(mesh);
+    int njobs = 0;
+    for (auto& m : mods)
+      if (m->needs_pre_scalars()) {
+        double* partial = mod_partial.p + (size_t)2 * nblocks * njobs++;
+        if (m->pre_fill(*this, pre, partial)) continue;
+        launch_pre();               // a second module of a kind: a pass of its own
+        begin_pre();
+        m->pre_fill(*this, pre, partial);
+      }
+    launch_pre();
+    for (auto& m : mods) m->pre_launch(*this);
     double dt = std::nan("");
     if (host) {
-      const int ns = 2 * (int)mods.size();
-      launch_gather_scalars(mod_scal.p, ns, step.p, err_flag, hscal, stream);
+      launch_finish_scalars(mod_partial.p, nblocks, njobs, step.p, err_flag, hscal, stream);
       hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
-      if (hscal[ns + 1] != 0.0) {
+      if (hscal[2 * njobs + 1] != 0.0) {
         hip_check(hipMemset(err_flag, 0, sizeof(int)), "hipMemset");
         throw Error(SPRUCE_E_NUMERIC, "Something went wrong in the min calculation (no finite dt)");
       }
-      const std::vector<double> sc(hscal, hscal + ns + 1);
-      dt = sc[ns];
-      for (size_t k = 0; k < mods.size(); ++k) mods[k]->pre_finish(dt, sc.data() + 2 * k);
+      const std::vector<double> sc(hscal, hscal + 2 * njobs + 1);
+      dt = sc[2 * njobs];
+      int job = 0;
+      for (auto& m : mods)
+        if (m->needs_pre_scalars()) m->pre_finish(dt, sc.data() + 2 * job++);
     }
     host_dt = dt;
     have_host_dt = host;
@@ -1014,16 +1043,18 @@ struct TcModule : GpuModule {
     o.emplace_back("thermal_conduction", avg.p);
     o.emplace_back("flux_saturation", sat.p);
   }
-  void pre_launch(Domain& d, double* scal) override {
+  bool pre_fill(Domain&, StepPreArgs& a, double* partial) override {
+    if (a.tc_partial) return false;
+    a.tc = p;
+    a.tc_partial = partial;
+    return true;
+  }
+  void pre_launch(Domain& d) override {
     // the strip form of the update forms the b_hat derivatives itself; the grids serve the cell
     // form and the adjoint's replay
     if (d.tc_kernel == 1 || (recording && (reuse || slot < 0)))
       d.timed("bhat_derivs",
               [&] { launch_bhat_derivs(d.bhx.p, d.bhy.p, d.mesh, dbxx.p, dbxy.p, dbyx.p, dbyy.p, d.stream); });
-    d.timed("tc_pre", [&] {
-      launch_tc_pre(d.L.view(), d.bhx.p, d.bhy.p, p, d.kc, d.mesh, d.mod_partial.p, solar_blocks(d.mesh), scal,
-                    d.stream);
-    });
   }
   void pre_finish(double dt, const double* scal) override {  // thermalconduction.cpp:179-193
     if (p.saturation && scal[1] == 0.0) { nsub = 0; return; }
@@ -1171,11 +1202,13 @@ struct RlModule : GpuModule {
   void file_output(OutList& o) override {  // radiativelosses.cpp:174-181
     if (to_file) o.emplace_back("rad", avg.p);
   }
-  void pre_launch(Domain& d, double* scal) override {
+  bool pre_fill(Domain& d, StepPreArgs& a, double* partial) override {
+    if (a.rl_partial) return false;
     if (p.prevent) d.refresh_dt_grid();
-    d.timed("rl_pre", [&] {
-      launch_rl_pre(d.L.view(), d.dtgrid.p, p, d.kc, d.mesh, d.mod_partial.p, solar_blocks(d.mesh), scal, d.stream);
-    });
+    a.rl = p;
+    a.dt_grid = d.dtgrid.p;
+    a.rl_partial = partial;
+    return true;
   }
   void pre_finish(double dt, const double* scal) override {  // radiativelosses.cpp:200-205
     if (scal[1] == 0.0) { nsub = 0; return; }
@@ -1188,7 +1221,12 @@ struct RlModule : GpuModule {
     h_last = h;
     if (p.prevent) d.refresh_dt_grid();
     const int ig = integ == "euler" ? 0 : (integ == "rk2" ? 1 : 2);
-    d.timed("rl_iterate", [&] { launch_rl_iterate(d.L.view(), d.dtgrid.p, p, d.kc, d.mesh, nsub, h, ig, tout.p, d.stream); });
+    // the pass that ends the iterate reads te before and after where something else is derived from both
+    const bool propagate = !to_file && !d.multispecies_on && !inactive;
+    d.timed("rl_iterate", [&] {
+      launch_rl_iterate(d.L.view(), d.dtgrid.p, p, d.kc, d.mesh, nsub, h, ig, tout.p, propagate ? 1 : 0,
+                        d.any_open ? 1 : 0, d.stream);
+    });
     if (to_file) launch_out_rate(tout.p, d.L.te.p, dt, d.N, avg.p, d.stream);   // (:93)
     if (d.multispecies_on) {                                                   // (:94-97)
       if (msf < 1.0) launch_ms_change(d.ms(1), tout.p, d.L.te.p, 1.0 - msf, true, d.N, d.stream);
@@ -1196,7 +1234,8 @@ struct RlModule : GpuModule {
     }
     if (inactive) return;
     d.L.te.swap(tout);   // the result buffer becomes the live thermal energy (no copy)
-    d.propagate_live();
+    if (propagate) d.finish_propagate();
+    else d.propagate_live();
   }
 };
 
@@ -1265,7 +1304,6 @@ struct ViscModule : GpuModule {
   }
   bool needs_pre_scalars() const override { return false; }
   bool iterates() const override { return any_hyper; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
 
   static int var_code(const std::string& n) {
@@ -1566,7 +1604,6 @@ struct HeatModule : GpuModule {
   }
   bool needs_pre_scalars() const override { return false; }
   bool iterates() const override { return false; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
   void iterate(Domain&, double) override {}
   // the heating grid depends on positions only: built once on the host with the C library's exp
@@ -1656,7 +1693,6 @@ struct PvModule : GpuModule {
             "Physical Viscosity MS electron heating fraction must be between 0 and 1");
   }
   bool needs_pre_scalars() const override { return false; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
   static PvSet view(DBuf* b) { return PvSet{b[0].p, b[1].p, b[2].p, b[3].p, b[4].p, b[5].p, b[6].p, b[7].p}; }
   // constructCoefficientGrid (:252-270), once on the host with the C library's exp
@@ -1832,7 +1868,6 @@ struct SourceRev {
 struct PostSourceModule : GpuModule {
   bool needs_pre_scalars() const override { return false; }
   bool iterates() const override { return false; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
   void iterate(Domain&, double) override {}
   // false when post() at `now` leaves the state alone (outside the module's time window)
@@ -2088,7 +2123,7 @@ struct FieldHeatModule : GpuModule {
   void file_output(OutList& o) override {                                  // :73-80
     if (to_file) o.emplace_back("field_heating", heat.p);
   }
-  void pre_launch(Domain& d, double*) override {  // preIterateModule -> computeHeating (:34-54)
+  void pre_launch(Domain& d) override {  // preIterateModule -> computeHeating (:34-54)
     d.timed("fheat", [&] { launch_fheat_pre(d.L.view(), d.stat(), d.bhx.p, d.bhy.p, p, d.mesh, heat.p, d.stream); });
   }
   void pre_finish(double, const double*) override {}
@@ -2110,7 +2145,6 @@ struct DivCleanModule : GpuModule {
     }
   }
   bool needs_pre_scalars() const override { return false; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
   // coeff = (1 / (1/dx^2 + 1/dy^2)) / 2 / time_scale, on the host (:22-26)
   void setup(Domain& d) override {
@@ -2260,7 +2294,6 @@ struct ResistModule : GpuModule {
   }
   ~ResistModule() override { if (changed) (void)hipFree(changed); }
   bool needs_pre_scalars() const override { return false; }
-  void pre_launch(Domain&, double*) override {}
   void pre_finish(double, const double*) override {}
 
   ArParams ar_params() const {

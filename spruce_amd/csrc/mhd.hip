@@ -378,15 +378,6 @@ __global__ void __launch_bounds__(256) k_mhd_derived(MhdSet S, MhdStatic st, Mhd
 
 inline dim3 grid2d(int nx, int ny, dim3 b) { return dim3((ny + b.x - 1) / b.x, (nx + b.y - 1) / b.y); }
 
-// n module scalars, the step size and the error flag into host-visible memory in one launch, so the
-// host reads everything a step's subcycle counts need after a single synchronisation
-__global__ void k_gather_scalars(const double* scal, int n, const double* step, const int* err, double* out) {
-  const int t = threadIdx.x;
-  if (t < n) out[t] = scal[t];
-  if (t == n) out[n] = *step;
-  if (t == n + 1) out[n + 1] = (double)*err;
-}
-
 }  // namespace
 
 void launch_mhd_stage(const StageArgs& a, hipStream_t s) {
@@ -436,11 +427,6 @@ void launch_moc_visc(MhdSet S, MhdStatic st, MhdConst k, Mesh mesh, double gv, d
   const dim3 g = grid2d(mesh.nx, mesh.ny, b);
   hipLaunchKernelGGL(k_moc_visc_part, g, b, 0, s, S, st, k, mesh, partial);
   hipLaunchKernelGGL(k_moc_visc_final, dim3(1), dim3(1024), 0, s, (const double*)partial, (int)(g.x * g.y), gv, vc, err);
-}
-
-void launch_gather_scalars(const double* scal, int n, const double* step, const int* err, double* host_out,
-                           hipStream_t s) {
-  hipLaunchKernelGGL(k_gather_scalars, dim3(1), dim3(((n + 2 + 63) / 64) * 64), 0, s, scal, n, step, err, host_out);
 }
 
 void launch_reduce_step(const double* partial, int n, double eps, double* step, double* history, int idx, int* err,

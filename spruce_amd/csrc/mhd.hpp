@@ -132,9 +132,6 @@ void launch_mhd_dt(MhdSet L, MhdStatic st, MhdConst k, Mesh mesh, double* dt_gri
 // when the minimum is not finite.  partial holds mhd_dt_blocks() values.
 void launch_moc_visc(MhdSet S, MhdStatic st, MhdConst k, Mesh mesh, double gv, double* partial, double* vc, int* err,
                      hipStream_t s);
-// out[0..n) = scal, out[n] = *step, out[n+1] = *err (out: host memory from hipHostMalloc)
-void launch_gather_scalars(const double* scal, int n, const double* step, const int* err, double* host_out,
-                           hipStream_t s);
 void launch_reduce_step(const double* partial, int n, double eps, double* step, double* history, int idx,
                         int* err, hipStream_t s);
 // with moc non-null the open_moc characteristic terms are added to the ghost cells (idealmhd.cpp:99-103)

@@ -51,14 +51,21 @@ __device__ __forceinline__ double block_reduce(double v, bool is_min) {
   return v;
 }
 
+__device__ __forceinline__ void bhat_at(const MhdSet& L, const MhdStatic& st, size_t c, double& hx, double& hy) {
+  const double bx = st.bex[c] + L.bx[c], by = st.bey[c] + L.by[c], bz = st.bez[c] + L.bz[c];
+  const double bm = sqrt(bx * bx + by * by + bz * bz);
+  hx = bm == 0.0 ? 0.0 : bx / bm;
+  hy = bm == 0.0 ? 0.0 : by / bm;
+}
+
 __global__ void __launch_bounds__(256) k_bhat(MhdSet L, MhdStatic st, Mesh M, double* bhx, double* bhy) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i >= M.nx || j >= M.ny) return;
   const size_t c = (size_t)i * M.ny + j;
-  const double bx = st.bex[c] + L.bx[c], by = st.bey[c] + L.by[c], bz = st.bez[c] + L.bz[c];
-  const double bm = sqrt(bx * bx + by * by + bz * bz);
-  bhx[c] = bm == 0.0 ? 0.0 : bx / bm;
-  bhy[c] = bm == 0.0 ? 0.0 : by / bm;
+  double hx, hy;
+  bhat_at(L, st, c, hx, hy);
+  bhx[c] = hx;
+  bhy[c] = hy;
 }
 
 __global__ void __launch_bounds__(256) k_bhat_derivs(const double* bhx, const double* bhy, Mesh M, double* dbxx,
@@ -121,54 +128,50 @@ __device__ __forceinline__ void grad_at(const Mesh& M, int i, int j, double Tc, 
   gy = qdiv(fint(M.y, jp, j, Tc, Typ) - fint(M.y, j, jm, Tym, Tc), M.y.d[j], M.y.rd[j]);
 }
 
-__global__ void __launch_bounds__(256) k_tc_pre(MhdSet L, const double* bhx, const double* bhy, TcParams p,
-                                                MhdConst K, Mesh M, double* pmin, double* pmax) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * blockDim.y + threadIdx.y;
-  double vmin = DBL_MAX, vmax = -DBL_MAX;
-  if (i < M.nx && j < M.ny && inside(M, i, j)) {
-    const size_t c = (size_t)i * M.ny + j;
-    auto T = [&](int a, int b) {
-      const size_t q = (size_t)wrp(a, M.nx, M.x.per) * M.ny + wrp(b, M.ny, M.y.per);
-      return temp_of(L.te[q], L.n[q], K);
-    };
-    const double Tc = T(i, j);
-    const double rho = L.rho[c];
-    double dts;
-    if (!p.saturation) {
-      // K_B/(w kappa_0) * (rho/m) * d_x * d_y / T^2.5 (thermalconduction.cpp:183)
-      dts = qdiv(rho, K.m, K.rm) * p.c1 * M.x.d[i] * M.y.d[j] / pow_2p5(Tc);
-    } else {
-      double gx, gy;
-      grad_at(M, i, j, Tc, T(i - 1, j), T(i + 1, j), T(i, j - 1), T(i, j + 1), gx, gy);
-      const double bx = bhx[c], by = bhy[c];
-      const double ftg = gx * bx + gy * by;
-      vmax = fabs(ftg);
-      const SatFlux s = sat_flux(Tc, gx, gy, rho, bx, by, M.x.d[i], M.y.d[j], p, K);
-      const double kap = fabs(s.sfm / ftg);                  // saturatedKappa (:236-248)
-      dts = K_B / kap * qdiv(rho, K.m, K.rm) * M.x.d[i] * M.y.d[j];
-    }
-    vmin = (dts < vmin) ? dts : vmin;
-  } else if (i < M.nx && j < M.ny) {
-    vmax = 0.0;  // |b_hat . grad T| is zero outside the interior
-  }
-  const double a = block_reduce(vmin, true);
-  const double b = block_reduce(vmax, false);
-  if (threadIdx.x == 0 && threadIdx.y == 0) {
-    const int blk = blockIdx.y * gridDim.x + blockIdx.x;
-    pmin[blk] = a;
-    pmax[blk] = b;
+// The conduction time scale at an interior cell and, with saturation, |b_hat . grad T|
+// (thermalconduction.cpp:179-193).
+__device__ __forceinline__ void tc_timescale(const MhdSet& L, double bx, double by, const TcParams& p, const MhdConst& K,
+                                             const Mesh& M, int i, int j, double& dts, double& ft) {
+  auto T = [&](int a, int b) {
+    const size_t q = (size_t)wrp(a, M.nx, M.x.per) * M.ny + wrp(b, M.ny, M.y.per);
+    return temp_of(L.te[q], L.n[q], K);
+  };
+  const double Tc = T(i, j);
+  const double rho = L.rho[(size_t)i * M.ny + j];
+  if (!p.saturation) {
+    // K_B/(w kappa_0) * (rho/m) * d_x * d_y / T^2.5 (thermalconduction.cpp:183)
+    dts = qdiv(rho, K.m, K.rm) * p.c1 * M.x.d[i] * M.y.d[j] / pow_2p5(Tc);
+  } else {
+    double gx, gy;
+    grad_at(M, i, j, Tc, T(i - 1, j), T(i + 1, j), T(i, j - 1), T(i, j + 1), gx, gy);
+    const double ftg = gx * bx + gy * by;
+    ft = fabs(ftg);
+    const SatFlux s = sat_flux(Tc, gx, gy, rho, bx, by, M.x.d[i], M.y.d[j], p, K);
+    const double kap = fabs(s.sfm / ftg);                  // saturatedKappa (:236-248)
+    dts = K_B / kap * qdiv(rho, K.m, K.rm) * M.x.d[i] * M.y.d[j];
   }
 }
 
-__global__ void __launch_bounds__(1024) k_finish_minmax(const double* pmin, const double* pmax, int n, double* out) {
-  double a = DBL_MAX, b = -DBL_MAX;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    a = (pmin[k] < a) ? pmin[k] : a;
-    b = (b < pmax[k]) ? pmax[k] : b;
+// Block k: module k's minimum and maximum over the blocks of k_step_pre, straight to the host's copy;
+// the first block also copies the step size and the error flag.
+__global__ void __launch_bounds__(1024) k_finish_scalars(const double* partial, int nblocks, int njobs, const double* step,
+                                                         const int* err, double* host_out) {
+  if ((int)blockIdx.x < njobs) {
+    const double* pmin = partial + (size_t)2 * nblocks * blockIdx.x;
+    const double* pmax = pmin + nblocks;
+    double a = DBL_MAX, b = -DBL_MAX;
+    for (int k = threadIdx.x; k < nblocks; k += blockDim.x) {
+      a = (pmin[k] < a) ? pmin[k] : a;
+      b = (b < pmax[k]) ? pmax[k] : b;
+    }
+    a = block_reduce(a, true);
+    b = block_reduce(b, false);
+    if (threadIdx.x == 0) { host_out[2 * blockIdx.x] = a; host_out[2 * blockIdx.x + 1] = b; }
   }
-  a = block_reduce(a, true);
-  b = block_reduce(b, false);
-  if (threadIdx.x == 0) { out[0] = a; out[1] = b; }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    host_out[2 * njobs] = *step;
+    host_out[2 * njobs + 1] = (double)*err;
+  }
 }
 
 __global__ void __launch_bounds__(256) k_tc_sat(const double* te, const double* n, const double* rho, const double* bhx,
@@ -444,38 +447,78 @@ __device__ __forceinline__ double rl_loss(double t, double n, double te_live, do
   return v;
 }
 
-__global__ void __launch_bounds__(256) k_rl_pre(MhdSet L, const double* dtg, RlParams p, MhdConst K, Mesh M,
-                                                double* pmin, double* pmax) {
+// What the modules need before their subcycles, one pass over the live grids: b_hat, and per block the
+// least and greatest values of the conduction and the radiation reductions.  Launch-bound on small grids:
+// as one kernel for each and one more to finish each reduction they were six launches of 1 to 4.5 us with
+// 4 us between two, 48 us of the 137 us a step of a 133x197 arcade took.
+__global__ void __launch_bounds__(256) k_step_pre(StepPreArgs a) {
+  const Mesh& M = a.mesh;
   const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * blockDim.y + threadIdx.y;
-  double vmin = DBL_MAX, vmax = -DBL_MAX;
+  double tmin = DBL_MAX, tmax = -DBL_MAX, rmin = DBL_MAX, rmax = -DBL_MAX;
   if (i < M.nx && j < M.ny) {
-    if (inside(M, i, j)) {
-      const size_t c = (size_t)i * M.ny + j;
-      const double te = L.te[c], n = L.n[c];
-      const double l = rl_loss(temp_of(te, n, K), n, te, p.prevent ? dtg[c] : 0.0, p);
-      vmax = l;
-      const double r = fabs(te / l);
-      vmin = (r < vmin) ? r : vmin;
+    const size_t c = (size_t)i * M.ny + j;
+    double hx = 0.0, hy = 0.0;
+    if (a.bhx) {
+      bhat_at(a.L, a.st, c, hx, hy);
+      a.bhx[c] = hx;
+      a.bhy[c] = hy;
+    }
+    if (!inside(M, i, j)) {
+      tmax = 0.0;   // |b_hat . grad T| and the losses are zero outside the interior
+      rmax = 0.0;
     } else {
-      vmax = 0.0;
+      if (a.tc_partial) {
+        double dts;
+        tc_timescale(a.L, hx, hy, a.tc, a.k, M, i, j, dts, tmax);
+        tmin = (dts < tmin) ? dts : tmin;
+      }
+      if (a.rl_partial) {
+        const double te = a.L.te[c], n = a.L.n[c];
+        const double l = rl_loss(temp_of(te, n, a.k), n, te, a.rl.prevent ? a.dt_grid[c] : 0.0, a.rl);
+        rmax = l;
+        const double r = fabs(te / l);
+        rmin = (r < rmin) ? r : rmin;
+      }
     }
   }
-  const double a = block_reduce(vmin, true);
-  const double b = block_reduce(vmax, false);
-  if (threadIdx.x == 0 && threadIdx.y == 0) {
-    const int blk = blockIdx.y * gridDim.x + blockIdx.x;
-    pmin[blk] = a;
-    pmax[blk] = b;
+  const int blk = blockIdx.y * gridDim.x + blockIdx.x, nblk = gridDim.x * gridDim.y;
+  const bool first = threadIdx.x == 0 && threadIdx.y == 0;
+  if (a.tc_partial) {
+    const double lo = block_reduce(tmin, true), hi = block_reduce(tmax, false);
+    if (first) { a.tc_partial[blk] = lo; a.tc_partial[nblk + blk] = hi; }
+  }
+  if (a.rl_partial) {
+    const double lo = block_reduce(rmin, true), hi = block_reduce(rmax, false);
+    if (first) { a.rl_partial[blk] = lo; a.rl_partial[nblk + blk] = hi; }
   }
 }
 
+// enforceMinimums then recomputeDerivedVarsFromEvolvedVars at one cell (idealmhd.cpp:234-252)
+__device__ __forceinline__ void propagate_cell(const MhdSet& L, const MhdConst& K, size_t c, double te, double* te_out,
+                                               int write_pre) {
+  const double rho1 = smax(qdiv(L.rho[c], K.m, K.rm), K.nmin) * K.m;
+  const double te1 = smax(te, K.temin);
+  const double n = smax(qdiv(rho1, K.m, K.rm), K.nmin);
+  if (write_pre) L.rho_pre[c] = rho1;
+  L.n[c] = n;
+  L.rho[c] = n * K.m;
+  te_out[c] = smax(te1, K.temin);
+}
+
+// propagate: te_out is the live thermal energy from here on and the cell is propagated too, which as a pass
+// of its own costs a small grid 3 us and a launch's gap of 4.
 __global__ void __launch_bounds__(256) k_rl_iterate(MhdSet L, const double* dtg, RlParams p, MhdConst K, Mesh M,
-                                                    int nsub, double h, int integ, double* te_out) {
+                                                    int nsub, double h, int integ, double* te_out, int propagate,
+                                                    int write_pre) {
   const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * blockDim.y + threadIdx.y;
   if (i >= M.nx || j >= M.ny) return;
   const size_t c = (size_t)i * M.ny + j;
   const double te_live = L.te[c];
-  if (!inside(M, i, j)) { te_out[c] = te_live; return; }
+  if (!inside(M, i, j)) {
+    if (propagate) propagate_cell(L, K, c, te_live, te_out, write_pre);
+    else te_out[c] = te_live;
+    return;
+  }
   const double n = L.n[c];
   const double dtl = p.prevent ? dtg[c] : 0.0;
   auto loss = [&](double te) { return rl_loss(temp_of(te, n, K), n, te_live, dtl, p); };
@@ -498,20 +541,13 @@ __global__ void __launch_bounds__(256) k_rl_iterate(MhdSet L, const double* dtg,
       te = smax(te + qdiv(hh * (k1 + 2.0 * k2 + 2.0 * k3 + k4), 6.0, K.r6), K.temin);
     }
   }
-  te_out[c] = te;
+  if (propagate) propagate_cell(L, K, c, te, te_out, write_pre);
+  else te_out[c] = te;
 }
 
 __global__ void __launch_bounds__(256) k_propagate_live(MhdSet L, MhdConst K, size_t N, int write_pre) {
   const size_t c = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= N) return;
-  // enforceMinimums then recomputeDerivedVarsFromEvolvedVars (idealmhd.cpp:234-252)
-  const double rho1 = smax(qdiv(L.rho[c], K.m, K.rm), K.nmin) * K.m;
-  const double te1 = smax(L.te[c], K.temin);
-  const double n = smax(qdiv(rho1, K.m, K.rm), K.nmin);
-  if (write_pre) L.rho_pre[c] = rho1;
-  L.n[c] = n;
-  L.rho[c] = n * K.m;
-  L.te[c] = smax(te1, K.temin);
+  if (c < N) propagate_cell(L, K, c, L.te[c], L.te, write_pre);
 }
 
 inline dim3 g2(const Mesh& m, dim3 b) { return dim3((m.ny + b.x - 1) / b.x, (m.nx + b.y - 1) / b.y); }
@@ -532,11 +568,14 @@ void launch_bhat_derivs(const double* bhx, const double* bhy, Mesh mesh, double*
   hipLaunchKernelGGL(k_bhat_derivs, g2(mesh, dim3(64, 4)), dim3(64, 4), 0, s, bhx, bhy, mesh, dbxx, dbxy, dbyx, dbyy);
 }
 
-void launch_tc_pre(MhdSet L, const double* bhx, const double* bhy, TcParams p, MhdConst k, Mesh mesh, double* partial,
-                   int nblocks, double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_tc_pre, g2(mesh, dim3(64, 4)), dim3(64, 4), 0, s, L, bhx, bhy, p, k, mesh, partial,
-                     partial + nblocks);
-  hipLaunchKernelGGL(k_finish_minmax, dim3(1), dim3(1024), 0, s, partial, partial + nblocks, nblocks, out);
+void launch_step_pre(const StepPreArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL(k_step_pre, g2(a.mesh, dim3(64, 4)), dim3(64, 4), 0, s, a);
+}
+
+void launch_finish_scalars(const double* partial, int nblocks, int njobs, const double* step, const int* err,
+                           double* host_out, hipStream_t s) {
+  hipLaunchKernelGGL(k_finish_scalars, dim3(njobs > 0 ? njobs : 1), dim3(1024), 0, s, partial, nblocks, njobs, step, err,
+                     host_out);
 }
 
 void launch_tc_sat(const double* te_src, const double* n, const double* rho, const double* bhx, const double* bhy,
@@ -586,17 +625,10 @@ void launch_tc_step(const TcStepArgs& a, hipStream_t s) {
   }
 }
 
-void launch_rl_pre(MhdSet L, const double* dt_grid, RlParams p, MhdConst k, Mesh mesh, double* partial, int nblocks,
-                   double* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_rl_pre, g2(mesh, dim3(64, 4)), dim3(64, 4), 0, s, L, dt_grid, p, k, mesh, partial,
-                     partial + nblocks);
-  hipLaunchKernelGGL(k_finish_minmax, dim3(1), dim3(1024), 0, s, partial, partial + nblocks, nblocks, out);
-}
-
 void launch_rl_iterate(MhdSet L, const double* dt_grid, RlParams p, MhdConst k, Mesh mesh, int nsub, double h,
-                       int integrator, double* te_out, hipStream_t s) {
+                       int integrator, double* te_out, int propagate, int write_pre, hipStream_t s) {
   hipLaunchKernelGGL(k_rl_iterate, g2(mesh, dim3(64, 4)), dim3(64, 4), 0, s, L, dt_grid, p, k, mesh, nsub, h,
-                     integrator, te_out);
+                     integrator, te_out, propagate, write_pre);
 }
 
 void launch_propagate_live(MhdSet L, MhdConst k, int nx, int ny, int write_pre, hipStream_t s) {

@@ -65,10 +65,28 @@ void launch_bhat(MhdSet L, MhdStatic st, Mesh mesh, double* bhx, double* bhy, hi
 // subcycles of a step all use the same values (thermalconduction.cpp:158-176).
 void launch_bhat_derivs(const double* bhx, const double* bhy, Mesh mesh, double* dbxx, double* dbxy, double* dbyx,
                         double* dbyy, hipStream_t s);
-// TC subcycle count inputs: min over the interior of the conduction time scale and, with saturation,
-// max |b_hat . grad T| (thermalconduction.cpp:179-193).  Writes out[0] = min, out[1] = max.
-void launch_tc_pre(MhdSet L, const double* bhx, const double* bhy, TcParams p, MhdConst k, Mesh mesh,
-                   double* partial, int nblocks, double* out, hipStream_t s);
+// One pass over the live grids before the modules' subcycles.  bhx, bhy: b_hat (null: not needed; the
+// conduction's reduction with saturation needs it).  tc_partial, rl_partial (null: not needed): per block the
+// minimum, then per block the maximum, of the conduction time scale and, with saturation, |b_hat . grad T|
+// (thermalconduction.cpp:179-193); of |te / losses| and the losses (radiativelosses.cpp:200-205).
+struct StepPreArgs {
+  MhdSet L;
+  MhdStatic st;
+  MhdConst k;
+  Mesh mesh;
+  double* bhx;
+  double* bhy;
+  TcParams tc;
+  double* tc_partial;
+  RlParams rl;
+  const double* dt_grid;   // radiation with prevent: the live step sizes
+  double* rl_partial;
+};
+void launch_step_pre(const StepPreArgs& a, hipStream_t s);
+// host_out[2 k], [2 k + 1]: minimum and maximum over the partials of job k (2 nblocks values each);
+// host_out[2 njobs], [2 njobs + 1]: the step size and the error flag.
+void launch_finish_scalars(const double* partial, int nblocks, int njobs, const double* step, const int* err,
+                           double* host_out, hipStream_t s);
 void launch_tc_sat(const double* te_src, const double* n, const double* rho, const double* bhx, const double* bhy,
                    TcParams p, MhdConst k, Mesh mesh, double* rx, double* ry, double* coef, hipStream_t s);
 // One conduction update: the wavefront-strip form with a.rows rows per strip, or one thread per cell
@@ -76,12 +94,10 @@ void launch_tc_sat(const double* te_src, const double* n, const double* rho, con
 void launch_tc_step(const TcStepArgs& a, hipStream_t s);
 // rows per strip of the strip form, chosen from the grid size
 int tc_strip_rows_default(int nx, int ny, bool saturation);
-// RL subcycle count inputs: out[0] = max losses, out[1] = min |te / losses| (radiativelosses.cpp:200-205).
-void launch_rl_pre(MhdSet L, const double* dt_grid, RlParams p, MhdConst k, Mesh mesh, double* partial, int nblocks,
-                   double* out, hipStream_t s);
-// All RL subcycles of one step in one launch (the losses are pointwise): integrator 0/1/2.
+// All RL subcycles of one step in one launch (the losses are pointwise): integrator 0/1/2.  propagate: also
+// propagateChanges up to the ghost fill, for a caller that makes te_out the live thermal energy.
 void launch_rl_iterate(MhdSet L, const double* dt_grid, RlParams p, MhdConst k, Mesh mesh, int nsub, double h,
-                       int integrator, double* te_out, hipStream_t s);
+                       int integrator, double* te_out, int propagate, int write_pre, hipStream_t s);
 // propagateChanges on the live grids up to the ghost fill: minimums then derived (pointwise).
 void launch_propagate_live(MhdSet L, MhdConst k, int nx, int ny, int write_pre, hipStream_t s);
 int solar_blocks(const Mesh& m);
