@@ -193,7 +193,8 @@ class Domain : public DomainBase {
   DBuf kbuf[3];
   DBuf partial, step, history, scratch;
   int* err_flag = nullptr;
-  double* hscal = nullptr;   // pinned host copy of the module scalars, step size and error flag
+  double* hscal = nullptr;   // pinned host copy of the module scalars, step size, error flag and tickets
+  uint64_t ticket = 0;       // of the latest copy
   int dt_blocks = 0;
   int kinds_all[4] = {0, 0, 0, 0}, kinds_ucnp[4] = {0, 0, 0, 0}, kinds_live[4] = {0, 0, 0, 0};
   double s1[4] = {1, 1, 1, 1}, s2[4] = {1, 1, 1, 1};
@@ -500,7 +501,8 @@ class Domain : public DomainBase {
       bhx.alloc(N);
       bhy.alloc(N);
       mod_partial.alloc(2 * (size_t)solar_blocks(mesh) * mods.size());
-      hip_check(hipHostMalloc((void**)&hscal, (2 * mods.size() + 2) * sizeof(double)), "hipHostMalloc");
+      hip_check(hipHostMalloc((void**)&hscal, (3 * mods.size() + 3) * sizeof(double)), "hipHostMalloc");
+      std::memset(hscal, 0, (3 * mods.size() + 3) * sizeof(double));
       for (auto& m : mods) {
         m->setup(*this);
         need_dt_grid = need_dt_grid || m->needs_dt_grid();
@@ -564,6 +566,19 @@ class Domain : public DomainBase {
     moc_limit(L.view());
   }
 
+  // Waits until launch_finish_scalars has stored its tickets, or the stream has ended without.
+  void await_scalars(int njobs) {
+    const uint64_t* t = reinterpret_cast<const uint64_t*>(hscal) + 2 * njobs + 2;
+    for (int k = 0; k < std::max(njobs, 1); ++k)
+      for (unsigned n = 1; __atomic_load_n(t + k, __ATOMIC_ACQUIRE) != ticket; ++n) {
+        if (n % 8192) continue;
+        const hipError_t e = hipStreamQuery(stream);
+        if (e == hipErrorNotReady) continue;
+        hip_check(e, "hipStreamQuery");
+        require(__atomic_load_n(t + k, __ATOMIC_ACQUIRE) == ticket, SPRUCE_E_HIP, "the step's scalars did not arrive");
+      }
+  }
+
   // ModuleHandler pre/iterate loops (modulehandler.cpp:34-50; evolution.cpp:65-66).
   void run_modules(int s) {
     bool bh = false;
@@ -597,8 +612,8 @@ class Domain : public DomainBase {
     for (auto& m : mods) m->pre_launch(*this);
     double dt = std::nan("");
     if (host) {
-      launch_finish_scalars(mod_partial.p, nblocks, njobs, step.p, err_flag, hscal, stream);
-      hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+      launch_finish_scalars(mod_partial.p, nblocks, njobs, step.p, err_flag, hscal, ++ticket, stream);
+      await_scalars(njobs);
       if (hscal[2 * njobs + 1] != 0.0) {
         hip_check(hipMemset(err_flag, 0, sizeof(int)), "hipMemset");
         throw Error(SPRUCE_E_NUMERIC, "Something went wrong in the min calculation (no finite dt)");

@@ -153,9 +153,11 @@ __device__ __forceinline__ void tc_timescale(const MhdSet& L, double bx, double 
 }
 
 // Block k: module k's minimum and maximum over the blocks of k_step_pre, straight to the host's copy;
-// the first block also copies the step size and the error flag.
+// the first block also copies the step size and the error flag.  Each block then stores the ticket in its
+// place behind them, which the host polls: it has the values when it sees the store, where a stream
+// synchronisation also waits for the launch to retire and for a marker behind it.
 __global__ void __launch_bounds__(1024) k_finish_scalars(const double* partial, int nblocks, int njobs, const double* step,
-                                                         const int* err, double* host_out) {
+                                                         const int* err, double* host_out, uint64_t ticket) {
   if ((int)blockIdx.x < njobs) {
     const double* pmin = partial + (size_t)2 * nblocks * blockIdx.x;
     const double* pmax = pmin + nblocks;
@@ -172,6 +174,9 @@ __global__ void __launch_bounds__(1024) k_finish_scalars(const double* partial, 
     host_out[2 * njobs] = *step;
     host_out[2 * njobs + 1] = (double)*err;
   }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(host_out) + 2 * njobs + 2 + blockIdx.x, ticket, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __global__ void __launch_bounds__(256) k_tc_sat(const double* te, const double* n, const double* rho, const double* bhx,
@@ -573,9 +578,9 @@ void launch_step_pre(const StepPreArgs& a, hipStream_t s) {
 }
 
 void launch_finish_scalars(const double* partial, int nblocks, int njobs, const double* step, const int* err,
-                           double* host_out, hipStream_t s) {
+                           double* host_out, uint64_t ticket, hipStream_t s) {
   hipLaunchKernelGGL(k_finish_scalars, dim3(njobs > 0 ? njobs : 1), dim3(1024), 0, s, partial, nblocks, njobs, step, err,
-                     host_out);
+                     host_out, ticket);
 }
 
 void launch_tc_sat(const double* te_src, const double* n, const double* rho, const double* bhx, const double* bhy,

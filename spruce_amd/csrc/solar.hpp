@@ -84,9 +84,10 @@ struct StepPreArgs {
 };
 void launch_step_pre(const StepPreArgs& a, hipStream_t s);
 // host_out[2 k], [2 k + 1]: minimum and maximum over the partials of job k (2 nblocks values each);
-// host_out[2 njobs], [2 njobs + 1]: the step size and the error flag.
+// host_out[2 njobs], [2 njobs + 1]: the step size and the error flag; then max(njobs, 1) words that receive
+// `ticket` after the values.
 void launch_finish_scalars(const double* partial, int nblocks, int njobs, const double* step, const int* err,
-                           double* host_out, hipStream_t s);
+                           double* host_out, uint64_t ticket, hipStream_t s);
 void launch_tc_sat(const double* te_src, const double* n, const double* rho, const double* bhx, const double* bhy,
                    TcParams p, MhdConst k, Mesh mesh, double* rx, double* ry, double* coef, hipStream_t s);
 // One conduction update: the wavefront-strip form with a.rows rows per strip, or one thread per cell
