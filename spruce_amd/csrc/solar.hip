@@ -284,8 +284,8 @@ __global__ void __launch_bounds__(256) k_tc_step(TcStepArgs a) {
 // each of ~20 divisions and both powers share one square root, so a row is about 250 VALU
 // instructions in one run instead of 400 in twenty pieces (1.78e7 against 2.79e7 a launch), and the
 // row's geometry comes through the scalar cache, so that nothing waits for the row being fetched but
-// its use.  Measured per subcycle: 2048x2048 79.5 -> 51.8 us, 512x1024 17.5 (one thread per cell) ->
-// 12.3 us, 133x197 7.7 -> 7.2 us.  160 VGPRs, three wavefronts per SIMD: at four (128) the two register
+// its use.  Measured per subcycle: 2048x2048 79.5 -> 47 to 52 us, 512x1024 17.5 (one thread per cell) ->
+// 11 to 12.3 us, 133x197 7.7 -> 5.0 us.  160 VGPRs, three wavefronts per SIMD: at four (128) the two register
 // sets of a pair of rows spill.
 //
 // With flux saturation the march also forms the saturated flux and coefficient of each row, from the
@@ -455,7 +455,8 @@ __device__ __forceinline__ double rl_loss(double t, double n, double te_live, do
 // What the modules need before their subcycles, one pass over the live grids: b_hat, and per block the
 // least and greatest values of the conduction and the radiation reductions.  Launch-bound on small grids:
 // as one kernel for each and one more to finish each reduction they were six launches of 1 to 4.5 us with
-// 4 us between two, 48 us of the 137 us a step of a 133x197 arcade took.
+// 4 us between two, 48 us of the 137 us a step of a 133x197 arcade took; this pass and k_finish_scalars
+// take 7 and 5.5 us there.
 __global__ void __launch_bounds__(256) k_step_pre(StepPreArgs a) {
   const Mesh& M = a.mesh;
   const int j = blockIdx.x * blockDim.x + threadIdx.x, i = blockIdx.y * blockDim.y + threadIdx.y;
