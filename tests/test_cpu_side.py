@@ -23,6 +23,13 @@ def test_library_exports_every_declared_symbol():
     assert not missing, missing
 
 
+def test_every_source_is_compiled():
+    """A source that nothing compiles is dead, and one that repeats another's symbols waits to be linked."""
+    from spruce_amd.build import CSRC, SOURCES
+    found = sorted(f for f in os.listdir(CSRC) if f.endswith((".hip", ".cpp")))
+    assert found == sorted(SOURCES + ["run_main.cpp"])
+
+
 def test_reciprocal_corrected_division_is_exact():
     with tempfile.TemporaryDirectory() as tmp:
         exe = os.path.join(tmp, "arith_check")
