@@ -197,14 +197,15 @@ struct DtState {
   bool cell = false;           // this lane's cell takes part
   bool pending = false;
   double worst = 0.0;
-  __device__ __forceinline__ void finish(double b2, const MhdConst& K, double dy, double rdy) {
+  // in_range: the mesh and gamma are (StageArgs)
+  __device__ __forceinline__ void finish(bool in_range, double b2, const MhdConst& K, double dy, double rdy) {
     RangeTest t;
     t.density(rho);
     t.add(te);
     t.add(mx);
     t.add(my);
     t.add(b2);
-    const bool out = t.out() || !(te > 0.0);
+    const bool out = t.out() || !(te > 0.0) || !in_range;
     double s;
     if (__any(cell && out)) s = dt_inverse<false>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
     else s = dt_inverse<true>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
@@ -400,7 +401,7 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
       f[F_ZIN][lane] = qdiv_t<IN>(cz0 * biy - cz1 * bix, 4.0 * PI, K.r4pi);
     }
     block_barrier();
-    if (DT && ROLE == FLUID && dt.pending) dt.finish(sh.b2[slot ^ 1][lane], K, gy.d, gy.rd);
+    if (DT && ROLE == FLUID && dt.pending) dt.finish(a.in_range, sh.b2[slot ^ 1][lane], K, gy.d, gy.rd);
     if (IN && tested_out(slot)) return false;
     if (!DT && !col.out) return true;
     double o_rho = 1.0, o_te = 1.0, o_mx = 0.0, o_my = 0.0, o_b2 = 0.0;   // what the step size reads
@@ -519,7 +520,7 @@ __device__ __forceinline__ void strip_rows(const StageArgs& a, const Column& col
     block_barrier();
     if constexpr (ROLE == FLUID) {
       const double2 d = sh.geom[5][threadIdx.x];
-      if (dt.pending) dt.finish(sh.b2[(rend - 1) & 1][threadIdx.x], a.k, d.x, d.y);
+      if (dt.pending) dt.finish(a.in_range, sh.b2[(rend - 1) & 1][threadIdx.x], a.k, d.x, d.y);
       double m = dt.worst;
       for (int off = 32; off > 0; off >>= 1) {
         const double o = __shfl_xor(m, off, 64);

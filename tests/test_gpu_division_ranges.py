@@ -84,6 +84,19 @@ def test_mesh_out_of_range():
     check(st, cfg, {"stage_kernel": "strip", "strip_rows": 4})
 
 
+@pytest.mark.parametrize("d", [1e-302, 1e300])
+def test_step_size_on_a_mesh_out_of_range(d):
+    """A state at rest: the speed over the cell size overflows (a step size of 0), or is almost 0."""
+    st, cfg = wave(14, 70, "rk2", PERIODIC)
+    for k in ("d_x", "d_y", "pos_x", "pos_y"):
+        st.grids[k] = st.grids[k] * (d / 1e7)
+    for k in ("rho", "temp"):
+        st.grids[k][:] = st.grids[k].mean()
+    for k in ("mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z"):
+        st.grids[k][:] = 0.0
+    check(st, cfg, {"stage_kernel": "strip", "strip_rows": 4})
+
+
 @pytest.mark.parametrize("sat,integ", [(False, "euler"), (True, "rk2"), (False, "rk4")])
 @pytest.mark.parametrize("what", ["bhat", "mesh"])
 def test_conduction_out_of_range(sat, integ, what):
