@@ -170,9 +170,9 @@ int spruce_gpu_device_grid(spruce_gpu_domain* d, const char* name, double** dev_
  *   "multispecies_mode" = "true" | "false" (the config setting of that name, fileio.cpp:322):
  *                    accumulate the cumulative heating grids (before setup);
  *   "block"        = ideal_2F launch shape: "<columns>x<rows>" thread block of every kernel, stage
- *                    one thread per cell, or "strip<rows>" (rows a multiple of 4 up to 64): the
- *                    stage kernel in strips, the other kernels in 64x4 (default: strips whose rows
- *                    follow from the domains' sizes). */
+ *                    one thread per cell, "strip<rows>" (rows a multiple of 4 up to 64): the stage
+ *                    kernel in strips, the other kernels in 64x4, or "auto" (default): strips whose
+ *                    rows follow from the domains' sizes. */
 int spruce_gpu_set_option(spruce_gpu_domain* d, const char* key, const char* value);
 
 /* Average duration (ms) of each kernel of the most recent spruce_gpu_step call, measured with HIP
@@ -240,8 +240,8 @@ spruce_gpu_batch* spruce_gpu_batch_create(spruce_gpu_domain* const* domains, int
  * replaced by strips of 4 rows) | "false" (default). */
 int spruce_gpu_batch_set_option(spruce_gpu_batch* b, const char* key, const char* value);
 /* Times trial_steps steps for each candidate block shape, keeps the fastest and restores the state
- * of every member, so tuning does not advance the simulation.  chosen receives "<cols>x<rows>" or
- * "strip<rows>x60". */
+ * of every member, so tuning does not advance the simulation.  The default, "auto", is a candidate.
+ * chosen receives "<cols>x<rows>", "strip<rows>x60" or "auto<rows>x60"; "block" takes each of them. */
 int spruce_gpu_batch_autotune(spruce_gpu_batch* b, int32_t trial_steps, char* chosen, int32_t chosen_len,
                               double* ms_per_step);
 /* nsteps steps of every member; dt_out (may be NULL) receives n*nsteps step sizes, member-major. */

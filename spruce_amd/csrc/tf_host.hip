@@ -68,6 +68,13 @@ void TfDomain::set_grid(const std::string& name, const double* p, int64_t count)
 
 TfShape parse_tf_shape(const std::string& v) {
   TfShape sh;
+  if (v.rfind("auto", 0) == 0) {   // "auto", or the name of an automatic shape: "auto<rows>x60"
+    const std::string rows = v.substr(4, v.size() > 7 ? v.size() - 7 : 0);
+    require(v == "auto" || (v.size() > 7 && v.substr(v.size() - 3) == "x60" &&
+                            rows.find_first_not_of("0123456789") == std::string::npos),
+            SPRUCE_E_ARG, "block must be <columns>x<rows>, strip<rows> or auto");
+    return sh;
+  }
   sh.automatic = false;
   if (v.rfind("strip", 0) == 0) {
     const int r = std::stoi(v.substr(5));
@@ -480,8 +487,8 @@ void TfBatchRun::check_history() {
   }
 }
 
-// Times each candidate block shape on a copy of the batch state and keeps the fastest; the state
-// is restored afterwards, so tuning does not advance the simulation.
+// Times each candidate shape, the automatic strips among them, on a copy of the batch state and keeps the
+// fastest; the state is restored afterwards, so tuning does not advance the simulation.
 double TfBatchRun::autotune(int trial_steps, std::string* chosen) {
   hipStream_t s = members[0]->stream;
   struct Save { std::vector<DBuf*> src; std::vector<std::unique_ptr<DBuf>> copy; double t; int it; };
@@ -499,7 +506,7 @@ double TfBatchRun::autotune(int trial_steps, std::string* chosen) {
     saves[k].t = d->time;
     saves[k].it = d->iter;
   }
-  std::vector<TfShape> shapes;
+  std::vector<TfShape> shapes(1);   // the automatic strips, the default
   for (auto& bxy : std::vector<std::pair<int, int>>{{64, 1}, {64, 2}, {64, 4}, {128, 1}, {128, 2}, {32, 2}, {32, 4},
                                                     {32, 8}, {16, 4}, {16, 8}}) {
     TfShape t;
@@ -548,8 +555,8 @@ double TfBatchRun::autotune(int trial_steps, std::string* chosen) {
   (void)hipEventDestroy(e1);
   for (size_t k = 0; k < members.size(); ++k) { members[k]->time = saves[k].t; members[k]->iter = saves[k].it; }
   rebuild(bestsh);
-  for (auto* d : members) d->shape = bestsh;
-  if (chosen) *chosen = bestsh.str();
+  for (auto* d : members) d->shape = bestsh;   // automatic: each member's own rows when it steps alone
+  if (chosen) *chosen = shape.str();
   return best / trial_steps;
 }
 

@@ -18,12 +18,14 @@ class TfBatchRun;
 struct TfShape {
   int bx = 64, by = 4, R = 0;
   bool automatic = true;
-  // "<columns>x<rows>", or "strip<rows>x60" (rows by output columns)
+  // "<columns>x<rows>", or "strip<rows>x60", "auto<rows>x60" (rows by output columns)
   std::string str() const {
+    if (automatic) return "auto" + std::to_string(R) + "x60";
     return R > 0 ? "strip" + std::to_string(R) + "x60" : std::to_string(bx) + "x" + std::to_string(by);
   }
 };
-// "<columns>x<rows>" (64, 128, 192 or 256 threads) or "strip<rows>", "strip<rows>x60" (rows a multiple of 4, 4..64)
+// "<columns>x<rows>" (64, 128, 192 or 256 threads), "strip<rows>", "strip<rows>x60" (rows a multiple of 4, 4..64),
+// or "auto", "auto<rows>x60" (the default: rows from the members' sizes, whatever the name says)
 TfShape parse_tf_shape(const std::string& v);
 
 class TfDomain : public DomainBase {

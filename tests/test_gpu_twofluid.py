@@ -168,6 +168,31 @@ def test_autotune_keeps_state_and_results():
             d.close()
 
 
+def test_autotune_times_the_automatic_strips_and_names_a_block():
+    """The strips whose height follows from the members' sizes are a candidate (a small domain's 1-row strips
+    step in two thirds of the time of 4-row strips, the lowest of the other candidates), and what is chosen can
+    be set again; "auto" returns to them."""
+    specs = _members("rk2", False, sizes=[(64, 64)])
+    alone, dts_a = _run_alone(specs, [3])
+    for block in ("64x4", None):
+        doms = [GpuDomain(s) for s in specs]
+        b = GpuBatch(doms, graph=True, block=block)
+        try:
+            shape, ms = b.autotune(50)
+            print("autotune from", block, "chose", shape, ms, flush=True)
+            assert shape == "auto1x60"
+            for value in (shape, "strip8x60", "auto"):
+                b.set_option("block", value)
+            for value in ("strip7", "strip7x60", "auto7", "autox60", "automatic", "auto1x61"):
+                with pytest.raises(Exception):
+                    b.set_option("block", value)
+            _check_same(doms, alone, b.step(3), dts_a, "after autotune")
+        finally:
+            b.close()
+            for d in doms:
+                d.close()
+
+
 def test_domain_in_batch_cannot_step_alone_and_recovers():
     specs = _members("rk2", False, sizes=[(64, 64), (48, 80)])
     doms = [GpuDomain(s) for s in specs]
