@@ -9,6 +9,7 @@
 
 #include "arith.hpp"
 #include "tf_host.hpp"
+#include "tf_rows.hpp"
 
 namespace spruce {
 
@@ -314,13 +315,16 @@ void TfBatchRun::destroy_graph() {
 
 void TfBatchRun::rebuild(TfShape sh) {
   destroy_graph();
+  b.any_curl = 0;
+  for (auto* d : members)
+    if (d->dom.c.curl) b.any_curl = 1;
   if (sh.automatic) {
     std::vector<int> rows, tiles;
     for (auto* d : members) {
       rows.push_back(d->nx);
       tiles.push_back((d->ny + 59) / 60);
     }
-    sh.R = tf_strip_rows_default(rows.data(), tiles.data(), (int)rows.size());
+    sh.R = tf_strip_rows_default(rows.data(), tiles.data(), (int)rows.size(), b.any_curl != 0);
   }
   shape = sh;
   const int bx = sh.bx, by = sh.by;
@@ -373,13 +377,10 @@ void TfBatchRun::rebuild(TfShape sh) {
   b.strip_dom = d_strip_dom;
   b.nstrip_tiles = sbase;
   b.strip_rows = sh.R;
-  b.any_curl = 0;
   b.stopping_sides = 0;
-  for (auto* d : members) {
-    if (d->dom.c.curl) b.any_curl = 1;
+  for (auto* d : members)
     for (int k = 0; k < 4; ++k)
       if (d->desc.bc[k] == SPRUCE_BC_FIXED || d->desc.bc[k] == SPRUCE_BC_REFLECT) b.stopping_sides = 1;
-  }
 }
 
 // One PlasmaDomain::advanceTime of every domain (evolution.cpp:59-124); no host interaction, so a

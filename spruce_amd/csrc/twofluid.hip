@@ -1453,20 +1453,6 @@ k_tf_persistent(TfBatch b, int nsteps, int integrator, int ucnp_mask, int final_
 }
 }  // namespace
 
-int tf_strip_rows_default(const int* rows, const int* tiles, int n) {
-  // 1024 blocks (2 wavefronts per SIMD; half as many again without curl terms) run at once and a strip
-  // costs its rows plus about three: the height with the least rounds x cost, the taller of equals
-  int best = 1;
-  long least = 0;
-  for (int R = 1; R <= 64; ++R) {
-    long blocks = 0;
-    for (int k = 0; k < n; ++k) blocks += (long)tiles[k] * ((rows[k] + R - 1) / R);
-    const long cost = (blocks + 1535) / 1536 * (R + 3);
-    if (R == 1 || cost <= least) { best = R; least = cost; }
-  }
-  return best;
-}
-
 void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, bool dt, hipStream_t s) {
   const int want_dt = dt ? 1 : 0;
   if (b.strip_rows > 0 && b.any_curl)

@@ -71,8 +71,6 @@ enum TfSetSel { TF_SEL_L = 0, TF_SEL_W = 1, TF_SEL_W2 = 2 };
 // T = minimums(B + mult*step * k(S)) for every domain of the batch.  dt (strips only): the stage also
 // writes one minimum of T's per-cell step size per strip, as it is after a ghost fill.
 void launch_tf_stage(const TfBatch& b, int S, int B, int T, double mult, int mode, int kslot, bool dt, hipStream_t s);
-// rows per strip for these domains (numbers of rows and of 60-column tiles)
-int tf_strip_rows_default(const int* rows, const int* tiles, int n);
 // ghost fill of set G of every domain; kinds_mask selects which boundary kinds act (bit per kind).
 void launch_tf_ghost(const TfBatch& b, int G, int kinds_mask, int maxn, hipStream_t s);
 // per-tile dt minima of the live sets (partials: the last stage has left them per strip), then one step
