@@ -54,9 +54,9 @@ def measured_traffic(workload: str, kernel: str, rows: str, summary: str = "hbm_
     return None
 
 
-def resolved_stage_kernel(option: str, nx: int, ny: int) -> str:
-    """The stage kernel the library runs for --stage-kernel auto: strips at every size."""
-    return option if option != "auto" else "strip"
+def resolved_stage_kernel(option: str) -> str:
+    """The stage kernel the library runs for --stage-kernel: strips at every size for "auto" and "tile"."""
+    return "cell" if option == "cell" else "strip"
 
 
 def stage_bytes_per_cell(integrator: str) -> float:
@@ -295,7 +295,7 @@ def bench_batch(args) -> dict:
     # default launch shape and with the batch's tuned shape; the faster of the two is the baseline
     seq_steps = max(5, min(args.steps, 100))
     seq = {}
-    for sh in ("64x4", shape):
+    for sh in ("auto", shape):
         if sh in seq:
             continue
         seq_wall = 0.0
@@ -514,7 +514,7 @@ def main() -> None:
         return
     st, cfg, spec, desc = make_workload(args.workload)
     cells = spec.xdim * spec.ydim
-    kernel = resolved_stage_kernel(args.stage_kernel, spec.xdim, spec.ydim)
+    kernel = resolved_stage_kernel(args.stage_kernel)
     opts = {"stage_kernel": args.stage_kernel, "tc_kernel": args.tc_kernel}
     if args.strip_rows:
         opts["strip_rows"] = args.strip_rows

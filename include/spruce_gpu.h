@@ -152,8 +152,8 @@ int spruce_gpu_device_grid(spruce_gpu_domain* d, const char* name, double** dev_
 
 /* Execution options (no reference counterpart; step results are identical for every setting):
  *   "stage_kernel" = "auto" (default: strips) | "strip" (strips of a block of two wavefronts
- *                    marching along x) | "tile" (8x8 tiles) | "cell" (one thread per cell, faces
- *                    recomputed per cell);
+ *                    marching along x) | "tile" (accepted; strips) | "cell" (one thread per cell,
+ *                    faces recomputed per cell);
  *   "strip_rows"   = rows per strip, a multiple of 4 (default: chosen from the grid size);
  *   "tc_kernel"    = thermal-conduction update: "auto" (default: strips) | "strip" (wavefront strips,
  *                    every face computed once, b_hat derivatives formed in the kernel) | "cell" (one

@@ -41,11 +41,16 @@ def rel_linf(a, b):
     return float(np.max(np.abs(a - b)) / scale) if scale > 0 else float(np.max(np.abs(a - b)))
 
 
-@pytest.mark.parametrize("kernel", ["strip", "cell", "tile"])
+# strips of the default height (1 row on grids this small) and of 8
+KERNELS = {"strip": {"stage_kernel": "strip"}, "cell": {"stage_kernel": "cell"},
+           "strip8": {"stage_kernel": "strip", "strip_rows": 8}}
+
+
+@pytest.mark.parametrize("kernel", KERNELS)
 @pytest.mark.parametrize("case", CASES)
 def test_moc_matches_reference_golden_bitwise(case, kernel):
     g = load_golden(case)
-    dom = GpuDomain(g.spec(), options={"stage_kernel": kernel})
+    dom = GpuDomain(g.spec(), options=KERNELS[kernel])
     try:
         for name, ref in g.frame(0).items():
             assert same_bits(dom.grid(name), ref), "%s setup %s" % (case, name)

@@ -19,7 +19,9 @@ VISC = [c for c in golden_names() if c.startswith(("visc_", "heat_")) and "_tc_"
 # cases through a libm power in the reference: conduction, physical viscosity (T^2.5)
 VISC_TC = [c for c in golden_names() if (c.startswith(("visc_", "heat_")) and "_tc_" in c) or c.startswith("pv_")]
 VARS = ["rho", "temp", "mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z", "n", "thermal_energy", "press", "dt"]
-KERNELS = ["cell", "strip", "tile"]
+# strips of the default height (1 row on grids this small) and of 8
+KERNELS = {"cell": {"stage_kernel": "cell"}, "strip": {"stage_kernel": "strip"},
+           "strip8": {"stage_kernel": "strip", "strip_rows": 8}}
 
 
 def same_bits(a, b):
@@ -39,7 +41,7 @@ def describe(a, b):
 def test_viscosity_matches_reference_golden(case, kernel):
     print("case", case, kernel, flush=True)
     g = load_golden(case)
-    dom = GpuDomain(g.spec(), options={"stage_kernel": kernel})
+    dom = GpuDomain(g.spec(), options=KERNELS[kernel])
     try:
         step = 0
         for k in g.frames[1:]:
@@ -114,7 +116,7 @@ def test_viscosity_matches_oracle(case, kernel):
     name, nx, ny, bc, integ, terms, extra = case
     print("case", name, kernel, flush=True)
     spec = _visc_spec(nx, ny, 61, bc, integ, terms, **dict(extra))
-    gpu = GpuDomain(spec, options={"stage_kernel": kernel})
+    gpu = GpuDomain(spec, options=KERNELS[kernel])
     ora = OracleDomain(spec)
     try:
         rg, ro = gpu.rhs(), ora.rhs()
