@@ -1,7 +1,8 @@
 """Values outside the range of the strip kernels' untested divisions take the tested ones, bit for bit.
 
 Each case plants values out of range (range.hpp) in part of the grid, or takes the mesh or the external
-field out of range, and compares every evolved grid and step size with the CPU restatement.
+field out of range, and compares every evolved grid and step size with the CPU restatement, signs of zeros
+included.
 """
 import numpy as np
 import pytest
@@ -10,8 +11,11 @@ from oracle.oracle import OracleDomain
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
+PLASMA = ("i_rho", "e_rho", "i_mom_x", "i_mom_y", "e_mom_x", "e_mom_y", "i_thermal_energy", "e_thermal_energy", "E_x", "E_y",
+          "E_z", "bi_x", "bi_y", "bi_z")
 EVOLVED = ("rho", "mom_x", "mom_y", "mom_z", "thermal_energy", "bi_x", "bi_y", "bi_z")
 
 
@@ -50,8 +54,7 @@ def check(st, cfg, options, steps=3, names=EVOLVED):
         assert np.array_equal(a.view(np.int64), b.view(np.int64)), (a, b)
         for v in names:
             x, y = gpu.grid(v), ora.grid(v)
-            assert np.array_equal(x.view(np.int64), y.view(np.int64)) or np.array_equal(x, y, equal_nan=True), \
-                (v, np.argwhere(x != y)[:4])
+            assert same_bits(x, y), (v, np.argwhere((x != y) | (np.signbit(x) != np.signbit(y)))[:4])
     finally:
         gpu.close()
         ora.close()
@@ -121,6 +124,39 @@ def test_conduction_out_of_range(sat, integ, what):
         set_pow_mode(0)
 
 
+def plasma_signs(nx, ny):
+    """Zero momenta of both signs beside moving cells, with everything else of the momentum equation -0 where
+    v_y is: whether a momentum of -0 keeps its sign is then up to the sign of the limited fluxes' difference,
+    which the untested limiter does not settle (in about one such cell in 30 it has the other one)."""
+    st = W.ucnp_state(nx, ny, seed=nx)
+    g, rng = st.grids, np.random.default_rng(3)
+    for k in ("i_rho", "e_rho", "i_temp", "e_temp"):
+        g[k] = np.full((nx, ny), g[k].max())
+    for k in ("E_x", "E_y", "grav_x", "grav_y"):
+        g[k] = np.full((nx, ny), -0.0)
+    m = 1e4 * g["i_rho"].max()
+    for k in ("i_mom_x", "e_mom_x"):
+        g[k] = rng.choice([0.0, -0.0, m, -m], size=(nx, ny), p=[0.2, 0.6, 0.1, 0.1])
+    for k in ("i_mom_y", "e_mom_y"):
+        g[k] = rng.choice([0.0, -0.0], size=(nx, ny))
+    return st
+
+
+@pytest.mark.parametrize("curl", [False, True])
+def test_two_fluid_momenta_of_minus_zero(curl):
+    st = plasma_signs(62, 121)
+    cfg = W.ucnp_config(steps=4, integrator="euler", remove_curl_terms=not curl, bc=PERIODIC)
+    ora = OracleDomain(spec_from_files(cfg, st))
+    try:
+        ora.step(1)
+        x = ora.grid("i_mom_x")
+        assert 1000 < np.sum((x == 0.0) & np.signbit(x)) < np.sum(np.signbit(st.grids["i_mom_x"]) & (st.grids["i_mom_x"] == 0.0))
+    finally:
+        ora.close()
+    for options in ({"block": "64x4"}, {"block": "strip4"}, {}):
+        check(st, cfg, options, steps=1, names=PLASMA)
+
+
 @pytest.mark.parametrize("curl", [False, True])
 @pytest.mark.parametrize("what,nx,ny,bc", [("minus_zero", 21, 62, "open_ucnp"), ("tiny", 23, 121, "open_ucnp"),
                                            ("none", 7, 59, "fixed"), ("none", 16, 120, "reflect"), ("mesh", 14, 61, "periodic")])
@@ -138,7 +174,5 @@ def test_two_fluid(curl, what, nx, ny, bc):
         for k in ("d_x", "d_y", "pos_x", "pos_y"):
             g[k] = g[k] * 1e-15
     cfg = W.ucnp_config(steps=4, integrator="rk2", remove_curl_terms=not curl, bc=(bc,) * 4)
-    names = ("i_rho", "e_rho", "i_mom_x", "i_mom_y", "e_mom_x", "e_mom_y", "i_thermal_energy", "e_thermal_energy", "E_x", "E_y",
-             "E_z", "bi_x", "bi_y", "bi_z")
-    check(st, cfg, {"block": "strip4"}, steps=3, names=names)
-    check(st, cfg, {}, steps=3, names=names)
+    check(st, cfg, {"block": "strip4"}, steps=3, names=PLASMA)
+    check(st, cfg, {}, steps=3, names=PLASMA)

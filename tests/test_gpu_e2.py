@@ -8,6 +8,7 @@ from oracle.oracle import OracleDomain
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain, SpruceError
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -16,12 +17,6 @@ E2_VARS = ["rho", "n", "mom_x", "mom_y", "i_thermal_energy", "e_thermal_energy",
            "b_hat_y", "dt"]
 CONS_VARS = ["rho", "temp", "mom_x", "mom_y", "bi_x", "bi_y", "n", "v_x", "v_y", "kinetic_energy", "b_x", "b_y",
              "b_mag", "mag_energy", "b_hat_x", "b_hat_y", "thermal_energy", "press", "press_tot", "energy", "dt"]
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def describe(a, b):

@@ -20,6 +20,7 @@ from oracle.oracle import OracleDomain, set_pow_mode
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain, SpruceError
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
 from cases import random_mhd_state  # noqa: E402
@@ -28,12 +29,6 @@ pytestmark = pytest.mark.gpu
 
 CASES = ["moc_x_periodic_rk2", "moc_y2_closed_euler", "moc_all_limits_rk4", "moc_mixed_stretch_rk2"]
 VARS = ["rho", "temp", "mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z", "n", "thermal_energy", "press", "dt"]
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def rel_linf(a, b):

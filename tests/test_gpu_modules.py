@@ -16,18 +16,13 @@ from oracle.oracle import OracleDomain, cr_pow, set_pow_mode
 from spruce_amd import workloads as W
 from spruce_amd.gpu import POW_EXPONENTS, GpuDomain, pow_probe
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
 
 SOLAR = [c for c in golden_names() if c.startswith("solar_")]
 VARS = ["rho", "temp", "mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z", "n", "thermal_energy", "press", "dt"]
 REL_TOL = 1e-10
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def rel_linf(a, b):

@@ -23,6 +23,7 @@ from oracle.oracle import OracleDomain, set_pow_mode
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden"))
 from cases import random_mhd_state  # noqa: E402
@@ -34,12 +35,6 @@ EXACT = ["lheat_ramp_rk2", "lheat_periodic_euler", "mass_inj_rk4", "mom_inj_rot_
          "outflow_exp_y2_rk2", "outflow_gauss_x1_dyn_euler", "outflow_flat_y1_rk4", "outflow_exp_x2_aligned_rk2"]
 VARS = ["rho", "temp", "mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z", "n", "thermal_energy", "press", "dt"]
 REL_TOL = 1e-10
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def rel_linf(a, b):

@@ -10,7 +10,8 @@ from oracle.oracle import OracleDomain, set_pow_mode
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain
 from spruce_amd.spec import spec_from_files
-from tests.test_gpu_tc_strip import VARS, describe, same_bits
+from tests.bits import same_bits
+from tests.test_gpu_tc_strip import VARS, describe
 
 pytestmark = pytest.mark.gpu
 

@@ -5,7 +5,8 @@ by one), periodic and closed sides on either axis, each subcycle integrator."""
 import pytest
 
 from spruce_amd.gpu import GpuDomain
-from tests.test_gpu_tc_strip import VARS, conduction_case, describe, same_bits
+from tests.bits import same_bits
+from tests.test_gpu_tc_strip import VARS, conduction_case, describe
 
 pytestmark = pytest.mark.gpu
 

@@ -8,6 +8,7 @@ from oracle.oracle import OracleDomain
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuBatch, GpuDomain
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -15,12 +16,6 @@ EVOLVED = ["i_rho", "e_rho", "i_mom_x", "i_mom_y", "e_mom_x", "e_mom_y", "i_ther
            "E_x", "E_y", "E_z", "bi_x", "bi_y", "bi_z"]
 DERIVED = ["i_temp", "e_temp", "i_n", "e_n", "i_v_x", "e_v_y", "j_x", "j_y", "press", "rho_c", "dn", "dt", "dt_i",
            "b_mag", "b_hat_x", "curlE_z", "divE", "divB", "i_dPdx", "e_dPdx"]
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def describe(a, b):

@@ -13,17 +13,12 @@ from oracle.oracle import OracleDomain
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain, SpruceError
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
 
 EVOLVED = ["rho", "mom_x", "mom_y", "mom_z", "thermal_energy", "bi_x", "bi_y", "bi_z"]
 DERIVED = ["n", "temp", "press", "v_x", "v_y", "b_mag", "b_hat_x", "dt"]
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def describe(a, b):

@@ -12,6 +12,7 @@ from oracle.oracle import OracleDomain, set_pow_mode
 from spruce_amd import workloads as W
 from spruce_amd.gpu import GpuDomain
 from spruce_amd.spec import spec_from_files
+from tests.bits import same_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -22,12 +23,6 @@ VARS = ["rho", "temp", "mom_x", "mom_y", "mom_z", "bi_x", "bi_y", "bi_z", "n", "
 # strips of the default height (1 row on grids this small) and of 8
 KERNELS = {"cell": {"stage_kernel": "cell"}, "strip": {"stage_kernel": "strip"},
            "strip8": {"stage_kernel": "strip", "strip_rows": 8}}
-
-
-def same_bits(a, b):
-    a = np.asarray(a, np.float64)
-    b = np.asarray(b, np.float64)
-    return a.shape == b.shape and (np.array_equal(a.view(np.int64), b.view(np.int64)) or np.array_equal(a, b, equal_nan=True))
 
 
 def describe(a, b):
