@@ -127,7 +127,7 @@ def test_batch_mixed_boundaries_and_blocks():
              tf_spec(72, 48, 9, ("fixed",) * 4, "rk2", True),
              tf_spec(40, 96, 10, ("open",) * 4, "rk2", False, open_boundary_strength=0.4)]
     alone, dts_a = _run_alone(specs, [5])
-    for block in ("16x4", "32x8", "128x2", "strip4", "strip8", "strip16"):
+    for block in ("16x4", "32x8", "128x2", "strip4", "strip8", "strip16", "auto"):
         doms = [GpuDomain(s) for s in specs]
         b = GpuBatch(doms, graph=True, block=block)
         try:
