@@ -44,6 +44,13 @@ def _run(exe, args, cwd):
 
 
 def _both(tmp, args_of):
+    """Both programs on the same arguments.  Where the reference executable is not built the GPU's program still
+    has to run to its end, and the comparison is skipped."""
+    if not os.path.exists(REF):
+        rc, _, se = _run(RUN, args_of(os.path.join(tmp, "gpu")), tmp)
+        assert rc == 134 and "successfully reached" in se, se[-500:]
+        assert "mhd.out" in _files(os.path.join(tmp, "gpu"))
+        pytest.skip("the reference executable oracle/_ref/run is not built: nothing to compare the files with")
     out = {}
     for tag, exe in (("ref", REF), ("gpu", RUN)):
         d = os.path.join(tmp, tag)
