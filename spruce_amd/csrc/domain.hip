@@ -202,8 +202,8 @@ class Domain : public DomainBase {
   uint64_t row_mask[N_STATIC];   // per static field, 0 where every row equals row 0
   bool in_range = false;  // the mesh and the external field allow untested divisions (range.hpp)
   int stage_kernel = 0;   // 0: wavefront strips (mhd2.hip), 1: one thread per cell (mhd.hip)
-  // the final stage of a step also forms the next step size's per-block minima (strip form, no
-  // limiter or module after the integrator)
+  // the final stage of a step also forms the next step size's per-block minima (strip form, mesh and
+  // gamma in the range of the untested divisions, no limiter or module after the integrator)
   bool fuse_dt = false;
   int dt_still = 0;       // sides whose ghost fill zeroes the momenta of the interior row next to them
   int strip_rows = 0;     // rows per wavefront strip; 0 = chosen from the grid size
@@ -448,7 +448,8 @@ class Domain : public DomainBase {
       for (int i = 1; same && i < nx; ++i) same = std::memcmp(&g[(size_t)i * ny], &g[0], ny * sizeof(double)) == 0;
       row_mask[k] = same ? 0 : ~(uint64_t)0;
     }
-    in_range = ax.in_range && ay.in_range && kc.gm1 >= 0x1p-60 && kc.gm1 <= 0x1p+10;
+    const bool mesh_in_range = ax.in_range && ay.in_range && kc.gm1 >= 0x1p-60 && kc.gm1 <= 0x1p+10;
+    in_range = mesh_in_range;
     for (const char* s : {"be_x", "be_y", "be_z"})
       for (double v : host_grids[s]) in_range = in_range && field_in_range(v);
 
@@ -474,7 +475,7 @@ class Domain : public DomainBase {
 
     if (strip_rows == 0) strip_rows = mhd_strip_rows_default(nx, ny);
     if (tc_kernel < 0) tc_kernel = 0;   // the strips are the faster form at every size
-    fuse_dt = !any_moc;
+    fuse_dt = !any_moc && mesh_in_range;   // the stage tests the cell's values only before untested divisions
     for (auto& m : mods) fuse_dt = fuse_dt && !m->acts_after_integrator();
     for (int k = 0; k < 4; ++k)
       if (bc[k] == SPRUCE_BC_FIXED || bc[k] == SPRUCE_BC_REFLECT) dt_still |= 1 << k;

@@ -101,8 +101,8 @@ struct StageArgs {
   // open_moc characteristic terms (8 * nx*ny, evolved order), added to the ghost cells' RHS; null
   // without open_moc sides
   const double* moc;
-  // strip form only, null otherwise: one minimum per block of the target's per-cell dt over the
-  // interior (the final stage of a step that no limiter or module follows); dt_still: a bit per side
+  // strip form with mesh and gamma in range only, null otherwise: one minimum per block of the target's per-cell
+  // dt over the interior (the final stage of a step that no limiter or module follows); dt_still: a bit per side
   // (x lower, x upper, y lower, y upper) whose ghost fill zeroes the momenta of the interior row next
   // to it
   double* dt_partial;

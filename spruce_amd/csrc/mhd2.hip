@@ -152,8 +152,8 @@ __device__ __forceinline__ void velocities(double rho, const double* m, double* 
   for (int k = 0; k < N; ++k) v[k] = IN ? qdiv_in(m[k], rho, rr) : qdiv_d(m[k], rho, rr);
 }
 
-// The inverse of IdealMHD::recomputeDT at one cell (idealmhd.cpp:279-304).  IN: rho, te, mom and b2 are
-// in range and te is positive.  There |v| stands for sqrt(v*v), which equals it, and the slow speed,
+// The inverse of IdealMHD::recomputeDT at one cell (idealmhd.cpp:279-304).  IN: rho, te, mom, b2, the mesh
+// and gamma are in range and te is positive.  There |v| stands for sqrt(v*v), which equals it, and the slow speed,
 // never above the fast one (or NaN with it), is left out of the maximum.
 template <bool IN>
 __device__ __forceinline__ double dt_inverse(double rho, double te, double mx, double my, double b2, const MhdConst& K,
@@ -191,21 +191,21 @@ __device__ __forceinline__ double dt_inverse(double rho, double te, double mx, d
 }
 // What the fluid's wavefront keeps of an updated row until the field's |b|^2 of it is there, and the
 // largest inverse step size so far (1/x falls as x grows, so the smallest step size is 1 over the
-// largest inverse; a NaN never replaces it, as std::min drops it).
+// largest inverse; a NaN never replaces it, as std::min drops it).  The mesh and gamma are in range: without
+// that the host has the step size formed by a kernel of its own.
 struct DtState {
   double rho, te, mx, my, dx, rdx;
   bool cell = false;           // this lane's cell takes part
   bool pending = false;
   double worst = 0.0;
-  // in_range: the mesh and gamma are (StageArgs)
-  __device__ __forceinline__ void finish(bool in_range, double b2, const MhdConst& K, double dy, double rdy) {
+  __device__ __forceinline__ void finish(double b2, const MhdConst& K, double dy, double rdy) {
     RangeTest t;
     t.density(rho);
     t.add(te);
     t.add(mx);
     t.add(my);
     t.add(b2);
-    const bool out = t.out() || !(te > 0.0) || !in_range;
+    const bool out = t.out() || !(te > 0.0);
     double s;
     if (__any(cell && out)) s = dt_inverse<false>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
     else s = dt_inverse<true>(rho, te, mx, my, b2, K, dx, rdx, dy, rdy);
@@ -401,7 +401,7 @@ __device__ __forceinline__ int march(const StageArgs& a, const Column& col, Shar
       f[F_ZIN][lane] = qdiv_t<IN>(cz0 * biy - cz1 * bix, 4.0 * PI, K.r4pi);
     }
     block_barrier();
-    if (DT && ROLE == FLUID && dt.pending) dt.finish(a.in_range, sh.b2[slot ^ 1][lane], K, gy.d, gy.rd);
+    if (DT && ROLE == FLUID && dt.pending) dt.finish(sh.b2[slot ^ 1][lane], K, gy.d, gy.rd);
     if (IN && tested_out(slot)) return false;
     if (!DT && !col.out) return true;
     double o_rho = 1.0, o_te = 1.0, o_mx = 0.0, o_my = 0.0, o_b2 = 0.0;   // what the step size reads
@@ -520,7 +520,7 @@ __device__ __forceinline__ void strip_rows(const StageArgs& a, const Column& col
     block_barrier();
     if constexpr (ROLE == FLUID) {
       const double2 d = sh.geom[5][threadIdx.x];
-      if (dt.pending) dt.finish(a.in_range, sh.b2[(rend - 1) & 1][threadIdx.x], a.k, d.x, d.y);
+      if (dt.pending) dt.finish(sh.b2[(rend - 1) & 1][threadIdx.x], a.k, d.x, d.y);
       double m = dt.worst;
       for (int off = 32; off > 0; off >>= 1) {
         const double o = __shfl_xor(m, off, 64);
