@@ -15,11 +15,11 @@
 // made once per loaded value (range.hpp) instead of at each of the ~90 divisions per cell, where
 // they cost twice the instructions and ended a basic block each.  One wavefront for all eleven
 // quantities needs more than 256 registers once the code is straight, and a spilled value's reload
-// also waits for the rows being fetched; the split leaves room (249 registers, no spill, two
+// also waits for the rows being fetched; the split leaves room (231 to 240 vector registers, none spilled, two
 // wavefronts per SIMD) to fetch a row two rows ahead.  Measured on 2048x2048 (RK2, periodic): 536 us
 // a stage with tested divisions and one wavefront per strip, 404 us with untested ones, 350 us with
 // the split, 281 us with the longer fetch distance, the geometry gathered and read through the scalar
-// cache, and the static rows; 1.09 GB of HBM traffic a launch, VALU 46% busy.  512x1024: 110 -> 41 us;
+// cache, and the static rows; 0.81 GB of HBM traffic a launch, VALU 46% busy.  512x1024: 110 -> 41 us;
 // 64x48: 17 (8x8 tiles) -> 9 us.
 #include <cfloat>
 #include <type_traits>

@@ -279,20 +279,20 @@ __global__ void __launch_bounds__(256) k_tc_step(TcStepArgs a) {
 // is bit-identical to the one-thread-per-cell form.
 //
 // What bounds it: HBM and the latency of a row's chain.  A 2048x2048 subcycle moves at least 168 MB
-// (40 B per cell), 34 us at the 4.9 TB/s a large copy reaches here; an 18-row strip's halo rows and
-// lanes make it 188 MB.  The divisions' range tests are made once per row (range.hpp) instead of at
+// (40 B per cell), 34 us at the 4.9 TB/s a large copy reaches here; a 23-row strip's halo rows and
+// lanes make it 210 MB, at 4.7 TB/s.  The divisions' range tests are made once per row (range.hpp) instead of at
 // each of ~20 divisions and both powers share one square root, so a row is about 250 VALU
 // instructions in one run instead of 400 in twenty pieces (1.78e7 against 2.79e7 a launch), and the
 // row's geometry comes through the scalar cache, so that nothing waits for the row being fetched but
 // its use.  Measured per subcycle: 2048x2048 79.5 -> 47 to 52 us, 512x1024 17.5 (one thread per cell) ->
-// 11 to 12.3 us, 133x197 7.7 -> 5.0 us.  160 VGPRs, three wavefronts per SIMD: at four (128) the two register
+// 11 to 12.3 us, 133x197 7.7 -> 5.0 us.  157 to 161 VGPRs, three wavefronts per SIMD: at four (128) the two register
 // sets of a pair of rows spill.
 //
 // With flux saturation the march also forms the saturated flux and coefficient of each row, from the
 // temperature gradient it has there, and writes a row once the next row's coefficient is known: its cells
 // reach two rows and two lanes to each side, so lane l holds column 60*tile + l - 2 and lanes 2..61 write.
 // As a kernel of its own, which formed temperatures and gradients again, the coefficient took 24.5 us
-// per update at 700x1301 beside the update's 19.3; together they take 28.5.  VALU-bound; 213 VGPRs, two
+// per update at 700x1301 beside the update's 19.3; together they take 28.5.  VALU-bound; 207 to 213 VGPRs, two
 // wavefronts per SIMD (three spill).
 //
 // Rows rs .. rend-1.  D = DIV_IN: the geometric divisions and the powers without their operand tests;
